@@ -853,17 +853,43 @@ def adjoint_waves_default(cm, precision, adjoint_precision=None):
     return 1
 
 
-def sheet_cpt(precision):
-    """Cells per thread of the persistent sheet driver (4: a tile is 64 x 16
-    cells for a 256-thread workgroup)."""
+def sheet_cpt(precision, dims=None, n_states=8):
+    """Cells per thread of the persistent sheet driver (tiles of 64 x 4 cpt
+    cells for a 256-thread workgroup) on a sheet of ``dims`` (nx, ny) cells:
+    the fewest (1, 2 or 4) whose tiles are all resident within the register
+    budgets of :func:`sheet_waves` on 256 CUs, so that a small sheet uses as
+    much of the device as it can. Measured on LR1991 (us per time step; grid
+    driver, then 1, 2 and 4 cells per thread): single precision 64 x 64
+    6.4, 2.0, 3.0, 5.1; 301 x 217 6.8, 2.3, 3.2, 5.4; 400 x 400 7.6, 2.7,
+    4.1, 5.4; 600 x 600 10.0, 4.1, 5.1, 6.7; 725 x 725 12.4, -, 7.2, 8.3;
+    1024 x 1024 20.6, -, -, 10.5; double precision 64 x 64 9.1, 6.0, 10.4,
+    18.8; 400 x 400 16.5, 11.9, 16.1, 18.8; 600 x 600 27.6, -, 22.7, 30.0.
+    4 for a sheet that fits with none of them; without ``dims``, the tile of
+    a small sheet."""
+    if dims is None:
+        return 1
+    for cpt in (1, 2):
+        tiles = -(-dims[0] // 64) * -(-dims[-1] // (4 * cpt))
+        if len(dims) == 2 and tiles <= 256 * sheet_waves(precision, cpt,
+                                                         n_states):
+            return cpt
     return 4
 
 
-def sheet_waves(precision):
-    """Waves per SIMD the sheet kernel's register budget must allow: 4 in
-    single precision (128 VGPRs, 4096 cells per CU, so 256 CUs hold 1024^2),
-    2 in double (256 VGPRs; sheets up to half that size, larger ones use the
-    grid driver)."""
+def sheet_waves(precision, cpt=4, n_states=8):
+    """Waves per SIMD the sheet kernel's register budget must allow, which
+    is also the workgroups per CU that are sure to be resident. 4 cells per
+    thread: 4 in single precision (128 VGPRs, 4096 cells per CU, so 256 CUs
+    hold 1024^2), 2 in double (256 VGPRs; sheets up to half that size). With
+    fewer cells per thread the state takes fewer registers, and cell models
+    of up to 12 states fit more waves without spilling (LR1991 on 600 x 600
+    cells, us per time step at 4 / 5 / 6 / 8 waves: 1 cell 4.0 / 4.0 / 4.0 /
+    4.5, 2 cells 5.1 / 4.9 / 5.3 / 5.3; double precision on 512 x 512, 1
+    cell, 2 / 4 / 5 waves: 15.5 / 15.6 / 15.9)."""
+    if n_states <= 12:
+        if precision == DOUBLE_PRECISION:
+            return {1: 4, 2: 3}.get(cpt, 2)
+        return {1: 6, 2: 5}.get(cpt, 4)
     return 2 if precision == DOUBLE_PRECISION else 4
 
 
@@ -932,8 +958,8 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         raise ValueError('block_threads must be a multiple of 64 in'
                          ' [64, 1024].')
     cpt = sheet_cpt(precision) if tile_cpt is None else int(tile_cpt)
-    waves = sheet_waves(precision) if tile_waves is None \
-        else int(tile_waves)
+    waves = sheet_waves(precision, cpt, len(cm.states)) \
+        if tile_waves is None else int(tile_waves)
     if cpt not in SHEET_CPT_CHOICES:
         raise ValueError('sheet_cpt must be one of '
                          + str(SHEET_CPT_CHOICES) + '.')

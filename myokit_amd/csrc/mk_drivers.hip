@@ -27,10 +27,11 @@
  *   mk_grid   any size: one fused step per launch, V of neighbours read from
  *             the previous state buffer, new state written to the other
  *             buffer (ping-pong);
- *   mk_sheet  large homogeneous 2D sheets: a persistent cooperative launch,
- *             one 64 x 16 tile per workgroup with its state in registers
- *             for every step of the launch; tile edges are exchanged
- *             through L2 as step-tagged words;
+ *   mk_sheet  2D sheets (one pair of conductances or a field of them): a
+ *             persistent cooperative launch, one 64 x 4 MK_SCPT tile per
+ *             workgroup with its state in registers for every step of the
+ *             launch; tile edges are exchanged through L2 as step-tagged
+ *             words;
  *   mk_chain  graphs of disjoint chains (cables): the same persistent
  *             scheme over the cells laid end to end, a cable spread over
  *             as many tiles as its length needs.
@@ -335,7 +336,10 @@ mk_grid(const MkArgs a, const Real* __restrict__ src, Real* __restrict__ dst,
         const long long tiles_x = (a.nx + 63) / 64;
         ix = (b % tiles_x) * 64 + (threadIdx.x & 63);
         iy = (b / tiles_x) * (MK_BT / 64) + (threadIdx.x >> 6);
-        if (ix >= a.nx || iy >= a.ny) return;
+        if (iy >= a.ny) return;
+        /* lanes beyond the last column compute and store the last cell once
+         * more: waves of at most 8 active lanes are slow (see mk_sheet) */
+        if (ix >= a.nx) ix = a.nx - 1;
         c = ix + iy * a.nx;
     } else {
         c = b * MK_BT + threadIdx.x;
@@ -496,6 +500,13 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
      * rather than registers, where it would add to the live state of all
      * the thread's cells across the halo wait */
     __shared__ Real ca[MK_NCARRY][MK_SCPT][256];
+#if MK_COUPLING == 2
+    /* the tile's conductances for the whole launch: gxs[r][k] between
+     * columns k - 1 and k of row r, gys[r][k] between rows r - 1 and r of
+     * column k (0 beyond the sheet, where it is not read) */
+    __shared__ Real gxs[MK_STH][65];
+    __shared__ Real gys[MK_STH + 1][64];
+#endif
     __shared__ int wg_flag;
     if (threadIdx.x == 0)
         wg_flag = mk_halted(a, a.steps[s1 - 1].row) ? 1 : 0;
@@ -512,7 +523,14 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
     Real y[MK_SCPT][MK_NS];
     Real fv[MK_SCPT][MK_NFA];
     Real q[MK_NQA];
-    bool act[MK_SCPT];
+    /* own: the thread's column is one of the sheet's; row: the cell's row
+     * is. The lanes of an existing row beyond the sheet's last column
+     * compute a copy of that column's cell, which is not stored: waves with
+     * at most 8 active lanes run several times slower on gfx950 once many
+     * CUs have one (dependent FMAs 2.0 ns each with 9 lanes, 7.2 ns with 8,
+     * on 16 CUs and more) */
+    const bool own = ix < nx;
+    bool row[MK_SCPT];
     bool paced[MK_SCPT];
     /* cell indices in 32 bits (a co-resident sheet has far fewer than 2^31
      * cells) and whether the NaN test reads the cell */
@@ -522,19 +540,33 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
     for (int k = 0; k < MK_SCPT; ++k) {
         const int r = w * MK_SCPT + k;
         const long long iy = gy0 + r;
-        act[k] = ix < nx && iy < ny;
-        const long long c = act[k] ? ix + iy * nx : 0;
+        row[k] = iy < ny;
+        const long long c = row[k] ? (own ? ix : nx - 1) + iy * nx : 0;
         cid[k] = (int)c;
-        nanc[k] = act[k] && a.nan_check && c == a.nan_cell;
-        paced[k] = act[k] && mk_is_paced(a, c, ix, iy);
+        nanc[k] = own && row[k] && a.nan_check && c == a.nan_cell;
+        paced[k] = row[k] && mk_is_paced(a, c, ix, iy);
 #pragma unroll
         for (int i = 0; i < MK_NS; ++i)
-            y[k][i] = act[k] ? a.state_a[(long long)i * a.npad + c] : (Real)0;
+            y[k][i] = row[k] ? a.state_a[(long long)i * a.npad + c] : (Real)0;
 #pragma unroll
         for (int f = 0; f < MK_NF; ++f)
-            fv[k][f] = act[k] ? a.fields[(long long)f * a.npad + c] : (Real)0;
+            fv[k][f] = row[k] ? a.fields[(long long)f * a.npad + c] : (Real)0;
         vt[0][r + 1][lx + 1] = y[k][MK_IVM];
     }
+#if MK_COUPLING == 2
+    for (int q = threadIdx.x; q < MK_STH * 65; q += 256) {
+        const int r = q / 65, k = q - r * 65;
+        const long long x = gx0 + k - 1, yy = gy0 + r;
+        gxs[r][k] = (x >= 0 && x < nx - 1 && yy < ny)
+                        ? a.gx_field[yy * (nx - 1) + x] : (Real)0;
+    }
+    for (int q = threadIdx.x; q < (MK_STH + 1) * 64; q += 256) {
+        const int r = q >> 6, k = q & 63;
+        const long long x = gx0 + k, yy = gy0 + r - 1;
+        gys[r][k] = (yy >= 0 && yy < ny - 1 && x < nx)
+                        ? a.gy_field[yy * nx + x] : (Real)0;
+    }
+#endif
     /* Halo ring at the start of the launch, from the global state */
     {
         const Real* V = a.state_a + (long long)MK_IVM * a.npad;
@@ -574,7 +606,7 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
          * are on their way meanwhile */
 #pragma unroll
         for (int k = 0; k < MK_SCPT; ++k) {
-            if (act[k]) {
+            if (row[k]) {
                 if (p.row >= 0 && nanc[k] && y[k][0] != y[k][0])
                     __atomic_store_n(a.halt, p.row, __ATOMIC_RELAXED);
                 const Real pace = paced[k] ? p.pace : (Real)0;
@@ -585,7 +617,8 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
 #pragma unroll
                 for (int j = 0; j < MK_NCARRY; ++j)
                     ca[j][k][threadIdx.x] = cy[j];
-                if (p.row >= 0) mk_write_log_part<0>(a, cid[k], p.row, q);
+                if (p.row >= 0 && own)
+                    mk_write_log_part<0>(a, cid[k], p.row, q);
             }
             /* one cell after the other: interleaving the cells' part A
              * buys no latency the other waves do not hide, and multiplies
@@ -634,10 +667,24 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
 #pragma unroll
         for (int k = 0; k < MK_SCPT; ++k) {
             const int r = w * MK_SCPT + k;
-            if (act[k]) {
+            if (row[k]) {
                 const long long iy = gy0 + r;
                 const Real v = vt[cur][r + 1][lx + 1];
                 Real id;
+#if MK_COUPLING == 2
+                /* the sums of mk_hetero */
+                id = (Real)0;
+                if (nx > 1) {
+                    if (ix > 0) id += gxs[r][lx] * (v - vt[cur][r + 1][lx]);
+                    if (ix < nx - 1)
+                        id += gxs[r][lx + 1] * (v - vt[cur][r + 1][lx + 2]);
+                }
+                if (ny > 1) {
+                    if (iy > 0) id += gys[r][lx] * (v - vt[cur][r][lx + 1]);
+                    if (iy < ny - 1)
+                        id += gys[r + 1][lx] * (v - vt[cur][r + 2][lx + 1]);
+                }
+#else
                 if (nx > 1) {
                     if (ix == 0) id = a.gx * (v - vt[cur][r + 1][lx + 2]);
                     else if (ix == nx - 1) id = a.gx * (v - vt[cur][r + 1][lx]);
@@ -652,6 +699,7 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
                     else id += a.gy * (((Real)2 * v - vt[cur][r][lx + 1])
                                        - vt[cur][r + 2][lx + 1]);
                 }
+#endif
                 const Real pace = paced[k] ? p.pace : (Real)0;
                 const long long c = cid[k];
                 Real cy[MK_NCARRY];
@@ -659,8 +707,9 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
                 for (int j = 0; j < MK_NCARRY; ++j)
                     cy[j] = ca[j][k][threadIdx.x];
                 mk_cell_b<true>(y[k], p.t, p.dt, pace, id, fv[k], q, cy);
-                if (p.row >= 0) mk_write_log_part<1>(a, c, p.row, q);
-                if (sh.traj) mk_store_traj(a, sh.traj, i, c, y[k]);
+                if (p.row >= 0 && own)
+                    mk_write_log_part<1>(a, c, p.row, q);
+                if (sh.traj && own) mk_store_traj(a, sh.traj, i, c, y[k]);
                 vt[cur ^ 1][r + 1][lx + 1] = y[k][MK_IVM];
             }
         }
@@ -670,17 +719,17 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
          * after the other) */
         if (!last) {
             const int step = sh.g0 + i + 1;
-            if (w == 0 && act[0])
+            if (w == 0 && own && row[0])
                 mk_tput(mk_edge(sh, par, tile, 0, lx), y[0][MK_IVM], step);
-            if (w == 3 && act[MK_SCPT - 1])
+            if (w == 3 && own && row[MK_SCPT - 1])
                 mk_tput(mk_edge(sh, par, tile, 1, lx),
                         y[MK_SCPT - 1][MK_IVM], step);
-            if (lx == 0 || lx == 63) {
+            if ((lx == 0 || lx == 63) && own) {
                 MkXWord* ep = mk_edge(sh, par, tile, lx == 0 ? 2 : 3,
                                       w * MK_SCPT);
 #pragma unroll
                 for (int k = 0; k < MK_SCPT; ++k)
-                    if (act[k]) mk_tput(ep + k * MK_XW, y[k][MK_IVM], step);
+                    if (row[k]) mk_tput(ep + k * MK_XW, y[k][MK_IVM], step);
             }
         }
         /* The next step's barrier (after its halo) orders this step's LDS
@@ -692,7 +741,7 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
      * two in a one-step launch). The host swaps the buffers. */
 #pragma unroll
     for (int k = 0; k < MK_SCPT; ++k) {
-        if (act[k]) {
+        if (own && row[k]) {
             const long long c = ix + (gy0 + w * MK_SCPT + k) * nx;
 #pragma unroll
             for (int i = 0; i < MK_NS; ++i)

@@ -318,6 +318,8 @@ struct Sim : SimBase {
     long long sh_steps = 0;
     long long max_domain = 0;
     int max_block_cells = 0;
+    /* sheets of more cells than this run on the persistent sheet driver */
+    static constexpr long long sheet_cells = 512;
 
     /* graph connections kept on the host for re-layout */
     std::vector<long long> ci, cj;
@@ -399,7 +401,9 @@ struct Sim : SimBase {
         ndom = 1;
         max_domain = n;
         pace_mode = 0;
-        if (cfg.sheet_cpt > 0 && cfg.ny > 1 && p->f_sheet) {
+        if (cfg.sheet_cpt > 0 && cfg.ny > 1 && p->f_sheet &&
+            (cfg.coupling == MKH_COUPLING_STENCIL ||
+             cfg.coupling == MKH_COUPLING_HETERO)) {
             int per_cu = 0, dev = cfg.device;
             MKH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(
                 &per_cu, p->f_sheet, 256, 0));
@@ -439,7 +443,8 @@ struct Sim : SimBase {
             return cfg.coupling == MKH_COUPLING_GRAPH && is_chain &&
                    ch_tiles > 0 && ch_edges.p;
         case MKH_DRIVER_SHEET:
-            return cfg.coupling == MKH_COUPLING_STENCIL && cfg.ny > 1 &&
+            return (cfg.coupling == MKH_COUPLING_STENCIL ||
+                    cfg.coupling == MKH_COUPLING_HETERO) && cfg.ny > 1 &&
                    sh_tx > 0 && sh_ty > 0 && sh_edges.p &&
                    (long long)sh_tx * sh_ty <= sh_capacity;
         default:
@@ -455,9 +460,7 @@ struct Sim : SimBase {
         }
         if (cfg.coupling == MKH_COUPLING_NONE) {
             driver = MKH_DRIVER_CELLS;
-        } else if (cfg.coupling == MKH_COUPLING_STENCIL && cfg.ny > 1 &&
-                   n > 4096 && sh_tx > 0 &&
-                   (long long)sh_tx * sh_ty <= sh_capacity) {
+        } else if (n > sheet_cells && feasible(MKH_DRIVER_SHEET)) {
             driver = MKH_DRIVER_SHEET;
         } else if (max_domain <= max_block_cells &&
                    (ndom >= 64 || max_domain <= 512)) {

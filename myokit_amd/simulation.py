@@ -911,14 +911,20 @@ class SimulationOpenCL:
             return 256
         return int(min(1024, max(64, -(-largest // 64) * 64)))
 
+    def _sheet_cpt(self):
+        """Cells per thread of the persistent sheet: the value given to
+        :meth:`set_tuning`, else the one for this sheet's size."""
+        return self._tuning.get('sheet_cpt') or _kernelgen.sheet_cpt(
+            self._precision, self._dims, self._nstate)
+
     def tuning(self):
         """The current launch configuration (see :meth:`set_tuning`)."""
         return {'driver': self._tuning.get('driver', 'auto'),
                 'block_threads': self._threads(),
-                'sheet_cpt': self._tuning.get(
-                    'sheet_cpt', _kernelgen.sheet_cpt(self._precision)),
+                'sheet_cpt': self._sheet_cpt(),
                 'sheet_waves': self._tuning.get(
-                    'sheet_waves', _kernelgen.sheet_waves(self._precision)),
+                    'sheet_waves', _kernelgen.sheet_waves(
+                        self._precision, self._sheet_cpt(), self._nstate)),
                 'chain_cpt': self._tuning.get(
                     'chain_cpt', _kernelgen.chain_cpt(self._precision)),
                 'chain_waves': self._tuning.get(
@@ -989,7 +995,7 @@ class SimulationOpenCL:
             cm, self._precision, coupling, threads,
             self._native_math, adjoint=adjoint,
             adjoint_precision=adjoint_precision,
-            tile_cpt=tune.get('sheet_cpt'),
+            tile_cpt=self._sheet_cpt(),
             tile_waves=tune.get('sheet_waves'),
             adjoint_waves=tune.get('adjoint_waves'),
             chain_cells=tune.get('chain_cpt'),
@@ -1058,8 +1064,7 @@ class SimulationOpenCL:
         cfg.nx = self._nx
         cfg.ny = self._ny
         cfg.device = self._device
-        cpt = tune.get('sheet_cpt') or _kernelgen.sheet_cpt(self._precision)
-        cfg.sheet_cpt = cpt if _kernelgen.sheet_enabled(self._precision) \
+        cfg.sheet_cpt = self._sheet_cpt() if _kernelgen.sheet_enabled(self._precision) \
             else 0
         cfg.chain_cpt = tune.get('chain_cpt') or \
             _kernelgen.chain_cpt(self._precision)

@@ -66,12 +66,12 @@ def candidates(sim):
         drivers = ['block', 'grid', 'chain']
     else:
         drivers = ['block', 'grid']
-        if c == _native.COUPLING_STENCIL and sim._ny > 1:
+        if sim._ny > 1:
             drivers.append('sheet')
     for d in drivers:
         if d == 'sheet':
             waves = (2, 3) if sim._precision == 64 else (3, 4, 5)
-            cpts = (2, 4) if sim._precision == 64 else (2, 4, 8)
+            cpts = (2, 4) if sim._precision == 64 else (1, 2, 4, 8)
             for cpt in cpts:
                 for w in waves:
                     out.append({'driver': 'sheet', 'block_threads': 256,
@@ -131,7 +131,8 @@ def autotune(sim, duration=None, reps=2, cache=True, verbose=False):
         duration = 200 * sim._step_size
     saved = sim.tuning()
     trials = []
-    for cfg in candidates(sim):
+    # the settings it has (by default those of the fixed rules) count too
+    for cfg in candidates(sim) + [dict(saved)]:
         s = _trial(sim, cfg, duration, reps)
         trials.append((cfg, s))
         if verbose:

@@ -1,0 +1,56 @@
+"""
+The persistent sheet's tiles at their edges: sheets whose sizes leave one
+column, one row or a few lanes in the last tile, each tile height, and
+conductance fields, in double precision against the CPU oracle bit for bit
+and in single precision against the one-step grid driver.
+"""
+import numpy as np
+import pytest
+
+import myokit_amd as myokit
+from tests.helpers import Scenario, run_both
+
+pytestmark = pytest.mark.gpu
+
+# widths with 1, 8 and 64 cells in the last tile column; heights with one
+# row in the last tile row of each tile height, and a sheet of one tile
+SHAPES = [(65, 33), (72, 17), (128, 9), (40, 20)]
+
+
+def _scenario(shape, field, rl=True):
+    nx, ny = shape
+    rng = np.random.default_rng(nx + 7 * ny)
+    g = None
+    if field:
+        gx = rng.uniform(2, 12, (ny, nx - 1))
+        gy = rng.uniform(2, 12, (ny - 1, nx))
+        gx[:, nx // 2] = 0.0
+        g = (gx, gy)
+    return Scenario('lr1991', shape, rl=rl, dt=0.01, gx=9.5, gy=6.0,
+                    paced=(4, ny, 0, 0), conductance_field=g)
+
+
+@pytest.mark.parametrize('shape', SHAPES)
+@pytest.mark.parametrize('field', [False, True])
+def test_fp64_sheet_edges_bit_exact(shape, field):
+    P, O = run_both(_scenario(shape, field), 4.0, myokit.DOUBLE_PRECISION)
+    assert P['sim'].engine_driver() == 'sheet'
+    assert P['sim'].tuning()['sheet_cpt'] == 1
+    np.testing.assert_array_equal(P['V'], O['V'])
+    np.testing.assert_array_equal(P['state'], O['state'])
+
+
+@pytest.mark.parametrize('cpt', [1, 2, 4])
+@pytest.mark.parametrize('field', [False, True])
+def test_fp32_every_tile_height_equals_grid(cpt, field):
+    # the same operations in the same order in every driver and tile height
+    for shape in SHAPES:
+        V = []
+        for kw in ({'driver': 'sheet', 'sheet_cpt': cpt}, {'driver': 'grid'}):
+            s = _scenario(shape, field, rl=False).product(32)
+            s.set_tuning(**kw)
+            b = s.run_block(3.0, ['membrane.V'], log_interval=0.5)
+            assert s.engine_driver() == kw['driver']
+            V.append((b['membrane.V'], np.array(s.state())))
+        np.testing.assert_array_equal(V[0][0], V[1][0])
+        np.testing.assert_array_equal(V[0][1], V[1][1])

@@ -118,3 +118,24 @@ def test_grid_register_budget_in_kernel_source():
         assert '#define MK_GBLOCKS %d' % blocks in src
     with pytest.raises(ValueError):
         _kernelgen.generate_kernel(cm, 64, 1, grid_budget=9)
+
+
+def test_sheet_tiles_follow_the_size():
+    # the fewest cells per thread whose tiles are all sure to be resident:
+    # 64 x 4 cpt cells each, 256 CUs times the waves of the budget
+    from myokit_amd import _kernelgen as k
+    for prec, one, two in ((32, 1536, 1280), (64, 1024, 768)):
+        assert k.sheet_waves(prec, 1) * 256 == one
+        assert k.sheet_waves(prec, 2) * 256 == two
+        # one column of tiles, exactly full and one row more
+        assert k.sheet_cpt(prec, (64, 4 * one)) == 1
+        assert k.sheet_cpt(prec, (64, 4 * one + 1)) == 2
+        assert k.sheet_cpt(prec, (1, 8 * two)) == 2
+        assert k.sheet_cpt(prec, (65, 4 * two + 1)) == 4
+        assert k.sheet_cpt(prec, (5000, 5000)) == 4
+        assert k.sheet_cpt(prec) == 1
+        # large cell models keep the wider register budget
+        assert k.sheet_waves(prec, 1, 30) == k.sheet_waves(prec, 4, 30) \
+            == k.sheet_waves(prec, 4)
+    assert sim((100, 70)).tuning()['sheet_cpt'] == 1
+    assert sim((1024, 1024)).tuning()['sheet_cpt'] == 4
