@@ -61,6 +61,9 @@ extern "C" {
 #define MKH_DRIVER_CHAIN 4  /* graphs of disjoint chains (cables) laid end to
                                end: persistent one-wave tiles, all steps per
                                launch */
+#define MKH_DRIVER_STRAND 5 /* a line of cells: persistent tiles, each step
+                               shared by four waves, all steps of a batch in
+                               one launch */
 
 /* Simulation geometry and kernel layout. */
 typedef struct mkh_sim_config {

@@ -97,6 +97,17 @@ class HipExpressionWriter:
         # exp() code -> (C name of a power B^n, factor exp(m)), single
         # precision exponential families
         self.exp_members = {}
+        # variable -> its equation's text, where the writer is shared
+        self.texts = None
+
+    def rhs(self, var):
+        """The text of a variable's equation."""
+        if self.texts is None:
+            return self.ex(var.rhs())
+        text = self.texts.get(var)
+        if text is None:
+            text = self.texts[var] = self.ex(var.rhs())
+        return text
 
     def set_exp_members(self, members):
         """Writes each exponential in ``members`` (code -> (C name of B^n,
@@ -384,6 +395,9 @@ class CellModel:
         self.fields = list(fields)
         self.quantities = list(quantities)
         self.states = list(model.states())
+        # (precision, native maths) -> writer shared by one kernel's
+        # functions (forward_writer)
+        self.writers = {}
         for q in self.quantities:
             if not (q.is_state() or q.is_intermediary() or q in self.bound):
                 raise ValueError('Cannot log <' + q.qname() + '>.')
@@ -434,6 +448,24 @@ def cell_writer(cm, precision, native_maths=False):
     return w
 
 
+def forward_writer(cm, precision, native_maths=False):
+    """``(writer, lines)``: the writer of the forward cell step, with its
+    exponential families (single precision) and the statements that compute
+    them. The functions of one kernel share it, and with it the text of the
+    equations."""
+    key = (precision, bool(native_maths))
+    hit = cm.writers.get(key)
+    if hit is None:
+        w = cell_writer(cm, precision, native_maths)
+        fam = []
+        if precision == SINGLE_PRECISION:
+            fam, members = exp_families(cm, w)
+            w.set_exp_members(members)
+        w.texts = {}
+        hit = cm.writers[key] = (w, fam)
+    return hit
+
+
 def forward_sweep(cm, w, tab='    '):
     """C statements evaluating every equation of one cell (states read from
     ``y``), in dependency order."""
@@ -443,16 +475,16 @@ def forward_sweep(cm, w, tab='    '):
                      + str(i) + '];')
     for var in cm.per_cell_constants:
         lines.append(tab + 'const Real ' + _cname(var, 'c_') + ' = '
-                     + w.ex(var.rhs()) + ';')
+                     + w.rhs(var) + ';')
     for var in cm.order:
         if var.is_state():
             if var in cm.rl_states:
                 continue
             lines.append(tab + 'const Real ' + _cname(var, 'd_') + ' = '
-                         + w.ex(var.rhs()) + ';')
+                         + w.rhs(var) + ';')
         else:
             lines.append(tab + 'const Real ' + _cname(var) + ' = '
-                         + w.ex(var.rhs()) + ';')
+                         + w.rhs(var) + ';')
     return lines
 
 
@@ -577,7 +609,7 @@ def exp_families(cm, w, max_power=24, v_range=200.0):
 
 def generate_cell_function(cm, precision, native_maths=False):
     """Returns the HIP source of ``mk_cell<LOG>`` for a CellModel."""
-    w = cell_writer(cm, precision, native_maths)
+    w, fam = forward_writer(cm, precision, native_maths)
     lines = []
     tab = '    '
 
@@ -590,10 +622,6 @@ def generate_cell_function(cm, precision, native_maths=False):
     lines.append('{')
     lines.append(tab + '(void)t; (void)dt; (void)pace; (void)idiff;'
                  ' (void)fv; (void)q;')
-    fam = []
-    if precision == SINGLE_PRECISION:
-        fam, members = exp_families(cm, w)
-        w.set_exp_members(members)
     sweep = forward_sweep(cm, w, tab)
     ns = len(cm.states)
     lines.extend(sweep[:ns] + [tab + x for x in fam] + sweep[ns:])
@@ -671,62 +699,16 @@ def generate_split_cell_function(cm, precision, native_maths=False):
     cells before it waits for the neighbours' potentials of the step, and
     part B after. ``mk_qpart[k]`` says which part sets logged quantity k."""
     import re
-    w = cell_writer(cm, precision, native_maths)
     tab = '    '
-    dep, dstates = diffusion_dependents(cm)
-    fam = []
-    if precision == SINGLE_PRECISION:
-        fam, members = exp_families(cm, w)
-        w.set_exp_members(members)
-    a_lines, b_lines = [], []
-    declared = []
-    for i, s in enumerate(cm.states):
-        a_lines.append('const Real ' + _cname(s, 'x_') + ' = y[' + str(i)
-                       + '];')
-        declared.append(_cname(s, 'x_'))
-    for var in cm.per_cell_constants:
-        a_lines.append('const Real ' + _cname(var, 'c_') + ' = '
-                       + w.ex(var.rhs()) + ';')
-        declared.append(_cname(var, 'c_'))
-    for line in fam:
-        a_lines.append(line)
-        declared.append(line.split()[2])
-    for var in cm.order:
-        if var.is_state():
-            if var in cm.rl_states:
-                continue
-            name, into = _cname(var, 'd_'), (b_lines if var in dstates
-                                               else a_lines)
-        else:
-            name, into = _cname(var), (b_lines if var in dep else a_lines)
-        line = 'const Real ' + name + ' = ' + w.ex(var.rhs()) + ';'
-        into.append(line)
-        if into is a_lines:
-            declared.append(name)
-    qa, qb, qpart = [], [], []
-    for k, var in enumerate(cm.quantities):
-        line = 'q[' + str(k) + '] = ' + w.ex(ex.Name(var)) + ';'
-        in_b = var in dep
-        (qb if in_b else qa).append(line)
-        qpart.append(1 if in_b else 0)
-    ua, ub = [], []
-    # a state that part B advances still holds its value at t in y when
-    # part B starts (part A does not write it): B reads it there
-    in_y = {}
-    for i, s in enumerate(cm.states):
-        if s in cm.rl_states:
-            inf, tau = cm.rl_states[s]
-            in_b = inf in dep or tau in dep
-        else:
-            in_b = s in dstates
-        (ub if in_b else ua).append(_state_update(cm, w, precision, i, s))
-        if in_b:
-            in_y[_cname(s, 'x_')] = i
+    a_lines, b_lines, declared, qa, qb, qpart, ua, ub, in_y = _split_lines(
+        cm, precision, native_maths)
     # what part B reads of part A's values
-    b_text = '\n'.join(b_lines + qb + ub)
+    b_text = '\n'.join(b_lines + qb + list(ub.values()))
     used = set(re.findall(r'[A-Za-z_][A-Za-z0-9_]*', b_text))
     from_y = [n for n in declared if n in used and n in in_y]
     carry = [n for n in declared if n in used and n not in in_y]
+    qa, qb = list(qa.values()), qb
+    ua, ub = list(ua.values()), list(ub.values())
     out = ['#define MK_NCARRY ' + str(max(1, len(carry))),
            '__device__ constexpr int mk_qpart[' + str(max(1, len(qpart)))
            + '] = {' + ', '.join(str(x) for x in (qpart or [0])) + '};']
@@ -767,6 +749,280 @@ def generate_split_cell_function(cm, precision, native_maths=False):
         out.append(tab + '}')
     out += [tab + x for x in ub]
     out.append('}')
+    return '\n'.join(out) + '\n'
+
+
+def _split_lines(cm, precision, native_maths, defer=()):
+    """The statements of a cell step in two parts (see
+    :func:`generate_split_cell_function`): ``(a_lines, b_lines, declared,
+    qa, qb, qpart, ua, ub, in_y)``, with the values declared in part A, its
+    logged quantities by index, part B's as a list, the part of each
+    quantity, the state updates of both parts by state index, and the
+    states that part B advances (name -> index; they hold their value at t
+    in y when part B starts). Variables in ``defer`` are evaluated in part
+    B."""
+    w, fam = forward_writer(cm, precision, native_maths)
+    dep, dstates = diffusion_dependents(cm)
+    late = dep | set(defer)
+    a_lines, b_lines = [], []
+    declared = []
+    for i, s in enumerate(cm.states):
+        a_lines.append('const Real ' + _cname(s, 'x_') + ' = y[' + str(i)
+                       + '];')
+        declared.append(_cname(s, 'x_'))
+    for var in cm.per_cell_constants:
+        a_lines.append('const Real ' + _cname(var, 'c_') + ' = '
+                       + w.rhs(var) + ';')
+        declared.append(_cname(var, 'c_'))
+    for line in fam:
+        a_lines.append(line)
+        declared.append(line.split()[2])
+    for var in cm.order:
+        if var.is_state():
+            if var in cm.rl_states:
+                continue
+            name, into = _cname(var, 'd_'), (b_lines if var in dstates
+                                               else a_lines)
+        else:
+            name, into = _cname(var), (b_lines if var in late else a_lines)
+        line = 'const Real ' + name + ' = ' + w.rhs(var) + ';'
+        into.append(line)
+        if into is a_lines:
+            declared.append(name)
+    qa, qb, qpart = {}, [], []
+    for k, var in enumerate(cm.quantities):
+        line = 'q[' + str(k) + '] = ' + w.ex(ex.Name(var)) + ';'
+        in_b = var in late
+        if in_b:
+            qb.append(line)
+        else:
+            qa[k] = line
+        qpart.append(1 if in_b else 0)
+    ua, ub = {}, {}
+    # a state that part B advances still holds its value at t in y when
+    # part B starts (part A does not write it): B reads it there
+    in_y = {}
+    for i, s in enumerate(cm.states):
+        if s in cm.rl_states:
+            inf, tau = cm.rl_states[s]
+            in_b = inf in dep or tau in dep
+        else:
+            in_b = s in dstates
+        (ub if in_b else ua)[i] = _state_update(cm, w, precision, i, s)
+        if in_b:
+            in_y[_cname(s, 'x_')] = i
+    return a_lines, b_lines, declared, qa, qb, qpart, ua, ub, in_y
+
+
+def _is_sum(e):
+    """Whether ``e`` only adds and subtracts names and numbers."""
+    if isinstance(e, (ex.Plus, ex.Minus, ex.PrefixPlus, ex.PrefixMinus)):
+        return all(_is_sum(x) for x in e)
+    return isinstance(e, (ex.Name, ex.Number))
+
+
+def _deferred(cm):
+    """The variables that :func:`generate_group_cell_functions` evaluates
+    after the groups have met, because the values that need the diffusion
+    current read them and they are sums of other variables (the total ionic
+    current) or depend on no state (the stimulus current)."""
+    dep, dstates = diffusion_dependents(cm)
+    order = [v for v in cm.order if not v.is_state()]
+    free = set()
+    for v in order:
+        if all(r.var() in cm.bound or r.var() in cm.constants
+               or r.var() in free for r in v.rhs().references()):
+            free.add(v)
+    out = set()
+    for v in reversed(cm.order):
+        if not (v in dep or v in dstates or v in out):
+            continue
+        for r in v.rhs().references():
+            u = r.var()
+            if u in order and u not in dep and u not in cm.bound and (
+                    u in free or _is_sum(u.rhs())):
+                out.add(u)
+    # whatever part A reads stays there
+    rl = set(v for it in cm.rl_states.values() for v in it)
+    while True:
+        read = set(r.var() for v in cm.order
+                   if v not in dep and v not in dstates and v not in out
+                   and v not in cm.rl_states
+                   for r in v.rhs().references()) | rl
+        if not (out & read):
+            return out
+        out -= read
+
+
+def _text_cost(text, precision):
+    """Rough VALU cost of a C statement, for balancing the groups."""
+    import re
+    if precision == DOUBLE_PRECISION:
+        price = {'mk_exp': 24, 'mk_log': 40, 'mk_log10': 42, 'mk_pow': 70,
+                 'mk_sin': 40, 'mk_cos': 40, 'mk_tan': 70, 'mk_atan': 50,
+                 'mk_asin': 60, 'mk_acos': 60, 'mk_powi': 3, '/': 11,
+                 '__builtin_sqrt': 14}
+    else:
+        price = {'__builtin_amdgcn_exp2f': 2, '__builtin_amdgcn_rcpf': 2,
+                 'mk_expf': 8, 'mk_expf_native': 3, 'logf': 12, '__logf': 4,
+                 'powf': 30, '__powf': 8, 'sinf': 30, 'cosf': 30,
+                 'tanf': 40, 'atanf': 20, 'asinf': 25, 'acosf': 25,
+                 'mk_powif': 3, 'sqrtf': 8, '/': 10}
+    n = 0
+    for t in re.findall(r'[A-Za-z_][A-Za-z0-9_]*|[-+*/?<>]', text):
+        n += price.get(t, 1 if t in '-+*?<>/' else 0)
+    return n
+
+
+# Groups of waves that share one cell step in the strand driver
+STRAND_GROUPS = 4
+
+
+def strand_cells(coupling, dims):
+    """Whether the strand driver may run these cells (the library decides
+    by the device's CUs): uncoupled cells or a line of cells, at most 4 tiles
+    of 64 cells per CU of 256."""
+    n = dims[0] * (dims[1] if len(dims) == 2 else 1)
+    line = len(dims) == 1 or dims[1] == 1
+    return n <= 64 * 4 * 256 and (coupling == 0
+                                  or (coupling in (1, 2) and line))
+
+
+def generate_group_cell_functions(cm, precision, native_maths=False,
+                                  groups=STRAND_GROUPS):
+    """Returns the HIP source of ``mk_ga<g>`` and ``mk_gb<g>``: the cell
+    step of ``mk_cell`` shared by ``groups`` waves that hold the same cells,
+    with the same operations. Part A is what does not depend on the
+    diffusion current, cut into roots (each state's update, each value that
+    part B reads, each logged quantity); a root belongs to one group, which
+    evaluates everything the root needs (an equation that several groups
+    need is evaluated by each). Roots go to the groups in order of cost,
+    each to the group that is then cheapest. ``mk_ga<g>`` leaves the values
+    that other groups read in an exchange area (one column per lane of
+    MK_NXS values); after a barrier, ``mk_gb<g>`` reads them, finishes the
+    sums of :func:`_deferred` and advances the states that depend on the
+    diffusion current, in every group alike.
+
+    ``mk_gown[i]``: group that advances state i (-1: all, in part B);
+    ``mk_gheld[g]``: bit i set if group g holds state i; ``mk_gq[k]``: group
+    that logs quantity k. MK_NG is 0 (no such functions) for models of more
+    than 64 states."""
+    import re
+    ns = len(cm.states)
+    if ns > 64:
+        return '#define MK_NG 0\n'
+    a_lines, b_lines, declared, qa, qb, qpart, ua, ub, in_y = _split_lines(
+        cm, precision, native_maths, _deferred(cm))
+    word = re.compile(r'[A-Za-z_][A-Za-z0-9_]*')
+    line_of = dict(zip(declared, a_lines))
+    pos = {n: k for k, n in enumerate(declared)}
+    xname = {_cname(s, 'x_'): i for i, s in enumerate(cm.states)}
+
+    def names(text):
+        return set(n for n in word.findall(text) if n in line_of)
+
+    need = {}       # declared name -> every declared name it needs
+    for n in declared:
+        d = names(line_of[n].split('=', 1)[1])
+        need[n] = set([n]).union(*[need[m] for m in d]) if d else {n}
+
+    def closure(text):
+        d = names(text)
+        return set().union(*[need[m] for m in d]) if d else set()
+    cost = {n: _text_cost(line_of[n].split('=', 1)[1], precision)
+            for n in declared}
+    b_names = names('\n'.join(b_lines + qb + list(ub.values())))
+    carry = [n for n in declared if n in b_names and n not in in_y]
+    roots = [('u', i, t) for i, t in ua.items()] \
+        + [('c', n, n) for n in carry] + [('q', k, t) for k, t in qa.items()]
+    roots = [(kind, key, t, closure(t), _text_cost(t, precision))
+             for kind, key, t in roots]
+    roots.sort(key=lambda r: -sum(cost[n] for n in r[3]) - r[4])
+    mine = [[] for _ in range(groups)]
+    have = [set() for _ in range(groups)]
+    load = [0] * groups
+    for r in roots:
+        after = [load[g] + sum(cost[n] for n in r[3] - have[g]) + r[4]
+                 for g in range(groups)]
+        g = min(range(groups), key=lambda g: (after[g], g))
+        mine[g].append(r[:3])
+        have[g] |= r[3]
+        load[g] = after[g]
+    own = [-1] * ns
+    qown = [0] * max(1, len(cm.quantities))
+    for g in range(groups):
+        for kind, key, _ in mine[g]:
+            if kind == 'u':
+                own[key] = g
+            elif kind == 'q':
+                qown[key] = g
+    held = []
+    for g in range(groups):
+        h = set(xname[n] for n in have[g] if n in xname) | set(ub) | set(i for i in range(ns) if own[i] == g)
+        held.append(h)
+    # exchange area: the carried values, then the states that a group holds
+    # and another one advances
+    slot = {n: k for k, n in enumerate(carry)}
+    for i in range(ns):
+        if own[i] >= 0 and any(i in held[g] for g in range(groups)
+                               if g != own[i]):
+            slot[i] = len(slot)
+    tab = '    '
+    out = ['#define MK_NG ' + str(groups),
+           '#define MK_NXS ' + str(max(1, len(slot))),
+           '__device__ constexpr int mk_gown[MK_NS] = {'
+           + ', '.join(str(x) for x in own) + '};',
+           '__device__ constexpr unsigned long long mk_gheld[MK_NG] = {'
+           + ', '.join(hex(sum(1 << i for i in h)) + 'ull' for h in held)
+           + '};',
+           '__device__ constexpr int mk_gq[' + str(len(qown)) + '] = {'
+           + ', '.join(str(x) for x in qown) + '};',
+           'template <int G> __device__ __forceinline__ void mk_ga(',
+           tab + 'Real* __restrict__ y, Real t, Real dt, Real pace,',
+           tab + 'const Real* __restrict__ fv, Real* __restrict__ q,',
+           tab + 'Real (*xo)[64], int lane);',
+           'template <int G> __device__ __forceinline__ void mk_gb(',
+           tab + 'Real* __restrict__ y, Real t, Real dt, Real pace, '
+           'Real idiff,',
+           tab + 'const Real* __restrict__ fv, Real* __restrict__ q,',
+           tab + 'const Real (*xi)[64], int lane);']
+    for g in range(groups):
+        out += ['template <> __device__ __forceinline__ void mk_ga<'
+                + str(g) + '>(',
+                tab + 'Real* __restrict__ y, const Real t, const Real dt, '
+                'const Real pace,',
+                tab + 'const Real* __restrict__ fv, Real* __restrict__ q,',
+                tab + 'Real (*xo)[64], const int lane)', '{',
+                tab + '(void)t; (void)dt; (void)pace; (void)fv; (void)q;'
+                ' (void)xo; (void)lane;']
+        out += [tab + line_of[n] for n in sorted(have[g], key=pos.get)]
+        out += [tab + t for kind, _, t in mine[g] if kind == 'q']
+        out += [tab + t for kind, _, t in mine[g] if kind == 'u']
+        out += [tab + 'xo[' + str(slot[key]) + '][lane] = ' + key + ';'
+                for kind, key, _ in mine[g] if kind == 'c']
+        out += [tab + 'xo[' + str(slot[i]) + '][lane] = y[' + str(i) + '];'
+                for i in range(ns) if own[i] == g and i in slot]
+        out += ['}',
+                'template <> __device__ __forceinline__ void mk_gb<'
+                + str(g) + '>(',
+                tab + 'Real* __restrict__ y, const Real t, const Real dt, '
+                'const Real pace,',
+                tab + 'const Real idiff, const Real* __restrict__ fv, '
+                'Real* __restrict__ q,',
+                tab + 'const Real (*xi)[64], const int lane)', '{',
+                tab + '(void)t; (void)dt; (void)pace; (void)idiff; (void)fv;'
+                ' (void)q;', tab + '(void)xi; (void)lane;']
+        out += [tab + 'const Real ' + n + ' = y[' + str(in_y[n]) + '];'
+                for n in declared if n in in_y and n in b_names]
+        out += [tab + 'const Real ' + n + ' = xi[' + str(slot[n])
+                + '][lane];' for n in carry]
+        out += [tab + x for x in b_lines]
+        if g == 0:
+            out += [tab + x for x in qb]
+        out += [tab + x for x in ub.values()]
+        out += [tab + 'y[' + str(i) + '] = xi[' + str(slot[i]) + '][lane];'
+                for i in range(ns) if own[i] not in (-1, g) and i in held[g]]
+        out.append('}')
     return '\n'.join(out) + '\n'
 
 
@@ -939,7 +1195,7 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
                     native_maths=False, adjoint=False, tile_cpt=None,
                     tile_waves=None, adjoint_precision=None,
                     adjoint_waves=None, chain_cells=None, chain_budget=None,
-                    adjoint_cpt=None, grid_budget=None):
+                    adjoint_cpt=None, grid_budget=None, strand=True):
     """Returns the complete HIP source for hiprtc. ``tile_cpt`` (cells
     per thread of the persistent sheet: tile height 4 x cpt) and
     ``tile_waves`` (waves per SIMD its register budget allows) default to
@@ -953,7 +1209,8 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
     :func:`chain_waves`), ``adjoint_cpt`` the persistent reverse sheet's
     cells per thread (default :func:`adjoint_sheet_cpt`), ``grid_budget``
     the waves per SIMD of the grid driver's register budget (default
-    :func:`grid_waves`; 0: no limit)."""
+    :func:`grid_waves`; 0: no limit). ``strand``: whether the text holds
+    the strand driver."""
     if block_threads % 64 or not 64 <= block_threads <= 1024:
         raise ValueError('block_threads must be a multiple of 64 in'
                          ' [64, 1024].')
@@ -1018,6 +1275,8 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         _FLOAT_HELPERS,
         generate_cell_function(cm, precision, native_maths),
         generate_split_cell_function(cm, precision, native_maths),
+        generate_group_cell_functions(cm, precision, native_maths)
+        if strand and int(coupling) != 3 else '#define MK_NG 0\n',
         _read('mk_drivers.hip'),
     ]
     if adjoint:

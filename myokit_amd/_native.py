@@ -30,6 +30,7 @@ DRIVER_BLOCK = 1
 DRIVER_GRID = 2
 DRIVER_SHEET = 3
 DRIVER_CHAIN = 4
+DRIVER_STRAND = 5
 
 # Every entry point declared in include/myokit_amd.h
 _c = ctypes

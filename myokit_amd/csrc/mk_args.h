@@ -117,4 +117,22 @@ struct MkChainT {
     int spin_limit;           /* polls before a wait is abandoned */
 };
 
+/* Persistent strand driver: a line of cells (or uncoupled cells) cut into
+ * tiles of `width` cells, each advanced by one workgroup whose lanes hold
+ * the tile and `halo` more cells on each side. */
+template <typename R>
+struct MkStrandT {
+    unsigned long long* edges;  /* [2][tiles][2][states][32][sizeof(R) / 4]
+                                   states of each tile's first and last
+                                   `halo` cells, tagged (by exchange
+                                   parity) */
+    int* err;                 /* set to 1 if a neighbour wait timed out */
+    int tiles;                /* number of tiles */
+    int width;                /* cells per tile (the last may have fewer) */
+    int halo;                 /* steps between exchanges; 0: no coupling */
+    int g0;                   /* exchanges completed before this launch */
+    int spin_limit;           /* polls before a wait is abandoned */
+    R* traj;                  /* as MkSheetT */
+};
+
 #endif

@@ -17,7 +17,7 @@
  * with the state at t, the intermediaries and idiff written to the log at
  * log steps. The reference runs this as 2-3 kernels per step with the state
  * in AoS layout; here the coupling and the update are fused in one pass over
- * SoA state, and five drivers cover the geometries:
+ * SoA state, and six drivers cover the geometries:
  *
  *   mk_cells  uncoupled cells: one thread per cell keeps its state in
  *             registers across every step of the launch (no synchronisation);
@@ -32,6 +32,8 @@
  *             workgroup with its state in registers for every step of the
  *             launch; tile edges are exchanged through L2 as step-tagged
  *             words;
+ *   mk_strand a line of cells (or uncoupled cells) too short to fill the
+ *             device: four waves share each step of 64 cells;
  *   mk_chain  graphs of disjoint chains (cables): the same persistent
  *             scheme over the cells laid end to end, a cable spread over
  *             as many tiles as its length needs.
@@ -941,6 +943,260 @@ mk_chain(const MkArgs a, const MkChain ch, const int s0, const int s1)
         }
     }
 }
+
+#if MK_NG > 0
+/* ------------------------------------------------------------------------
+ * Persistent strand: a line of cells (a cable, with one conductance or a
+ * field of them), or uncoupled cells, few enough that one wave per 64 cells
+ * would leave most of the device idle.
+ *
+ * One cell step is a chain of a few thousand dependent instructions, and a
+ * wave issues one of them every four cycles at best, so with one wave per
+ * SIMD a step takes as long as the instructions of one cell. Here MK_NG
+ * waves share the same 64 cells: each evaluates its part of the equations
+ * (mk_ga<g>, the split of generate_group_cell_functions), the values that
+ * the others read go through LDS, and after one barrier every wave finishes
+ * the step (mk_gb<g>: the sum of the currents, the diffusion current and
+ * the update of V). Same operations, same results as mk_cell.
+ *
+ * A workgroup owns st.width cells and holds st.halo more on each side
+ * (64 = width + 2 halo lanes), which it advances too: what a halo lane
+ * computes is right for as many steps as it is away from the tile's edge,
+ * so only every st.halo steps the neighbours exchange the states of their
+ * outer cells (step-tagged words, as mk_sheet's edges), and the exchange's
+ * latency is spread over st.halo steps. All steps of a batch run in one
+ * cooperative launch, log rows included.
+ *
+ * LR1991, forward Euler, us per step, one thread per cell (mk_block up to
+ * 512 cells, mk_grid) -> strand: 200 cells in double precision 4.3 -> 1.5,
+ * single 1.27 -> 0.63; 1,000 cells 8.2 -> 1.5 and 6.3 -> 0.63. What is left
+ * is issue: the largest group takes 417 instructions per step in double
+ * precision, 0.85 us at the 4.8 cycles a lone wave needs for each. Eight
+ * groups gave 1.28 us with one tile per CU but would halve the tiles that
+ * run side by side, and their barrier costs the same in single precision
+ * (0.62).
+ *
+ * The NaN test at a log step records the first row only; the host then
+ * takes the steps up to that row again from the launch's start state (which
+ * is in state_a, untouched), so that the run ends where it always did.
+ * ---------------------------------------------------------------------- */
+typedef MkStrandT<Real> MkStrand;
+
+/* State i of the kth of the outer cells of a tile's side e (0 first cells,
+ * 1 last cells), slot of exchange parity par. */
+__device__ __forceinline__ MkXWord* mk_sedge(const MkStrand& st, int par,
+                                             int tile, int e, int i, int k)
+{
+    return st.edges + ((((long long)(par * st.tiles + tile) * 2 + e) * MK_NS
+                        + i) * 32 + k) * MK_XW;
+}
+
+template <int G>
+__device__ __forceinline__ void mk_strand_run(
+    const MkArgs& a, const MkStrand& st, const int s0, const int s1,
+    Real (*xs)[MK_NXS][64], Real (*vt)[66], volatile int* flag)
+{
+    constexpr unsigned long long HELD = mk_gheld[G];
+    const int lane = threadIdx.x & 63, tile = blockIdx.x;
+    const long long n = a.n;
+    const long long c0 = (long long)tile * st.width;
+    const int len = (int)(n - c0 < st.width ? n - c0 : st.width);
+    /* the lane's cell: lanes before the first cell or after the last one
+     * compute a copy of that cell (which nothing reads) */
+    const long long cl = c0 + lane - st.halo;
+    const long long c = cl < 0 ? 0 : cl >= n ? n - 1 : cl;
+    const bool own = lane >= st.halo && lane < st.halo + len;
+    const bool paced = mk_is_paced(a, c, c % a.nx, c / a.nx);
+    Real y[MK_NS], fv[MK_NFA], q[MK_NQA];
+#pragma unroll
+    for (int i = 0; i < MK_NS; ++i)
+        y[i] = (HELD >> i & 1) ? a.state_a[(long long)i * a.npad + c]
+                               : (Real)0;
+#pragma unroll
+    for (int f = 0; f < MK_NF; ++f) fv[f] = a.fields[(long long)f * a.npad + c];
+#pragma unroll
+    for (int k = 0; k < MK_NQA; ++k) q[k] = (Real)0;
+    if (G == 0) vt[0][lane + 1] = y[MK_IVM];
+#if MK_COUPLING == 1
+    const bool first = c == 0, end = c == n - 1;
+#elif MK_COUPLING == 2
+    const Real gl = c > 0 ? a.gx_field[c - 1] : (Real)0;
+    const Real gr = c < n - 1 ? a.gx_field[c] : (Real)0;
+    const bool first = c == 0, end = c == n - 1;
+#endif
+    const bool nanc = own && a.nan_check && c == a.nan_cell
+                      && (mk_gown[0] < 0 ? 0 : mk_gown[0]) == G;
+    bool halted = false;
+    int left = st.halo, sup = 0, cur = 0;
+    bool fresh = false;     /* an exchange has just been taken */
+    MkStep p = a.steps[s0];
+    for (int s = s0; s < s1; ++s) {
+        const MkStep pn = a.steps[s + 1 < s1 ? s + 1 : s];
+        const Real pace = paced ? p.pace : (Real)0;
+        if (p.row >= 0 && nanc && !halted && y[0] != y[0]) {
+            halted = true;
+            __atomic_store_n(a.halt, p.row, __ATOMIC_RELAXED);
+        }
+        mk_ga<G>(y, p.t, p.dt, pace, fv, q, xs[cur], lane);
+        __syncthreads();
+        if (fresh) {
+            if (*flag) return;
+            fresh = false;
+        }
+        Real id = (Real)0;
+#if MK_COUPLING == 1
+        {
+            const Real v = vt[cur][lane + 1];
+            const Real vl = vt[cur][lane], vr = vt[cur][lane + 2];
+            if (n > 1) {
+                if (first) id = a.gx * (v - vr);
+                else if (end) id = a.gx * (v - vl);
+                else id = a.gx * (((Real)2 * v - vl) - vr);
+            }
+        }
+#elif MK_COUPLING == 2
+        {
+            const Real v = vt[cur][lane + 1];
+            const Real vl = vt[cur][lane], vr = vt[cur][lane + 2];
+            if (!first) id += gl * (v - vl);
+            if (!end) id += gr * (v - vr);
+        }
+#endif
+        mk_gb<G>(y, p.t, p.dt, pace, id, fv, q, xs[cur], lane);
+        if (p.row >= 0 && own) {
+#pragma unroll
+            for (int k = 0; k < MK_NQ; ++k) {
+                if (mk_gq[k] != G) continue;
+                const int col = a.colmap[(long long)k * a.npad + c];
+                if (col >= 0)
+                    a.logbuf[(long long)p.row * a.ncols + col] = q[k];
+            }
+        }
+        if (st.traj && own) {
+            Real* __restrict__ tr =
+                st.traj + (long long)(s - s0) * MK_NS * a.npad + c;
+#pragma unroll
+            for (int i = 0; i < MK_NS; ++i)
+                if ((mk_gown[i] < 0 ? 0 : mk_gown[i]) == G)
+                    tr[(long long)i * a.npad] = y[i];
+        }
+#if MK_COUPLING != 0
+        if (--left == 0 && st.tiles > 1 && s + 1 < s1) {
+            left = st.halo;
+            const int step = st.g0 + ++sup, par = step & 1;
+            /* the tile's outer cells for the neighbours: each state from
+             * the group that advances it */
+            const bool el = own && lane < 2 * st.halo && tile > 0;
+            const bool er = own && lane >= len && tile + 1 < st.tiles;
+#pragma unroll
+            for (int i = 0; i < MK_NS; ++i) {
+                if ((mk_gown[i] < 0 ? 0 : mk_gown[i]) != G) continue;
+                if (el)
+                    mk_tput(mk_sedge(st, par, tile, 0, i, lane - st.halo),
+                            y[i], step);
+                if (er)
+                    mk_tput(mk_sedge(st, par, tile, 1, i, lane - len), y[i],
+                            step);
+            }
+            /* the neighbours' into the halo lanes: all words of a round of
+             * polls in flight together */
+            const bool hl = lane < st.halo && tile > 0;
+            const bool hr = lane >= st.halo + len && tile + 1 < st.tiles
+                            && cl < n;
+            if (hl || hr) {
+                MkXWord* e = hl ? mk_sedge(st, par, tile - 1, 1, 0, lane)
+                                : mk_sedge(st, par, tile + 1, 0, 0,
+                                           lane - st.halo - len);
+                for (int spins = 0;; ++spins) {
+                    MkXWord w[MK_NS * MK_XW];
+                    bool ready = true;
+#pragma unroll
+                    for (int i = 0; i < MK_NS; ++i) {
+                        if (!(HELD >> i & 1)) continue;
+#pragma unroll
+                        for (int h = 0; h < MK_XW; ++h)
+                            w[i * MK_XW + h] = __hip_atomic_load(
+                                e + i * 32 * MK_XW + h, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+                    }
+#pragma unroll
+                    for (int i = 0; i < MK_NS; ++i) {
+                        if (!(HELD >> i & 1)) continue;
+#pragma unroll
+                        for (int h = 0; h < MK_XW; ++h)
+                            ready = ready
+                                    && (int)(w[i * MK_XW + h] >> 32) >= step;
+                    }
+                    if (ready) {
+#pragma unroll
+                        for (int i = 0; i < MK_NS; ++i) {
+                            if (!(HELD >> i & 1)) continue;
+                            if constexpr (sizeof(Real) == 4)
+                                y[i] = (Real)__uint_as_float((unsigned)w[i]);
+                            else
+                                y[i] = (Real)__longlong_as_double((long long)(
+                                    ((w[i * MK_XW] & 0xffffffffull) << 32)
+                                    | (w[i * MK_XW + MK_XW - 1]
+                                       & 0xffffffffull)));
+                        }
+                        break;
+                    }
+                    if (spins >= st.spin_limit) {
+                        __hip_atomic_store(st.err, 1, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                        *flag = 1;
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+            }
+            fresh = true;
+        }
+#endif
+        /* read after the next step's barrier; the other buffer's last
+         * readers passed this step's */
+        if (G == 0) vt[cur ^ 1][lane + 1] = y[MK_IVM];
+        cur ^= 1;
+        p = pn;
+    }
+    if (own) {
+#pragma unroll
+        for (int i = 0; i < MK_NS; ++i)
+            if ((mk_gown[i] < 0 ? 0 : mk_gown[i]) == G)
+                a.state_b[(long long)i * a.npad + c] = y[i];
+    }
+}
+
+/* mk_strand_run<g> for the wave's group g */
+template <int G>
+__device__ __forceinline__ void mk_strand_group(
+    int g, const MkArgs& a, const MkStrand& st, const int s0, const int s1,
+    Real (*xs)[MK_NXS][64], Real (*vt)[66], volatile int* flag)
+{
+    if (g == G) mk_strand_run<G>(a, st, s0, s1, xs, vt, flag);
+    else if constexpr (G + 1 < MK_NG)
+        mk_strand_group<G + 1>(g, a, st, s0, s1, xs, vt, flag);
+}
+
+extern "C" __global__ void __launch_bounds__(64 * MK_NG)
+mk_strand(const MkArgs a, const MkStrand st, const int s0, const int s1)
+{
+    __shared__ Real xs[2][MK_NXS][64];
+    __shared__ Real vt[2][66];
+    __shared__ int flag;
+    if (threadIdx.x == 0) flag = mk_halted(a, a.steps[s1 - 1].row) ? 1 : 0;
+    if (threadIdx.x < 2) {
+        vt[threadIdx.x][0] = (Real)0;
+        vt[threadIdx.x][65] = (Real)0;
+    }
+    __syncthreads();
+    const bool stop = flag;
+    __syncthreads();
+    if (stop) return;
+    mk_strand_group<0>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), a,
+                       st, s0, s1, xs, vt, &flag);
+}
+#endif
 
 /* ------------------------------------------------------------------------
  * Fiber-tissue junction (diff_step_fiber_tissue, openclsim.cl:601-628):

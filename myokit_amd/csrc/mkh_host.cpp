@@ -70,7 +70,7 @@ struct Program {
     hipModule_t module = nullptr;
     hipFunction_t f_cells = nullptr, f_block = nullptr, f_grid = nullptr;
     hipFunction_t f_sheet = nullptr, f_junction = nullptr;
-    hipFunction_t f_chain = nullptr;
+    hipFunction_t f_chain = nullptr, f_strand = nullptr;
     hipFunction_t f_adj_step = nullptr, f_adj_block = nullptr,
                   f_adj_probe = nullptr, f_adj_sheet = nullptr,
                   f_adj_gather = nullptr;
@@ -79,6 +79,26 @@ struct Program {
     int layout[6] = {0, 0, 0, 0, 0, 0};
     bool have_layout = false;
     std::vector<char> code;
+    /* The device's CUs and the workgroups of each persistent kernel that
+     * are resident on one (0: no such kernel), asked once when the module is
+     * loaded: the queries take about a millisecond each. */
+    int ncu = 0, cu_sheet = 0, cu_strand = 0, cu_chain = 0, cu_adj_sheet = 0;
+
+    hipError_t query()
+    {
+        hipError_t e = hipDeviceGetAttribute(
+            &ncu, hipDeviceAttributeMultiprocessorCount, device);
+        auto ask = [&](int* per_cu, hipFunction_t f, int threads) {
+            if (e == hipSuccess && f)
+                e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(
+                    per_cu, f, threads, 0);
+        };
+        ask(&cu_sheet, f_sheet, 256);
+        ask(&cu_strand, f_strand, 256);
+        ask(&cu_chain, f_chain, 64);
+        ask(&cu_adj_sheet, f_adj_sheet, 256);
+        return e;
+    }
 };
 
 unsigned long long fnv1a(const std::string& s, unsigned long long h)
@@ -314,6 +334,11 @@ struct Sim : SimBase {
     bool is_chain = false;
     int ch_tiles = 0, ch_len = 0;
     long long ch_steps = 0;
+    /* strand driver: lines of cells and uncoupled cells in few tiles */
+    DevBuf<unsigned long long> st_edges;
+    DevBuf<int> st_err;
+    int st_tiles = 0, st_width = 0, st_halo = 0;
+    long long st_done = 0;        /* exchanges completed in this run */
     int sh_tx = 0, sh_ty = 0, sh_capacity = 0;
     long long sh_steps = 0;
     long long max_domain = 0;
@@ -404,12 +429,7 @@ struct Sim : SimBase {
         if (cfg.sheet_cpt > 0 && cfg.ny > 1 && p->f_sheet &&
             (cfg.coupling == MKH_COUPLING_STENCIL ||
              cfg.coupling == MKH_COUPLING_HETERO)) {
-            int per_cu = 0, dev = cfg.device;
-            MKH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, p->f_sheet, 256, 0));
-            hipDeviceProp_t prop;
-            MKH_HIP(hipGetDeviceProperties(&prop, dev));
-            sh_capacity = per_cu * prop.multiProcessorCount;
+            sh_capacity = p->cu_sheet * p->ncu;
             const int th = 4 * cfg.sheet_cpt;
             sh_tx = (int)((cfg.nx + 63) / 64);
             sh_ty = (int)((cfg.ny + th - 1) / th);
@@ -422,7 +442,94 @@ struct Sim : SimBase {
                 MKH_HIP(hipMemset(sh_err.p, 0, sizeof(int)));
             }
         }
+        int e = build_strand_layout();
+        if (e) return e;
         choose_driver();
+        return 0;
+    }
+
+    /* Tiles of the strand driver: 64 uncoupled cells, a line of at most 64
+     * cells, or 64 - 2 h cells of a longer one with h more on each side and
+     * an exchange every h steps. h = 16, or 8 where the tiles would then
+     * outnumber the CUs. As many tiles per CU as leave the split of a step
+     * over four waves the faster way: uncoupled cells 3 (LR1991 forward
+     * Euler, us per step, split and one thread per cell: single precision
+     * 16,384 cells 0.36 and 0.65, 32,768 0.44 and 0.67, 49,152 0.57 and
+     * 0.68, 65,536 0.74 and 0.69; double precision 1.29 and 3.40, 2.03 and
+     * 3.42, 2.67 and 3.48, 3.38 and 3.54), a line 4 (strand and grid driver:
+     * 1,000 cells 0.63 and 6.3, 12,000 0.70 and 6.4, 49,000 1.2 and 6.4;
+     * double precision 1.5 and 8.2, 1.6 and 8.4, 4.4 and 8.7). */
+    int build_strand_layout()
+    {
+        st_tiles = 0;
+        const bool coupled = (cfg.coupling == MKH_COUPLING_STENCIL ||
+                              cfg.coupling == MKH_COUPLING_HETERO) &&
+                             cfg.ny == 1;
+        if (!prog->f_strand || !(coupled || cfg.coupling == MKH_COUPLING_NONE))
+            return 0;
+        const int per_cu = prog->cu_strand, ncu = prog->ncu;
+        if (per_cu < 1) return 0;
+        for (int h : {0, 16, 8}) {
+            if (h == 0 && coupled && n > 64) continue;
+            const long long width = 64 - 2 * h;
+            const long long tiles = (n + width - 1) / width;
+            const int most = h == 0 ? 3 : h == 16 ? 1 : 4;
+            if (tiles > (long long)std::min(most, per_cu) * ncu) continue;
+            st_halo = h;
+            st_width = (int)width;
+            st_tiles = (int)tiles;
+            break;
+        }
+        if (st_tiles == 0) return 0;
+        MKH_HIP(st_err.alloc(1));
+        MKH_HIP(hipMemset(st_err.p, 0, sizeof(int)));
+        if (st_halo > 0) {
+            MKH_HIP(st_edges.alloc((size_t)st_tiles * 4 * cfg.n_state * 32 *
+                                   XW));
+            MKH_HIP(hipMemset(st_edges.p, 0,
+                              st_edges.n * sizeof(unsigned long long)));
+        }
+        st_done = 0;
+        return 0;
+    }
+
+    /* Whether a run on driver `d` takes the strand kernel: that driver
+     * itself, and, where no driver was asked for, few uncoupled cells and
+     * the lines of cells that the adjoint keeps on the layouts of its
+     * reverse kernels. */
+    bool strand_for(int d) const
+    {
+        return st_tiles > 0 && ndom == 1 &&
+               (d == MKH_DRIVER_STRAND || forced_driver < 0);
+    }
+
+    /* Steps [s0, s1) from state `src` to state `dst` (two buffers) in one
+     * launch; `trajp` as MkStrandT. */
+    int strand_launch(Args a, R* src, R* dst, int s0, int s1, R* trajp)
+    {
+        a.state_a = src;
+        a.state_b = dst;
+        MkStrandT<R> st;
+        std::memset(&st, 0, sizeof(st));
+        st.edges = st_edges.p;
+        st.err = st_err.p;
+        st.tiles = st_tiles;
+        st.width = st_width;
+        st.halo = st_halo;
+        st.g0 = (int)st_done;
+        st.spin_limit = 1 << 20;
+        st.traj = trajp;
+        void* params[] = {&a, &st, &s0, &s1};
+        if (st_halo > 0) {
+            MKH_HIP(hipModuleLaunchCooperativeKernel(
+                prog->f_strand, (unsigned)st_tiles, 1, 1, 256, 1, 1, 0,
+                stream, params));
+            st_done += (s1 - s0 - 1) / st_halo;
+        } else {
+            MKH_HIP(hipModuleLaunchKernel(prog->f_strand, (unsigned)st_tiles,
+                                          1, 1, 256, 1, 1, 0, stream, params,
+                                          nullptr));
+        }
         return 0;
     }
 
@@ -439,6 +546,9 @@ struct Sim : SimBase {
             return max_domain <= max_block_cells;
         case MKH_DRIVER_GRID:
             return true;
+        case MKH_DRIVER_STRAND:
+            return st_tiles > 0 && ndom == 1 &&
+                   cfg.coupling != MKH_COUPLING_NONE;
         case MKH_DRIVER_CHAIN:
             return cfg.coupling == MKH_COUPLING_GRAPH && is_chain &&
                    ch_tiles > 0 && ch_edges.p;
@@ -460,6 +570,10 @@ struct Sim : SimBase {
         }
         if (cfg.coupling == MKH_COUPLING_NONE) {
             driver = MKH_DRIVER_CELLS;
+        } else if (feasible(MKH_DRIVER_STRAND) && !prog->f_adj_step) {
+            /* (the adjoint keeps the layouts of its reverse kernels; its
+             * forward steps take the strand kernel, strand_for) */
+            driver = MKH_DRIVER_STRAND;
         } else if (n > sheet_cells && feasible(MKH_DRIVER_SHEET)) {
             driver = MKH_DRIVER_SHEET;
         } else if (max_domain <= max_block_cells &&
@@ -625,12 +739,8 @@ struct Sim : SimBase {
             cf[a] |= 2u;
             cf[b] |= 1u;
         }
-        int per_cu = 0, ncu = 0;
-        MKH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, prog->f_chain, 64, 0));
-        MKH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount,
-                                      cfg.device));
-        const long long cap = (long long)per_cu * ncu;
+        const int ncu = prog->ncu;
+        const long long cap = (long long)prog->cu_chain * ncu;
         /* 64 * MK_CCPT cells per tile, fewer if the tiles would then not
          * give every SIMD a wave; more tiles than can be co-resident: as
          * many equal tiles as can */
@@ -967,6 +1077,12 @@ struct Sim : SimBase {
             MKH_HIP(hipMemset(ch_err.p, 0, sizeof(int)));
             ch_steps = 0;
         }
+        if (st_edges.p) {
+            MKH_HIP(hipMemset(st_edges.p, 0,
+                              st_edges.n * sizeof(unsigned long long)));
+            MKH_HIP(hipMemset(st_err.p, 0, sizeof(int)));
+            st_done = 0;
+        }
         size_t need = (size_t)batch_steps;
         MKH_HIP(steps.alloc(need));
         if (h_steps_cap < need) {
@@ -1165,17 +1281,21 @@ struct Sim : SimBase {
                                stream));
         MKH_HIP(hipStreamSynchronize(stream));
         MKH_HIP(hipStreamSynchronize(copy_stream));
-        if (driver == MKH_DRIVER_SHEET || driver == MKH_DRIVER_CHAIN) {
+        const bool strand = driver == MKH_DRIVER_STRAND && st_halo > 0;
+        const int* err = driver == MKH_DRIVER_SHEET   ? sh_err.p
+                         : driver == MKH_DRIVER_CHAIN ? ch_err.p
+                         : strand                     ? st_err.p
+                                                      : nullptr;
+        if (err) {
             int e = 0;
-            MKH_HIP(hipMemcpy(&e, driver == MKH_DRIVER_SHEET ? sh_err.p
-                                                             : ch_err.p,
-                              sizeof(int), hipMemcpyDeviceToHost));
+            MKH_HIP(hipMemcpy(&e, err, sizeof(int), hipMemcpyDeviceToHost));
             if (e) {
                 running = false;
-                return fail(MKH_E_HIP, std::string(driver == MKH_DRIVER_SHEET
-                                                       ? "sheet" : "chain") +
-                                           " driver: a neighbour exchange "
-                                           "timed out");
+                return fail(MKH_E_HIP,
+                            std::string(driver == MKH_DRIVER_SHEET ? "sheet"
+                                        : strand ? "strand"
+                                                 : "chain") +
+                                " driver: a neighbour exchange timed out");
             }
         }
         valid = b.nr;
@@ -1227,6 +1347,8 @@ struct Sim : SimBase {
         }
         /* Launch */
         const unsigned bt = (unsigned)cfg.block_threads;
+        const bool strand = driver == MKH_DRIVER_STRAND ||
+                            (driver == MKH_DRIVER_CELLS && strand_for(driver));
         if (driver == MKH_DRIVER_GRID) {
             for (long long s = 0; s < ns; ++s) {
                 e = grid_launch(b, s, nullptr);
@@ -1287,6 +1409,23 @@ struct Sim : SimBase {
                     if (e) return e;
                 }
             }
+        } else if (strand) {
+            /* the whole batch in one launch, then its log rows in one copy */
+            if (time_kernels) MKH_HIP(hipEventRecord(event(b.nev), stream));
+            e = strand_launch(base_args(), state[cur].p, state[cur ^ 1].p, 0,
+                              (int)ns, nullptr);
+            if (e) return e;
+            if (time_kernels) {
+                MKH_HIP(hipEventRecord(event(b.nev + 1), stream));
+                b.nev += 2;
+            }
+            launches++;
+            if (b.nr > 0 && ncols > 0 && dst_values)
+                MKH_HIP(hipMemcpyAsync(
+                    dst_values + (size_t)rows_done * ncols, logbuf.p,
+                    (size_t)b.nr * ncols * sizeof(R), hipMemcpyDeviceToHost,
+                    stream));
+            cur ^= 1;
         } else {
             hipFunction_t f = driver == MKH_DRIVER_CELLS ? prog->f_cells
                                                          : prog->f_block;
@@ -1312,6 +1451,19 @@ struct Sim : SimBase {
         int halted = -1;
         e = finish_batch(b, valid, halted);
         if (e) return e;
+        if (strand && halted >= 0) {
+            /* the launch went on after the row with the NaN: take the steps
+             * up to it again, from the state the launch started with, to
+             * leave the state where every driver leaves it */
+            long long s = 0;
+            while (s + 1 < ns && h_steps[s].row != halted) ++s;
+            if (s + 1 < ns) {
+                e = strand_launch(base_args(), state[cur ^ 1].p, state[cur].p,
+                                  0, (int)(s + 1), nullptr);
+                if (e) return e;
+                MKH_HIP(hipStreamSynchronize(stream));
+            }
+        }
         return close_batch(b, valid, halted, tout, status);
     }
 
@@ -1337,7 +1489,7 @@ struct Sim : SimBase {
                 forced_driver = (int)v;
                 return 0;
             }
-            if (v < -1 || v > MKH_DRIVER_CHAIN ||
+            if (v < -1 || v > MKH_DRIVER_STRAND ||
                 (v >= 0 && v != MKH_DRIVER_CHAIN && !feasible((int)v)) ||
                 (v == MKH_DRIVER_CHAIN && !is_chain) ||
                 (have_graph && v >= 0 && v != MKH_DRIVER_GRID &&
@@ -1473,8 +1625,11 @@ struct Sim : SimBase {
                              trace_out, nrows, nullptr, 0);
         /* the chain layout's adjoint runs on the grid driver (its CSR is
          * built with it) */
-        DriverAs as_grid(driver, driver == MKH_DRIVER_CHAIN ? MKH_DRIVER_GRID
-                                                            : driver);
+        const bool use_strand = strand_for(driver);
+        DriverAs as_grid(driver, driver == MKH_DRIVER_CHAIN ||
+                                         driver == MKH_DRIVER_STRAND
+                                     ? MKH_DRIVER_GRID
+                                     : driver);
         if (!prog->f_adj_step)
             return fail(MKH_E_STATE, "kernel was generated without the "
                                      "adjoint");
@@ -1624,7 +1779,7 @@ struct Sim : SimBase {
          * also has a persistent reverse kernel. */
         const bool use_pers = driver == MKH_DRIVER_SHEET ||
                               driver == MKH_DRIVER_BLOCK ||
-                              driver == MKH_DRIVER_CELLS;
+                              driver == MKH_DRIVER_CELLS || use_strand;
         const bool block_rev = driver == MKH_DRIVER_BLOCK;
         /* The persistent reverse sheet: 64 x 4 adj_cpt tiles (MK_ACPT in
          * the kernel source), all co-resident; they are no more than the
@@ -1637,12 +1792,7 @@ struct Sim : SimBase {
             prog->f_adj_sheet &&
             sh_edges.p && (size_t)rtx * rty * 4 * 64 * 2 * XW <= sh_edges.n &&
             (size_t)rtx * rty <= nparts) {
-            int per_cu = 0;
-            MKH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, prog->f_adj_sheet, 256, 0));
-            hipDeviceProp_t prop;
-            MKH_HIP(hipGetDeviceProperties(&prop, cfg.device));
-            sheet_rev = (long long)per_cu * prop.multiProcessorCount >=
+            sheet_rev = (long long)prog->cu_adj_sheet * prog->ncu >=
                         (long long)rtx * rty && !no_sheet_rev;
         }
         /* Small domains on the one-step kernels: segment sg - 1 is
@@ -1651,9 +1801,7 @@ struct Sim : SimBase {
          * where the workgroups of both kernels fit on the device at once
          * (otherwise each would only slow the other). Same kernels, same
          * inputs: the results are those of the in-line order. */
-        int ncu = 0;
-        MKH_HIP(hipDeviceGetAttribute(
-            &ncu, hipDeviceAttributeMultiprocessorCount, cfg.device));
+        const int ncu = prog->ncu;
         const bool overlap = !use_pers && nseg > 1 && !no_adj_overlap &&
                              (long long)ggrid + cgrid <= ncu;
         if (overlap) {
@@ -1671,7 +1819,7 @@ struct Sim : SimBase {
         DevBuf<R>& work = adj.work;
         DevBuf<R>& work2 = adj.work2;
         if (use_pers) MKH_HIP(work.alloc(SN));
-        if (use_pers && driver == MKH_DRIVER_SHEET)
+        if (driver == MKH_DRIVER_SHEET || use_strand)
             MKH_HIP(work2.alloc(SN));
         /* wcur: the scratch state the persistent drivers advance (the sheet
          * writes its result to the other buffer) */
@@ -1680,7 +1828,12 @@ struct Sim : SimBase {
             Args as = a;
             as.state_a = wcur;
             int i0 = (int)s0, i1 = (int)s1;
-            if (driver == MKH_DRIVER_SHEET) {
+            if (use_strand) {
+                R* wnext = wcur == work.p ? work2.p : work.p;
+                int e = strand_launch(as, wcur, wnext, i0, i1, trajp);
+                if (e) return e;
+                wcur = wnext;
+            } else if (driver == MKH_DRIVER_SHEET) {
                 R* wnext = wcur == work.p ? work2.p : work.p;
                 as.state_b = wnext;
                 MkSheetT<R> sh = sheet_args();
@@ -1933,13 +2086,14 @@ struct Sim : SimBase {
         }
         MKH_HIP(hipEventRecord(ev[3], stream));
         MKH_HIP(hipEventSynchronize(ev[3]));
-        if (use_pers && driver == MKH_DRIVER_SHEET) {
+        if (driver == MKH_DRIVER_SHEET || (use_strand && st_halo > 0)) {
             int e = 0;
-            MKH_HIP(hipMemcpy(&e, sh_err.p, sizeof(int),
-                              hipMemcpyDeviceToHost));
+            MKH_HIP(hipMemcpy(&e, use_strand ? st_err.p : sh_err.p,
+                              sizeof(int), hipMemcpyDeviceToHost));
             if (e)
-                return fail(MKH_E_HIP, "sheet driver: a neighbour exchange "
-                                       "timed out");
+                return fail(MKH_E_HIP,
+                            std::string(use_strand ? "strand" : "sheet") +
+                                " driver: a neighbour exchange timed out");
         }
         {
             float f0 = 0, f1 = 0;
@@ -2024,8 +2178,10 @@ struct Sim : SimBase {
         if (!prog->f_adj_probe)
             return fail(MKH_E_STATE, "kernel was generated without the "
                                      "adjoint");
-        DriverAs as_grid(driver, driver == MKH_DRIVER_CHAIN ? MKH_DRIVER_GRID
-                                                            : driver);
+        DriverAs as_grid(driver, driver == MKH_DRIVER_CHAIN ||
+                                         driver == MKH_DRIVER_STRAND
+                                     ? MKH_DRIVER_GRID
+                                     : driver);
         if (cfg.coupling == MKH_COUPLING_GRAPH && driver != MKH_DRIVER_GRID &&
             driver != MKH_DRIVER_BLOCK)
             return fail(MKH_E_STATE, "graph adjoint needs the grid or block "
@@ -2486,6 +2642,12 @@ int mkh_program_build(const char* source, const char* options,
         MKH_HIP(hipModuleGetFunction(&prog->f_chain, prog->module, "mk_chain"));
         MKH_HIP(hipModuleGetFunction(&prog->f_junction, prog->module,
                                      "mk_junction"));
+        /* lines of cells and uncoupled cells, of models it can split */
+        if (hipModuleGetFunction(&prog->f_strand, prog->module,
+                                 "mk_strand") != hipSuccess) {
+            prog->f_strand = nullptr;
+            (void)hipGetLastError();
+        }
         /* present only in kernels generated with gradients */
         if (hipModuleGetFunction(&prog->f_adj_step, prog->module,
                                  "mk_adj_step") != hipSuccess ||
@@ -2506,6 +2668,7 @@ int mkh_program_build(const char* source, const char* options,
             prog->f_adj_sheet = nullptr;
             (void)hipGetLastError();
         }
+        MKH_HIP(prog->query());
         hipDeviceptr_t lp = nullptr;
         size_t lsz = 0;
         if (hipModuleGetGlobal(&lp, &lsz, prog->module, "mk_layout") ==

@@ -805,7 +805,7 @@ class SimulationOpenCL:
         """Launch configuration of the device engine (chosen automatically
         by default; :func:`myokit_amd.tune.autotune` measures and picks
         one). ``driver``: ``'auto'``, ``'cells'``, ``'block'``, ``'grid'``,
-        ``'sheet'`` or ``'chain'``; ``block_threads``: threads per
+        ``'sheet'``, ``'chain'`` or ``'strand'``; ``block_threads``: threads per
         workgroup of the cells, block and grid kernels (multiple of 64);
         ``sheet_cpt``: cells per thread of the persistent sheet (tile
         64 x 4*cpt); ``sheet_waves``: waves per SIMD its register budget
@@ -820,7 +820,8 @@ class SimulationOpenCL:
         names = {'auto': -1, 'cells': _native.DRIVER_CELLS,
                  'block': _native.DRIVER_BLOCK, 'grid': _native.DRIVER_GRID,
                  'sheet': _native.DRIVER_SHEET,
-                 'chain': _native.DRIVER_CHAIN}
+                 'chain': _native.DRIVER_CHAIN,
+                 'strand': _native.DRIVER_STRAND}
         if block_threads is not None:
             block_threads = int(block_threads)
             if block_threads % 64 or not 64 <= block_threads <= 1024:
@@ -947,7 +948,7 @@ class SimulationOpenCL:
 
     def engine_driver(self):
         """Name of the device execution driver of the last run (``cells``,
-        ``block``, ``grid``, ``sheet`` or ``chain``), or None before the
+        ``block``, ``grid``, ``sheet``, ``chain`` or ``strand``), or None before the
         first run."""
         if self._engine is None:
             return None
@@ -955,7 +956,7 @@ class SimulationOpenCL:
         _native.check(_native.lib().mkh_sim_driver(self._engine.h,
                                                    ctypes.byref(d)), 'driver')
         return {0: 'cells', 1: 'block', 2: 'grid', 3: 'sheet',
-                4: 'chain'}[d.value]
+                4: 'chain', 5: 'strand'}[d.value]
 
     def engine_timing(self, reset=False):
         """Kernel timing of the device engine (needs the ``time_kernels``
@@ -1001,7 +1002,8 @@ class SimulationOpenCL:
             chain_cells=tune.get('chain_cpt'),
             chain_budget=tune.get('chain_waves'),
             adjoint_cpt=tune.get('adjoint_cpt'),
-            grid_budget=tune.get('grid_waves'))
+            grid_budget=tune.get('grid_waves'),
+            strand=_kernelgen.strand_cells(int(coupling), self._dims))
         if len(self._sources) >= 16:
             self._sources.pop(next(iter(self._sources)))
         self._sources[gkey] = (src, cm)

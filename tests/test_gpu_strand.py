@@ -1,0 +1,110 @@
+"""
+The strand driver (lines of cells and uncoupled cells, each step shared by
+four waves) at the edges of its tiles: one tile, one cell more, tiles of 32
+and 48 cells with a short last one, runs that end on, before and after an
+exchange. Double precision against the CPU oracle bit for bit, single
+precision against the drivers that compute a whole cell per thread.
+"""
+import numpy as np
+import pytest
+
+import myokit_amd as myokit
+from tests.helpers import Scenario, run_both
+
+pytestmark = pytest.mark.gpu
+
+DT = 0.005
+
+
+def _scenario(n, field=False, rl=False, model='lr1991'):
+    rng = np.random.default_rng(n)
+    g = (rng.uniform(2, 12, n - 1), None) if field else None
+    return Scenario(model, n, rl=rl, dt=DT, gx=9.5, paced=(4, 1, 0, 0),
+                    conductance_field=g)
+
+
+@pytest.mark.parametrize('n,field,rl', [
+    (1, False, False), (2, False, False), (64, False, True),
+    (65, False, False), (97, True, False), (161, True, True),
+    (200, False, False)])
+def test_fp64_bit_exact(n, field, rl):
+    P, O = run_both(_scenario(n, field, rl), 6.0, myokit.DOUBLE_PRECISION,
+                    log_interval=0.25)
+    assert P['sim'].engine_driver() == 'strand'
+    np.testing.assert_array_equal(P['V'], O['V'])
+    np.testing.assert_array_equal(P['state'], O['state'])
+
+
+def test_fp64_other_model_and_uncoupled():
+    P, O = run_both(_scenario(70, model='br1977'), 4.0,
+                    myokit.DOUBLE_PRECISION)
+    assert P['sim'].engine_driver() == 'strand'
+    np.testing.assert_array_equal(P['state'], O['state'])
+    rng = np.random.default_rng(0)
+    sc = Scenario('lr1991', 131, diffusion=False, dt=DT,
+                  events=((1, 0, 0.5, 1000, 0),),
+                  fields={'ina.gNa': 16 * rng.uniform(0.5, 2, 131)})
+    P, O = run_both(sc, 4.0, myokit.DOUBLE_PRECISION)
+    np.testing.assert_array_equal(P['V'], O['V'])
+    np.testing.assert_array_equal(P['state'], O['state'])
+
+
+def _run(s, steps, rows):
+    v = [s.run_block(k * DT, ['membrane.V', 'ica.ICa', 'membrane.i_diff'],
+                     log_interval=rows * DT) for k in steps]
+    return [np.concatenate([b[q] for b in v]) for q in
+            ('membrane.V', 'ica.ICa', 'membrane.i_diff')] \
+        + [np.array(s.state())]
+
+
+# 8,192 cells are 256 tiles of 32, one more makes 171 of 48; 49,152 cells are
+# 1,024 tiles of 48, one more takes another driver
+@pytest.mark.parametrize('n', [33, 64, 96, 513, 8192, 8193, 49152, 49153])
+@pytest.mark.parametrize('rl', [False, True])
+def test_fp32_equals_grid_across_run_lengths(n, rl):
+    out = []
+    for driver in ('auto', 'grid'):
+        s = _scenario(n, rl=rl).product(32)
+        s.set_tuning(driver=driver)
+        out.append(_run(s, (1, 15, 16, 17, 40, 33), 7))
+        assert s.engine_driver() == (
+            'grid' if driver == 'grid' or n > 49152 else 'strand')
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize('n', [64, 65, 49152, 49153])
+def test_fp32_uncoupled_equals_cells(n):
+    out = []
+    for driver in ('auto', 'cells'):
+        rng = np.random.default_rng(1)
+        s = myokit.SimulationOpenCL(
+            myokit.load_model('example'), myokit.pacing.blocktrain(1000, 0.5),
+            ncells=n, diffusion=False)
+        s.set_step_size(DT)
+        s.set_field('ina.gNa', 16 * rng.uniform(0.5, 2, n))
+        s.set_tuning(driver=driver)
+        b = s.run_block(1.0, ['membrane.V', 'ica.ICa'], log_interval=0.2)
+        assert s.engine_driver() == 'cells'
+        out.append([b['membrane.V'], b['ica.ICa'], np.array(s.state())])
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize('n', [40, 200])
+def test_nan_ends_the_run_where_other_drivers_do(n):
+    # a NaN in cell 0 at the second log row: the same rows, time and state
+    out = []
+    for driver in ('auto', 'grid'):
+        s = _scenario(n).product(32)
+        s.set_tuning(driver=driver)
+        st = np.array(s.state()).reshape(n, -1)
+        st[0, 7] = -1e-3        # log of a negative concentration
+        s.set_state(st.reshape(-1))
+        d = s.run(2.0, log=['membrane.V', 'engine.time'], log_interval=0.1,
+                  report_nan=False)
+        out.append((np.asarray(d['engine.time']),
+                    np.asarray(d['0.membrane.V']), np.array(s.state())))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+    assert len(out[0][0]) < 20 and np.isnan(out[0][2]).any()
