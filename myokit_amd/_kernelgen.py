@@ -1066,21 +1066,37 @@ __device__ __forceinline__ float mk_powif(float x, int n)
 
 # Cells per thread of the persistent reverse sheet (MK_ACPT in the kernel
 # source; the host library reads it from mkh_sim_config.adj_cpt)
-ADJ_SHEET_CPT_CHOICES = (2, 4, 5, 6, 8)
+ADJ_SHEET_CPT_CHOICES = (1, 2, 4, 5, 6, 8)
 
 
-def adjoint_sheet_cpt(precision):
+def adjoint_sheet_cpt(precision, dims=None):
     """Cells per thread of the persistent reverse sheet (tiles of
-    64 x 4 cpt cells). Every tile is co-resident, so a CU holds its share of
-    the sheet (4,096 cells of 1024^2) and mu of those cells in LDS (32 B
-    per cell in single precision) whatever the tile size; the tile size
-    only sets how many workgroups share it. 8: two workgroups of 73 KiB
-    per CU, and the LR1991 reverse step takes 241 registers per lane
-    without spills. 4 would give four workgroups per CU (four waves per
-    SIMD) but caps the step at 128 registers, where it spills 68; 5 gives
-    three per CU, whose 768 tiles per device are fewer than the 832 a
-    1024^2 sheet needs."""
-    return 8
+    64 x 4 cpt cells) on a sheet of ``dims`` (nx, ny) cells, or 0 where the
+    one-step kernel is the faster one. A tile's cells take their reverse
+    steps one after the other, so the fewest per thread whose tiles are all
+    resident (:func:`adjoint_sheet_waves` per CU of 256). Measured on LR1991
+    (us per reverse step; 1, 2, 8 cells per thread, one-step kernel): single
+    precision 64 x 40 3.8, 6.9, 22.4, 6.2; 301 x 217 4.5, 7.1, 24.3, 7.0;
+    400 x 400 6.0, 9.3, 25.6, 10.2; 800 x 800 -, -, 32.7, 24.4; 1024 x 1024
+    -, -, 33.7, 35.8 (8 cells per thread fill every tile there: mu of 4,096
+    cells per CU in LDS); double precision 200 x 150 8.5, 15.6, 57, 10.8;
+    301 x 217 12.2, 15.9, 57, 11.8; 400 x 400 -, 23.5, 61, 23.8. Without
+    ``dims``, the tile of a small sheet."""
+    if dims is None:
+        return 1
+    if len(dims) == 2:
+        most = 256 * adjoint_sheet_waves(precision)
+
+        def fits(cpt):
+            return -(-dims[0] // 64) * -(-dims[1] // (4 * cpt)) <= most
+        cpts = (1,) if precision == DOUBLE_PRECISION else (1, 2)
+        for cpt in cpts:
+            if fits(cpt):
+                return cpt
+        if precision != DOUBLE_PRECISION and fits(8) \
+                and dims[0] * dims[1] >= 1000000:
+            return 8
+    return 0
 
 
 def adjoint_sheet_groups(cm, precision, cpt=None):
@@ -1094,6 +1110,15 @@ def adjoint_sheet_groups(cm, precision, cpt=None):
     th = 4 * cpt
     lds = len(cm.states) * th * 64 * w + (th + 2) * 66 * w + 64 + 4
     return min(4, (160 * 1024) // lds)
+
+
+def adjoint_sheet_waves(precision):
+    """Workgroups per CU (waves per SIMD) that the registers of the
+    persistent reverse sheet are budgeted for, where LDS leaves room for as
+    many: 2 in single precision, 1 in double (the LR1991 reverse step takes
+    187-232 registers per lane and 264; at 4 waves it spills, and tiles of
+    64 x 8 took 9.5 us per step instead of 7.3)."""
+    return 1 if precision == DOUBLE_PRECISION else 2
 
 
 def adjoint_waves_default(cm, precision, adjoint_precision=None):
@@ -1236,6 +1261,9 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
     real = 'double' if precision == DOUBLE_PRECISION else 'float'
     acpt = adjoint_sheet_cpt(precision) if adjoint_cpt is None \
         else int(adjoint_cpt)
+    # 0: the reverse pass takes the one-step kernel
+    persistent = acpt != 0
+    acpt = acpt or 1
     if acpt not in ADJ_SHEET_CPT_CHOICES:
         raise ValueError('adjoint_cpt must be one of '
                          + str(ADJ_SHEET_CPT_CHOICES) + '.')
@@ -1262,10 +1290,12 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         '#define MK_ACPT ' + str(acpt),
         '#define MK_GBLOCKS ' + str(gblocks),
         '#define MK_ADJ_SHEET ' + ('1' if adjoint and int(coupling) == 1
-                                   and asg > 0
+                                   and asg > 0 and persistent
                                    and adjoint_precision in (None, precision)
                                    else '0'),
         '#define MK_ADJ_SWAVES ' + str(max(1, asg)),
+        '#define MK_ADJ_SREG ' + str(max(1, min(asg, adjoint_sheet_waves(
+            precision)))),
         '#define MK_ADJ_WAVES ' + str(max(1, int(
             adjoint_waves_default(cm, precision, adjoint_precision)
             if adjoint_waves is None else adjoint_waves))),

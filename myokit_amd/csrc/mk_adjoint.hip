@@ -50,19 +50,20 @@ __device__ __forceinline__ double mk_block_sum(double v, double* lds)
     return r;
 }
 
-/* Coupling transpose at cell c for abar_{s+1} (ab) and V(y_{s+1}) (V1):
- * returns sum_j g_cj (ab[c] - ab[j]) and adds the cell's terms of dL/dgx and
- * dL/dgy (graphs: dL/dscale, half from each end of a connection) to cx,
- * cy. Arrays are indexed as in the forward coupling: by cell on a grid or
- * a single stencil domain; graphs by CSR row `row` with neighbour indices
- * relative to the arrays, the cell itself at `self`. */
+/* Coupling transpose at cell c of a grid or a single stencil domain for
+ * abar_{s+1} (ab) and V(y_{s+1}) (V1): returns sum_j g_cj (ab[c] - ab[j]) and
+ * adds the cell's terms of dL/dgx and dL/dgy to cx, cy. Arrays are indexed
+ * as in the forward coupling. (Taking those terms from V(y_s) in the same
+ * step, as the graphs do, reads less but measured slower on sheets: 36 -> 39
+ * us per step of mk_adj_step on 1024 x 1024 cells, 33.5 -> 35.7 of
+ * mk_adj_sheet.) */
 __device__ __forceinline__ Real mk_adj_couple(
     const MkArgs& a, const Real* __restrict__ V1, const Real* __restrict__ ab,
-    int c, int row, int self, int ix, int iy, int nx, int ny, double& cx,
-    double& cy)
+    int c, int ix, int iy, int nx, int ny, double& cx, double& cy)
 {
     Real lv = (Real)0;
-    (void)row; (void)self; (void)ix; (void)iy; (void)c; (void)nx; (void)ny;
+    (void)ix; (void)iy; (void)c; (void)nx; (void)ny; (void)V1; (void)ab;
+    (void)cx; (void)cy;
 #if MK_COUPLING == 1
     const Real ac = ab[c], v = V1[c];
     Real ax = (Real)0, ay = (Real)0, xs = (Real)0, ys = (Real)0;
@@ -87,8 +88,30 @@ __device__ __forceinline__ Real mk_adj_couple(
         if (iy > 0) lv += a.gy_field[c - nx] * (ac - ab[c - nx]);
         if (iy < ny - 1) lv += a.gy_field[c] * (ac - ab[c + nx]);
     }
-#elif MK_COUPLING == 3
-    const Real ac = ab[self], v = V1[self];
+#endif
+    return lv;
+}
+
+#if MK_COUPLING == 3
+/* One walk of a cell's connections: returns the coupling transpose at
+ * abar_{s+1} (ab; 0 if ab is NULL) and sets idiff to the forward current at
+ * V(y_s) (V0) and dscale to that current's derivative by a common scale of
+ * the conductances, in double precision: the gradient of the scale is
+ * sum_s sum_c abar_s[c] dscale_s[c], with the cell's own abar_s (summed per
+ * connection instead, 1/2 g (abar_c - abar_j)(V_c - V_j) from each end, the
+ * walk would also gather the neighbours' potentials of y_{s+1}: 77.7 ->
+ * 72.3 us per step on 16 copies of 100,000 cells). The cell's row is `row`, the cell
+ * itself is at `self` of the arrays, which neighbour indices are relative
+ * to. Each sum takes the connections in list order, as mk_graph does, four
+ * at a time with their loads in flight together. */
+__device__ __forceinline__ Real mk_adj_couple_graph(
+    const MkArgs& a, const Real* __restrict__ ab, const Real* __restrict__ V0,
+    int row, int self, Real& idiff, double& dscale)
+{
+    const Real v0 = V0[self];
+    const Real ac = ab ? ab[self] : (Real)0;
+    Real lv = (Real)0, id = (Real)0;
+    double ds = 0.0;
     /* rows of one copy for a graph of interleaved copies (see mk_graph) */
     const int K = a.gcopies;
     int lane = 0;
@@ -98,77 +121,22 @@ __device__ __forceinline__ Real mk_adj_couple(
     }
     int e = a.csr_ptr[row];
     const int e1 = a.csr_ptr[row + 1];
-    /* four connections per round, loads first, sums in list order (as in
-     * mk_graph) */
-    for (; e + 4 <= e1; e += 4) {
-        int nb[4];
-        Real gg[4], an[4], vn[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int t = a.csr_idx[e + k];
-            nb[k] = (t < 0 ? ~t : t) * K + lane;
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            gg[k] = a.csr_g[e + k];
-            an[k] = ab[nb[k]];
-            vn[k] = V1[nb[k]];
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            lv += gg[k] * (ac - an[k]);
-            cx += 0.5 * (double)gg[k] * ((double)ac - (double)an[k])
-                  * ((double)v - (double)vn[k]);
-        }
-    }
-    for (; e < e1; ++e) {
-        int nb = a.csr_idx[e];
-        if (nb < 0) nb = ~nb;
-        nb = nb * K + lane;
-        const Real g = a.csr_g[e];
-        lv += g * (ac - ab[nb]);
-        cx += 0.5 * (double)g * ((double)ac - (double)ab[nb])
-              * ((double)v - (double)V1[nb]);
-    }
-#endif
-    return lv;
-}
-
-#if MK_COUPLING == 3
-/* mk_adj_couple and mk_graph in one walk of graph row c (the one-step
- * kernel: row = self = c): returns the coupling transpose at abar_{s+1}
- * (ab) and V(y_{s+1}) (V1), adds the cell's dL/dscale terms to cx, and
- * sets idiff to the forward current at V(y_s) (V0). Each sum takes the
- * same additions in the same order as in the separate walks. */
-__device__ __forceinline__ Real mk_adj_couple_graph(
-    const MkArgs& a, const Real* __restrict__ V1, const Real* __restrict__ ab,
-    const Real* __restrict__ V0, int c, double& cx, Real& idiff)
-{
-    const Real ac = ab[c], v = V1[c], v0 = V0[c];
-    Real lv = (Real)0, id = (Real)0;
-    /* rows of one copy for a graph of interleaved copies (see mk_graph) */
-    const int K = a.gcopies;
-    const int row = K > 1 ? c / K : c, lane = c - row * K;
-    int e = a.csr_ptr[row];
-    const int e1 = a.csr_ptr[row + 1];
     for (; e + 4 <= e1; e += 4) {
         int t[4];
-        Real gg[4], an[4], vn[4], wn[4];
+        Real gg[4], an[4], wn[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) t[k] = a.csr_idx[e + k];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int nb = (t[k] < 0 ? ~t[k] : t[k]) * K + lane;
             gg[k] = a.csr_g[e + k];
-            an[k] = ab[nb];
-            vn[k] = V1[nb];
+            an[k] = ab ? ab[nb] : (Real)0;
             wn[k] = V0[nb];
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             lv += gg[k] * (ac - an[k]);
-            cx += 0.5 * (double)gg[k] * ((double)ac - (double)an[k])
-                  * ((double)v - (double)vn[k]);
+            ds += (double)gg[k] * ((double)v0 - (double)wn[k]);
             if (t[k] >= 0) id = id + gg[k] * (v0 - wn[k]);
             else id = id - gg[k] * (wn[k] - v0);
         }
@@ -176,14 +144,14 @@ __device__ __forceinline__ Real mk_adj_couple_graph(
     for (; e < e1; ++e) {
         const int t = a.csr_idx[e];
         const int nb = (t < 0 ? ~t : t) * K + lane;
-        const Real g = a.csr_g[e];
-        lv += g * (ac - ab[nb]);
-        cx += 0.5 * (double)g * ((double)ac - (double)ab[nb])
-              * ((double)v - (double)V1[nb]);
-        if (t >= 0) id = id + g * (v0 - V0[nb]);
-        else id = id - g * (V0[nb] - v0);
+        const Real g = a.csr_g[e], w = V0[nb];
+        if (ab) lv += g * (ac - ab[nb]);
+        ds += (double)g * ((double)v0 - (double)w);
+        if (t >= 0) id = id + g * (v0 - w);
+        else id = id - g * (w - v0);
     }
     idiff = id;
+    dscale = ds;
     return lv;
 }
 #endif
@@ -200,22 +168,19 @@ __device__ __forceinline__ Real mk_adj_loss(const MkAdj& j, int c, Real v,
     return (Real)(2.0 * d);
 }
 
-/* Cell VJP of step p at state y (own cell), V the potentials of y_s indexed
- * as in the forward coupling. */
+/* Cell VJP of step p at state y (own cell) of a grid or a single stencil
+ * domain, V the potentials of y_s indexed as in the forward coupling. */
 __device__ __forceinline__ void mk_adj_cell(
     const MkArgs& a, const MkStep& p, const Real* y, const Real* fv,
-    const Real* __restrict__ V, int c, int row, int self, int ix, int iy,
-    int nx, int ny, const Real* lam, Real* mu, Real& abo, Real* fb)
+    const Real* __restrict__ V, int c, int ix, int iy, int nx, int ny,
+    const Real* lam, Real* mu, Real& abo, Real* fb)
 {
-    (void)row; (void)self; (void)nx; (void)ny;
+    (void)nx; (void)ny;
 #if MK_COUPLING == 1
     const Real idiff = mk_stencil(V, c, ix, iy, nx, ny, a.gx, a.gy);
 #elif MK_COUPLING == 2
     const Real idiff = mk_hetero(V, a.gx_field, a.gy_field, c, ix, iy, nx,
                                  ny);
-#elif MK_COUPLING == 3
-    const Real idiff = mk_graph(V, a.csr_ptr, a.csr_idx, a.csr_g, row, self,
-                                a.gcopies);
 #else
     const Real idiff = (Real)0;
     (void)V;
@@ -247,18 +212,15 @@ mk_adj_step(const MkArgs a, const MkAdj j, const int s)
         const Real* __restrict__ V1 = j.yn1 + MK_IVM * np;
         Real lv = mk_adj_loss(j, c, V1[c], j.target_row);
 #if MK_COUPLING == 3
-        /* both walks of the cell's connections in one */
-        Real idiff0 = (Real)0;
-        const bool fused = j.ab_in && j.yn;
-        if (fused)
-            lv += mk_adj_couple_graph(a, V1, j.ab_in, j.yn + MK_IVM * np, c,
-                                      cx, idiff0);
-        else if (j.ab_in)
+        /* the forward current, with the transpose of the coupling */
+        Real idiff0;
+        double ds;
+        lv += mk_adj_couple_graph(a, j.ab_in, j.yn + MK_IVM * np, c, c,
+                                  idiff0, ds);
 #else
         if (j.ab_in)
+            lv += mk_adj_couple(a, V1, j.ab_in, c, ix, iy, nx, ny, cx, cy);
 #endif
-            lv += mk_adj_couple(a, V1, j.ab_in, c, c, c, ix, iy, nx, ny, cx,
-                                cy);
         lam[MK_IVM] += lv;
         if (j.yn) {
             Real y[MK_NS], mu[MK_NS], fv[MK_NFA], fb[MK_NFA], abo;
@@ -268,19 +230,17 @@ mk_adj_step(const MkArgs a, const MkAdj j, const int s)
 #pragma unroll
             for (int k = 0; k < MK_NF; ++k) fv[k] = a.fields[k * np + c];
 #if MK_COUPLING == 3
-            if (!fused)
-                idiff0 = mk_graph(j.yn + MK_IVM * np, a.csr_ptr, a.csr_idx,
-                                  a.csr_g, c, c, a.gcopies);
             {
                 const MkStep& p = a.steps[s];
                 const Real pace = mk_is_paced(a, c, ix, iy) ? p.pace
                                                             : (Real)0;
                 mk_cell_vjp(y, p.t, p.dt, pace, idiff0, fv, lam, mu, &abo,
                             fb);
+                cx = (double)abo * ds;
             }
 #else
-            mk_adj_cell(a, a.steps[s], y, fv, j.yn + MK_IVM * np, c, c, c, ix,
-                        iy, nx, ny, lam, mu, abo, fb);
+            mk_adj_cell(a, a.steps[s], y, fv, j.yn + MK_IVM * np, c, ix, iy,
+                        nx, ny, lam, mu, abo, fb);
 #endif
             Real* __restrict__ mo = j.mu_out + c;
 #pragma unroll
@@ -291,7 +251,7 @@ mk_adj_step(const MkArgs a, const MkAdj j, const int s)
         }
     }
 #if MK_COUPLING == 1 || MK_COUPLING == 3
-    if (j.ab_in) {
+    if (MK_COUPLING == 3 || j.ab_in) {
         const double sx = mk_block_sum(cx, red[0]);
         const double sy = mk_block_sum(cy, red[1]);
         if (threadIdx.x == 0) {
@@ -349,15 +309,22 @@ mk_adj_block(const MkArgs a, const MkAdj j, const int s0, const int s1,
                                       : (int)(off + li);
             const int iy = (int)((unsigned)c / (unsigned)nx);
             const int ix = c - iy * nx;
-            const int row = (int)(off + li);
             Real lam[MK_NS], y[MK_NS], mu[MK_NS], fv[MK_NFA], fb[MK_NFA], abo;
 #pragma unroll
             for (int i = 0; i < MK_NS; ++i)
                 lam[i] = fresh ? (Real)0 : j.mu_out[(long long)i * a.npad + c];
             Real lv = mk_adj_loss(j, c, vsh[cur][li], s);
+#if MK_COUPLING == 3
+            Real idiff;
+            double ds;
+            lv += mk_adj_couple_graph(a, fresh ? nullptr : ash[cur],
+                                      vsh[cur ^ 1], (int)(off + li), li,
+                                      idiff, ds);
+#else
             if (!fresh)
-                lv += mk_adj_couple(a, vsh[cur], ash[cur], li, row, li, ix,
-                                    iy, nx, ny, cx, cy);
+                lv += mk_adj_couple(a, vsh[cur], ash[cur], li, ix, iy, nx, ny,
+                                    cx, cy);
+#endif
             lam[MK_IVM] += lv;
 #pragma unroll
             for (int i = 0; i < MK_NS; ++i)
@@ -365,8 +332,14 @@ mk_adj_block(const MkArgs a, const MkAdj j, const int s0, const int s1,
 #pragma unroll
             for (int k = 0; k < MK_NF; ++k)
                 fv[k] = a.fields[(long long)k * a.npad + c];
-            mk_adj_cell(a, p, y, fv, vsh[cur ^ 1], li, row, li, ix, iy, nx,
-                        ny, lam, mu, abo, fb);
+#if MK_COUPLING == 3
+            const Real pace = mk_is_paced(a, c, ix, iy) ? p.pace : (Real)0;
+            mk_cell_vjp(y, p.t, p.dt, pace, idiff, fv, lam, mu, &abo, fb);
+            cx += (double)abo * ds;
+#else
+            mk_adj_cell(a, p, y, fv, vsh[cur ^ 1], li, ix, iy, nx, ny, lam,
+                        mu, abo, fb);
+#endif
 #pragma unroll
             for (int i = 0; i < MK_NS; ++i)
                 j.mu_out[(long long)i * a.npad + c] = mu[i];
@@ -384,8 +357,8 @@ mk_adj_block(const MkArgs a, const MkAdj j, const int s0, const int s1,
         const int c = a.dom_cells ? a.dom_cells[off + li] : (int)(off + li);
         if (first_seg) {
             const int iy = (int)((unsigned)c / (unsigned)nx);
-            (void)mk_adj_couple(a, vsh[cur], ash[cur], li, (int)(off + li),
-                                li, c - iy * nx, iy, nx, ny, cx, cy);
+            (void)mk_adj_couple(a, vsh[cur], ash[cur], li, c - iy * nx, iy,
+                                nx, ny, cx, cy);
         } else {
             j.ab_out[c] = ash[cur][li];
         }
@@ -437,7 +410,7 @@ mk_adj_gather(const double* __restrict__ src,
  * Each workgroup owns a tile of 64 x MK_ATH cells (MK_ATH = 4 * MK_ACPT);
  * thread (lx, w) handles cells (x0 + lx, y0 + w * MK_ACPT + k), k <
  * MK_ACPT, one after the other. MK_ADJ_SWAVES workgroups per CU fit into
- * LDS, and the registers are budgeted for as many waves per SIMD. mu of the tile stays in LDS for the whole
+ * LDS; the registers are budgeted for MK_ADJ_SREG of them. mu of the tile stays in LDS for the whole
  * segment, abar of the tile and a one-cell ring around it too. The
  * potentials V_s and V_{s+1} come from the trajectory, complete in global
  * memory, so only abar crosses tiles: after each step a tile stores the
@@ -551,7 +524,7 @@ __device__ __forceinline__ bool mk_adj_sheet_halo(
     __syncthreads();
     return !*flag;
 }
-extern "C" __global__ void __launch_bounds__(256, MK_ADJ_SWAVES)
+extern "C" __global__ void __launch_bounds__(256, MK_ADJ_SREG)
 mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
              const int s1, const int flags)
 {
@@ -568,6 +541,10 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
     const int ix = tx * 64 + lx, gy0 = ty * MK_ATH;
     const long long np = a.npad;
     const long long SN = (long long)MK_NS * np;
+    /* lanes beyond the last column compute a copy of its cell and keep it to
+     * themselves (waves of at most 8 active lanes are slow, see mk_sheet) */
+    const bool own = ix < nx;
+    const int xc = own ? ix : nx - 1;
     const int nb[4] = {ty > 0 ? tile - sh.tiles_x : -1,
                        ty + 1 < sh.tiles_y ? tile + sh.tiles_x : -1,
                        tx > 0 ? tile - 1 : -1,
@@ -629,8 +606,8 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
 #pragma unroll 1
         for (int k = 0; k < MK_ACPT; ++k) {
             const int r = w * MK_ACPT + k, iy = gy0 + r;
-            if (!(ix < nx && iy < ny)) continue;
-            const int c = ix + iy * nx;
+            if (iy >= ny) continue;
+            const int c = xc + iy * nx;
             Real lam[MK_NS], y[MK_NS], mu[MK_NS], fv[MK_NFA], fb[MK_NFA], abo;
 #pragma unroll
             for (int q = 0; q < MK_NS; ++q) {
@@ -639,17 +616,17 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
             }
 #pragma unroll
             for (int f = 0; f < MK_NF; ++f) fv[f] = a.fields[f * np + c];
-            Real lv = mk_adj_loss(j, c, V1[c], s);
+            Real lv = mk_adj_loss(j, c, V1[c], own ? s : -1);
             Real ck = (Real)0;
 #pragma unroll
             for (int q = 0; q < MK_ACPT; ++q) if (q == k) ck = lc[q];
             lv += ck;
             lam[MK_IVM] += lv;
-            mk_adj_cell(a, p, y, fv, V0, c, c, c, ix, iy, nx, ny, lam, mu, abo,
-                        fb);
+            mk_adj_cell(a, p, y, fv, V0, c, xc, iy, nx, ny, lam, mu, abo, fb);
 #pragma unroll
             for (int q = 0; q < MK_NS; ++q) mul[q][r][lx] = mu[q];
             at[r + 1][lx + 1] = abo;
+            if (!own) continue;
             if (r == 0) mk_tput(mk_adj_edge(sh, par, tile, 0, lx), abo, i + 1);
             if (r == MK_ATH - 1)
                 mk_tput(mk_adj_edge(sh, par, tile, 1, lx), abo, i + 1);

@@ -434,7 +434,10 @@ struct Sim : SimBase {
             sh_tx = (int)((cfg.nx + 63) / 64);
             sh_ty = (int)((cfg.ny + th - 1) / th);
             if ((long long)sh_tx * sh_ty <= sh_capacity) {
-                const size_t nt = (size_t)sh_tx * sh_ty;
+                /* the reverse sheet shares the edge words */
+                const size_t nt = (size_t)std::max<long long>(
+                    (long long)sh_tx * sh_ty,
+                    p->f_adj_sheet ? adj_sheet_tiles() : 0);
                 MKH_HIP(sh_edges.alloc(2 * nt * 4 * 64 * XW));
                 MKH_HIP(sh_err.alloc(1));
                 MKH_HIP(hipMemset(sh_edges.p, 0,
@@ -531,6 +534,13 @@ struct Sim : SimBase {
                                           nullptr));
         }
         return 0;
+    }
+
+    /* Tiles of the persistent reverse sheet (64 x 4 adj_cpt cells). */
+    long long adj_sheet_tiles() const
+    {
+        const long long th = 4 * std::max(cfg.adj_cpt, 1);
+        return (long long)sh_tx * ((cfg.ny + th - 1) / th);
     }
 
     /* Whether driver d can run this geometry and coupling: the block
@@ -1681,11 +1691,16 @@ struct Sim : SimBase {
         const unsigned ggrid = grid_launch_size();
         const unsigned cgrid = (unsigned)((n + bt - 1) / bt);
         /* conductance-gradient partial sums: one per workgroup of the
-         * reverse kernel (per domain on the block layout) */
+         * reverse kernel (per domain on the block layout, per tile on the
+         * sheet) */
         const size_t nparts =
-            std::max<size_t>(cgrid, driver == MKH_DRIVER_BLOCK
-                                        ? (size_t)std::max<long long>(1, ndom)
-                                        : 1);
+            std::max<size_t>({(size_t)cgrid,
+                              driver == MKH_DRIVER_BLOCK
+                                  ? (size_t)std::max<long long>(1, ndom)
+                                  : 1,
+                              driver == MKH_DRIVER_SHEET
+                                  ? (size_t)adj_sheet_tiles()
+                                  : 1});
         DevBuf<Step>& dsteps = adj.steps;
         DevBuf<R>& ckpt = adj.ckpt;
         DevBuf<R>& traj = adj.traj;
@@ -1782,11 +1797,9 @@ struct Sim : SimBase {
                               driver == MKH_DRIVER_CELLS || use_strand;
         const bool block_rev = driver == MKH_DRIVER_BLOCK;
         /* The persistent reverse sheet: 64 x 4 adj_cpt tiles (MK_ACPT in
-         * the kernel source), all co-resident; they are no more than the
-         * forward sheet's (4 * sheet_cpt rows), whose edge buffer they use */
+         * the kernel source), all co-resident */
         const int rtx = sh_tx;
-        const int ath = 4 * std::max(cfg.adj_cpt, 1);
-        const int rty = (int)((cfg.ny + ath - 1) / ath);
+        const int rty = sh_tx > 0 ? (int)(adj_sheet_tiles() / sh_tx) : 0;
         bool sheet_rev = false;
         if (driver == MKH_DRIVER_SHEET && cfg.adj_cpt > 0 &&
             prog->f_adj_sheet &&
@@ -2079,8 +2092,10 @@ struct Sim : SimBase {
                 if (e) return e;
             }
         }
-        /* closing pass: conductance terms of step 0 (y_0 is slot 0) */
-        if (!block_rev && !sheet_rev) {
+        /* closing pass: conductance terms of step 0 (y_0 is slot 0); a
+         * graph's are taken in the step itself */
+        if (!block_rev && !sheet_rev &&
+            cfg.coupling != MKH_COUPLING_GRAPH) {
             int e = reverse_step(nullptr, slot(0), 0, -1);
             if (e) return e;
         }

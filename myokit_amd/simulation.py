@@ -918,6 +918,13 @@ class SimulationOpenCL:
         return self._tuning.get('sheet_cpt') or _kernelgen.sheet_cpt(
             self._precision, self._dims, self._nstate)
 
+    def _adjoint_cpt(self):
+        """Cells per thread of the persistent reverse sheet: the value given
+        to :meth:`set_tuning`, else the one for this sheet's size (0: the
+        reverse pass takes the one-step kernel)."""
+        return self._tuning.get('adjoint_cpt') or \
+            _kernelgen.adjoint_sheet_cpt(self._precision, self._dims)
+
     def tuning(self):
         """The current launch configuration (see :meth:`set_tuning`)."""
         return {'driver': self._tuning.get('driver', 'auto'),
@@ -931,9 +938,7 @@ class SimulationOpenCL:
                 'chain_waves': self._tuning.get(
                     'chain_waves', _kernelgen.chain_waves(self._precision)),
                 'adjoint_waves': self._tuning.get('adjoint_waves'),
-                'adjoint_cpt': self._tuning.get(
-                    'adjoint_cpt',
-                    _kernelgen.adjoint_sheet_cpt(self._precision)),
+                'adjoint_cpt': self._adjoint_cpt() or None,
                 'grid_waves': self._tuning.get(
                     'grid_waves', _kernelgen.grid_waves(self._precision))}
 
@@ -1001,7 +1006,7 @@ class SimulationOpenCL:
             adjoint_waves=tune.get('adjoint_waves'),
             chain_cells=tune.get('chain_cpt'),
             chain_budget=tune.get('chain_waves'),
-            adjoint_cpt=tune.get('adjoint_cpt'),
+            adjoint_cpt=self._adjoint_cpt(),
             grid_budget=tune.get('grid_waves'),
             strand=_kernelgen.strand_cells(int(coupling), self._dims))
         if len(self._sources) >= 16:
@@ -1070,8 +1075,7 @@ class SimulationOpenCL:
             else 0
         cfg.chain_cpt = tune.get('chain_cpt') or \
             _kernelgen.chain_cpt(self._precision)
-        cfg.adj_cpt = tune.get('adjoint_cpt') or \
-            _kernelgen.adjoint_sheet_cpt(self._precision)
+        cfg.adj_cpt = self._adjoint_cpt()
         eng = _Engine(prog, cfg)
         eng.options = {}
         eng.config_version = None

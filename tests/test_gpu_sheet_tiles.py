@@ -54,3 +54,29 @@ def test_fp32_every_tile_height_equals_grid(cpt, field):
             V.append((b['membrane.V'], np.array(s.state())))
         np.testing.assert_array_equal(V[0][0], V[1][0])
         np.testing.assert_array_equal(V[0][1], V[1][1])
+
+
+@pytest.mark.parametrize('shape', SHAPES)
+@pytest.mark.parametrize('cpt', [1, 2, 8])
+def test_reverse_sheet_edges_equal_one_step_kernel(shape, cpt):
+    # double precision: the loss and the field gradients bit for bit, the
+    # conductances' (whose terms are grouped by tile) to 1e-12
+    from myokit_amd.adjoint import TissueAdjoint
+    nx, ny = shape
+    res = []
+    for sheet in (1, 0):
+        s = _scenario(shape, False).product(64)
+        s.set_field('ina.gNa', np.linspace(14, 18, nx * ny).reshape(ny, nx))
+        s.set_tuning(adjoint_cpt=cpt)
+        s.set_engine_option('adj_sheet', sheet)
+        adj = TissueAdjoint(s, [(0, 0), (nx - 1, ny - 1)],
+                            checkpoint_every=23)
+        target = np.full((adj.n_steps(0.6), 2), -40.0)
+        loss, g, dgx, dgy = adj.loss_and_gradient(0.6, target)
+        kind = adj.reverse_kernel()[0]
+        assert (kind == 'sheet') == bool(sheet), kind
+        res.append((loss, g['ina.gNa'].copy(), dgx, dgy))
+    assert res[0][0] == res[1][0]
+    np.testing.assert_array_equal(res[0][1], res[1][1])
+    assert res[0][2] == pytest.approx(res[1][2], rel=1e-12)
+    assert res[0][3] == pytest.approx(res[1][3], rel=1e-12)

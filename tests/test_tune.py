@@ -139,3 +139,24 @@ def test_sheet_tiles_follow_the_size():
             == k.sheet_waves(prec, 4)
     assert sim((100, 70)).tuning()['sheet_cpt'] == 1
     assert sim((1024, 1024)).tuning()['sheet_cpt'] == 4
+
+
+def test_reverse_sheet_tiles_follow_the_size():
+    from myokit_amd import _kernelgen as k
+    for prec, most in ((32, 512), (64, 256)):
+        assert k.adjoint_sheet_waves(prec) * 256 == most
+        assert k.adjoint_sheet_cpt(prec) == 1
+        assert k.adjoint_sheet_cpt(prec, (64, 4 * most)) == 1
+        assert k.adjoint_sheet_cpt(prec, (1000, 1)) == 1
+        assert k.adjoint_sheet_cpt(prec, (1000,)) == 0
+    assert k.adjoint_sheet_cpt(64, (64, 1025)) == 0
+    assert k.adjoint_sheet_cpt(32, (64, 2049)) == 2
+    assert k.adjoint_sheet_cpt(32, (65, 2049)) == 0
+    assert k.adjoint_sheet_cpt(32, (1024, 1024)) == 8
+    assert k.adjoint_sheet_cpt(32, (1025, 1024)) == 0
+    # 0 leaves the persistent kernel out of the text
+    s = sim((800, 800), rl=True)
+    assert s.tuning()['adjoint_cpt'] is None
+    cm = k.CellModel(s._model, s._bound_variables, s._rl_states, [], [])
+    src = k.generate_kernel(cm, 32, 1, adjoint=True, adjoint_cpt=0)
+    assert '#define MK_ADJ_SHEET 0' in src
