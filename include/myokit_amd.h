@@ -209,6 +209,9 @@ int mkh_sim_clean(void* sim);
  *   "adj_overlap"   0: recompute earlier segments in line with the reverse
  *                   steps, also where a second stream could overlap them
  *                   (default 1)
+ *   "adj_linear"    0: keep lines of cells and uncoupled cells in double
+ *                   precision on the reverse kernels that apply the cell
+ *                   VJP step by step (default 1)
  *   "graph_copies"  K: the next graph is K identical copies held
  *                   interleaved (cell p of copy k is cell p * K + k), the
  *                   copies' connection lists one after the other; if every
@@ -269,6 +272,10 @@ int mkh_adj_timing(void* sim, double* ms3);
 #define MKH_ADJ_REV_BLOCK 1
 #define MKH_ADJ_REV_SHEET 2
 #define MKH_ADJ_REV_STEP_OVERLAP 3
+/* two launches per range of steps: the Jacobians of all its steps, then the
+ * products with them in turn (lines of cells and uncoupled cells, double
+ * precision) */
+#define MKH_ADJ_REV_LINEAR 4
 int mkh_adj_reverse(void* sim, int* kind, long long* launches);
 
 /* The caller's cell order for mkh_adj_run's field gradients: caller cell c

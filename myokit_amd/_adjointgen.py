@@ -789,3 +789,88 @@ def _vjp_source(cm, precision, islands=True):
         lines.append(tab + 'fbar[' + str(k) + '] = bf' + str(k) + ';')
     lines.append('}')
     return '\n'.join(lines) + '\n'
+
+
+# Most entries per cell and step of the linear reverse pass (its kernel keeps
+# those of several steps in registers)
+LINEAR_ENTRIES = 64
+
+
+def jacobian_pattern(cm):
+    """What the step of each state depends on, from the equations alone:
+    ``(states, fields, idiff)``, per state a set of state indices, a set of
+    field indices and whether it depends on the diffusion current."""
+    index = {s: i for i, s in enumerate(cm.states)}
+    findex = {v: k for k, v in enumerate(cm.fields)}
+    memo = {}
+
+    def of_refs(e):
+        out = set()
+        for r in e.references():
+            v = r.var()
+            if isinstance(r, ex.Derivative):
+                out |= of_var(v)
+            elif v in index:
+                out.add(('x', index[v]))
+            elif v in findex:
+                out.add(('f', findex[v]))
+            elif v in cm.bound:
+                if cm.bound[v] == 'idiff':
+                    out.add(('d', 0))
+            elif v not in cm.constants:
+                out |= of_var(v)
+        return out
+
+    def of_var(v):
+        if v not in memo:
+            memo[v] = of_refs(v.rhs())
+        return memo[v]
+    states, fields, idiff = [], [], []
+    for i, s in enumerate(cm.states):
+        if s in cm.rl_states:
+            d = set()
+            for v in cm.rl_states[s]:
+                d |= of_var(v)
+        else:
+            d = set(of_var(s))
+        d.add(('x', i))
+        states.append(set(k for what, k in d if what == 'x'))
+        fields.append(set(k for what, k in d if what == 'f'))
+        idiff.append(('d', 0) in d)
+    return states, fields, idiff
+
+
+def generate_jacobian_tables(cm):
+    """The tables of the linear reverse pass (``mk_adj_jac``,
+    ``mk_adj_lin``): which entries of a cell step's Jacobian exist
+    (``mk_jmask[i]`` bit j: state i' depends on state j; ``mk_fmask[i]`` on
+    field k; ``mk_dmask`` bit i: on the diffusion current), and where a
+    row's entries start. Returns ``(text, entries)``; the entries include
+    two more per cell and step (the loss term and dI/dgx)."""
+    states, fields, idiff = jacobian_pattern(cm)
+    jm = [sum(1 << j for j in s) for s in states]
+    fm = [sum(1 << k for k in f) for f in fields]
+    jr, fr, n = [], [], 0
+    for s in states:
+        jr.append(n)
+        n += len(s)
+    nj = n
+    for f in fields:
+        fr.append(n)
+        n += len(f)
+    dm = sum(1 << i for i, d in enumerate(idiff) if d)
+    nd = sum(idiff)
+    d0 = n
+    n += nd + 2
+
+    def table(kind, name, values, suffix=''):
+        return ('__device__ constexpr ' + kind + ' ' + name + '[MK_NS] = {'
+                + ', '.join(str(v) + suffix for v in values) + '};')
+    u = 'unsigned long long'
+    return '\n'.join([
+        '#define MK_NE ' + str(n), '#define MK_NJ ' + str(nj),
+        '#define MK_D0 ' + str(d0),
+        table(u, 'mk_jmask', jm, 'ull'), table(u, 'mk_fmask', fm, 'ull'),
+        table('int', 'mk_jrow', jr), table('int', 'mk_frow', fr),
+        '__device__ constexpr ' + u + ' mk_dmask = ' + str(dm) + 'ull;',
+    ]) + '\n', n

@@ -1310,8 +1310,19 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         _read('mk_drivers.hip'),
     ]
     if adjoint:
-        from ._adjointgen import generate_vjp_function
-        parts.append(generate_vjp_function(cm, precision, adjoint_precision))
+        from . import _adjointgen
+        parts.append(_adjointgen.generate_vjp_function(cm, precision,
+                                                       adjoint_precision))
+        # the linear reverse pass: double precision, where the strand driver
+        # may run
+        lin = precision == DOUBLE_PRECISION and strand \
+            and int(coupling) != 3 and len(cm.states) <= 64
+        if lin:
+            tables, entries = _adjointgen.generate_jacobian_tables(cm)
+            lin = entries <= _adjointgen.LINEAR_ENTRIES
+        parts.append('#define MK_ADJ_LIN ' + str(int(lin)))
+        if lin:
+            parts.append(tables)
         parts.append(_read('mk_adjoint.hip'))
     return '\n'.join(parts)
 

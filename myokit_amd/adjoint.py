@@ -157,18 +157,21 @@ class TissueAdjoint:
 
     def reverse_kernel(self):
         """The reverse kernel of the last ``loss_and_gradient`` and its
-        number of launches: ``('step' | 'step-overlap' | 'block' | 'sheet',
-        launches)``, or ``(None, 0)`` before the first call. 'step-overlap'
-        is the one-step kernel with each earlier segment recomputed on a
-        second stream while the later one's reverse steps run (small
-        domains)."""
+        number of launches: ``('step' | 'step-overlap' | 'block' | 'sheet'
+        | 'linear', launches)``, or ``(None, 0)`` before the first call.
+        'step-overlap' is the one-step kernel with each earlier segment
+        recomputed on a second stream while the later one's reverse steps
+        run (small domains); 'linear' evaluates the Jacobians of a range of
+        steps together and then only multiplies by them step by step (lines
+        of cells and uncoupled cells in double precision)."""
         eng = getattr(self, '_eng', None)
         if eng is None:
             return None, 0
         kind, n = ctypes.c_int(-1), ctypes.c_longlong(0)
         _native.check(_native.lib().mkh_adj_reverse(
             eng.h, ctypes.byref(kind), ctypes.byref(n)), 'mkh_adj_reverse')
-        names = {0: 'step', 1: 'block', 2: 'sheet', 3: 'step-overlap'}
+        names = {0: 'step', 1: 'block', 2: 'sheet', 3: 'step-overlap',
+                 4: 'linear'}
         return names.get(kind.value), n.value
 
     def release(self):

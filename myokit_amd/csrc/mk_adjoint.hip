@@ -681,3 +681,294 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
     }
 }
 #endif
+
+#if MK_ADJ_LIN
+/* ------------------------------------------------------------------------
+ * Linear reverse pass: a line of cells, or uncoupled cells, on the tiles of
+ * mk_strand.
+ *
+ * A reverse step is linear in lam, and its matrix depends on the trajectory
+ * alone, which is complete when the reverse pass starts. Only the products
+ * with lam have to be taken in turn; the cell VJPs, which are nearly all of
+ * the work (2,000 instructions in double precision, 9 us per step one after
+ * the other), need not be. mk_adj_jac evaluates the Jacobian's entries of
+ * every cell and step of a range of steps at once, one VJP per state (1,000
+ * cells x 200 steps fill the device); mk_adj_lin then walks the steps with
+ * one lane per cell: about 30 multiply-adds, the entries loaded four steps
+ * ahead. LR1991, 1,000 cells in double precision: 9.2 us per reverse step on
+ * mk_adj_step, 1.3 here (entries and walk).
+ *
+ * Entry e of cell c at step s: jac[((s - base) * MK_NE + e) * npad + c].
+ * Rows of the Jacobian first (state i' by state j, existing entries only),
+ * then its derivatives by the fields, by the diffusion current, and last
+ * the loss term dL/dV(y_{s+1}) and dI/dgx at y_s.
+ * ---------------------------------------------------------------------- */
+typedef MkLinT<Real> MkLin;
+
+/* read by the host library when it loads the module */
+extern "C" __device__ const int mk_entries = MK_NE;
+
+__device__ __forceinline__ constexpr int mk_bits(unsigned long long m)
+{
+    int n = 0;
+    for (; m; m &= m - 1) ++n;
+    return n;
+}
+
+/* Steps s0 + blockIdx.x / tiles, cells of tile blockIdx.x % tiles. j.yn is
+ * y_{s0} of the trajectory. */
+extern "C" __global__ void __launch_bounds__(256)
+mk_adj_jac(const MkArgs a, const MkAdj j, const MkLin ln, const int s0,
+           const int tiles)
+{
+    const int k = blockIdx.x / tiles;
+    const int c = (blockIdx.x - k * tiles) * 256 + threadIdx.x;
+    if (c >= (int)a.n) return;
+    const long long np = a.npad, SN = (long long)MK_NS * np;
+    const Real* __restrict__ ys = j.yn + k * SN;
+    const Real* __restrict__ V = ys + MK_IVM * np;
+    const MkStep p = a.steps[s0 + k];
+    Real* __restrict__ o = ln.jac + (long long)(s0 + k - ln.base) * MK_NE * np
+                           + c;
+    Real y[MK_NS], fv[MK_NFA], lam[MK_NS], mu[MK_NS], fb[MK_NFA], abo;
+#pragma unroll
+    for (int i = 0; i < MK_NS; ++i) y[i] = ys[i * np + c];
+#pragma unroll
+    for (int f = 0; f < MK_NF; ++f) fv[f] = a.fields[f * np + c];
+    Real idiff = (Real)0, xs = (Real)0;
+#if MK_COUPLING == 1
+    idiff = mk_stencil(V, c, c, 0, (int)a.n, 1, a.gx, a.gy);
+    if (c > 0) xs += V[c] - V[c - 1];
+    if (c < (int)a.n - 1) xs += V[c] - V[c + 1];
+#elif MK_COUPLING == 2
+    idiff = mk_hetero(V, a.gx_field, a.gy_field, c, c, 0, (int)a.n, 1);
+#endif
+    const int nx = (int)a.nx;
+    const Real pace = mk_is_paced(a, c, c % nx, c / nx) ? p.pace : (Real)0;
+    Real loss = (Real)0;
+    const int q = j.probe_of[c];
+    if (q >= 0)
+        loss = (Real)(2.0 * ((double)V[SN + c]
+                             - j.target[(long long)(s0 + k) * j.n_probe + q]));
+    o[(long long)(MK_NE - 2) * np] = loss;
+    o[(long long)(MK_NE - 1) * np] = xs;
+#pragma unroll 1
+    for (int i = 0; i < MK_NS; ++i) {
+#pragma unroll
+        for (int r = 0; r < MK_NS; ++r) lam[r] = r == i ? (Real)1 : (Real)0;
+        mk_cell_vjp(y, p.t, p.dt, pace, idiff, fv, lam, mu, &abo, fb);
+        const unsigned long long jm = mk_jmask[i], fm = mk_fmask[i];
+        int e = mk_jrow[i];
+#pragma unroll
+        for (int r = 0; r < MK_NS; ++r)
+            if (jm >> r & 1) o[(long long)e++ * np] = mu[r];
+        e = mk_frow[i];
+#pragma unroll
+        for (int f = 0; f < MK_NF; ++f)
+            if (fm >> f & 1) o[(long long)e++ * np] = fb[f];
+        if (mk_dmask >> i & 1)
+            o[(long long)(MK_D0
+                          + __builtin_popcountll(
+                                mk_dmask & ((1ull << i) - 1))) * np] = abo;
+    }
+}
+
+/* Value i (states, then abar) of the kth of the outer cells of a tile's side
+ * e, slot of exchange parity par (as mk_sedge). */
+__device__ __forceinline__ MkXWord* mk_ledge(const MkLin& ln, int par,
+                                             int tile, int e, int i, int k)
+{
+    return ln.edges + ((((long long)(par * ln.tiles + tile) * 2 + e)
+                        * (MK_NS + 1) + i) * 32 + k) * MK_XW;
+}
+
+/* Reverse steps s1 - 1 .. s0 from mu, abar of step s1 (j.mu_in, j.ab_in) to
+ * those of step s0 (j.mu_out, j.ab_out: other buffers, a neighbour may still
+ * be reading its launch-start halo). */
+extern "C" __global__ void __launch_bounds__(64)
+mk_adj_lin(const MkArgs a, const MkAdj j, const MkLin ln, const int s0,
+           const int s1)
+{
+    constexpr int AHEAD = MK_NE <= 32 ? 4 : 2;
+    const int lane = threadIdx.x, tile = blockIdx.x;
+    const long long n = a.n, np = a.npad;
+    const long long c0 = (long long)tile * ln.width;
+    const int len = (int)(n - c0 < ln.width ? n - c0 : ln.width);
+    const long long cl = c0 + lane - ln.halo;
+    const long long c = cl < 0 ? 0 : cl >= n ? n - 1 : cl;
+    const bool own = lane >= ln.halo && lane < ln.halo + len;
+    Real mu[MK_NS], ab = (Real)0;
+#pragma unroll
+    for (int i = 0; i < MK_NS; ++i)
+        mu[i] = ln.fresh ? (Real)0 : j.mu_in[i * np + c];
+    if (!ln.fresh) ab = j.ab_in[c];
+#if MK_COUPLING == 2
+    const Real gl = c > 0 ? a.gx_field[c - 1] : (Real)0;
+    const Real gr = c < n - 1 ? a.gx_field[c] : (Real)0;
+#endif
+    double gf[MK_NFA], cx = 0.0, loss = 0.0;
+#pragma unroll
+    for (int f = 0; f < MK_NFA; ++f) gf[f] = 0.0;
+    const Real* __restrict__ jc = ln.jac + c;
+    Real E[AHEAD][MK_NE];
+#pragma unroll
+    for (int b = 0; b < AHEAD; ++b) {
+        const int s = s1 - 1 - b < s0 ? s0 : s1 - 1 - b;
+#pragma unroll
+        for (int e = 0; e < MK_NE; ++e)
+            E[b][e] = jc[((long long)(s - ln.base) * MK_NE + e) * np];
+    }
+    int left = ln.halo, sup = 0;
+    for (int sb = s1 - 1; sb >= s0; sb -= AHEAD) {
+#pragma unroll
+        for (int b = 0; b < AHEAD; ++b) {
+            const int s = sb - b;
+            if (s < s0) break;
+            Real lam[MK_NS];
+#pragma unroll
+            for (int i = 0; i < MK_NS; ++i) lam[i] = mu[i];
+            Real lv = E[b][MK_NE - 2];
+            loss += 0.25 * (double)lv * (double)lv;
+#if MK_COUPLING == 1 || MK_COUPLING == 2
+            {
+                const Real al = __shfl_up(ab, 1, 64);
+                const Real ar = __shfl_down(ab, 1, 64);
+#if MK_COUPLING == 1
+                Real ax = (Real)0;
+                if (c > 0) ax += ab - al;
+                if (c < n - 1) ax += ab - ar;
+                lv += a.gx * ax;
+#else
+                if (c > 0) lv += gl * (ab - al);
+                if (c < n - 1) lv += gr * (ab - ar);
+#endif
+            }
+#endif
+            lam[MK_IVM] += lv;
+            /* products with an adjoint of 0 are 0, also where an entry is
+             * not finite (mk_gmul) */
+            bool nz[MK_NS];
+#pragma unroll
+            for (int i = 0; i < MK_NS; ++i) nz[i] = lam[i] != (Real)0;
+#pragma unroll
+            for (int r = 0; r < MK_NS; ++r) {
+                Real m = (Real)0;
+#pragma unroll
+                for (int i = 0; i < MK_NS; ++i) {
+                    if (!(mk_jmask[i] >> r & 1)) continue;
+                    const int e = mk_jrow[i]
+                                  + mk_bits(mk_jmask[i] & ((1ull << r) - 1));
+                    m = __builtin_fma(lam[i], nz[i] ? E[b][e] : (Real)0, m);
+                }
+                mu[r] = m;
+            }
+            Real abn = (Real)0;
+#pragma unroll
+            for (int i = 0; i < MK_NS; ++i) {
+                if (!(mk_dmask >> i & 1)) continue;
+                const int e = MK_D0 + mk_bits(mk_dmask & ((1ull << i) - 1));
+                abn = __builtin_fma(lam[i], nz[i] ? E[b][e] : (Real)0, abn);
+            }
+            ab = abn;
+#pragma unroll
+            for (int f = 0; f < MK_NF; ++f) {
+#pragma unroll
+                for (int i = 0; i < MK_NS; ++i) {
+                    if (!(mk_fmask[i] >> f & 1)) continue;
+                    const int e = mk_frow[i]
+                                  + mk_bits(mk_fmask[i] & ((1ull << f) - 1));
+                    gf[f] = __builtin_fma(lam[i],
+                                          nz[i] ? E[b][e] : (Real)0, gf[f]);
+                }
+            }
+            cx = __builtin_fma((double)ab, (double)E[b][MK_NE - 1], cx);
+            /* the entries of the step AHEAD steps on */
+            {
+                const int sn = s - AHEAD < s0 ? s0 : s - AHEAD;
+#pragma unroll
+                for (int e = 0; e < MK_NE; ++e)
+                    E[b][e] = jc[((long long)(sn - ln.base) * MK_NE + e) * np];
+            }
+#if MK_COUPLING != 0
+            if (--left == 0 && ln.tiles > 1 && s > s0) {
+                /* the exchange of mk_strand, for mu and abar */
+                left = ln.halo;
+                const int step = ln.g0 + ++sup, par = step & 1;
+                const bool el = own && lane < 2 * ln.halo && tile > 0;
+                const bool er = own && lane >= len && tile + 1 < ln.tiles;
+#pragma unroll
+                for (int i = 0; i <= MK_NS; ++i) {
+                    const Real v = i < MK_NS ? mu[i < MK_NS ? i : 0] : ab;
+                    if (el)
+                        mk_tput(mk_ledge(ln, par, tile, 0, i, lane - ln.halo),
+                                v, step);
+                    if (er)
+                        mk_tput(mk_ledge(ln, par, tile, 1, i, lane - len), v,
+                                step);
+                }
+                const bool hl = lane < ln.halo && tile > 0;
+                const bool hr = lane >= ln.halo + len
+                                && tile + 1 < ln.tiles && cl < n;
+                bool bad = false;
+                if (hl || hr) {
+                    MkXWord* e = hl ? mk_ledge(ln, par, tile - 1, 1, 0, lane)
+                                    : mk_ledge(ln, par, tile + 1, 0, 0,
+                                               lane - ln.halo - len);
+                    for (int spins = 0;; ++spins) {
+                        MkXWord w[(MK_NS + 1) * MK_XW];
+                        bool ready = true;
+#pragma unroll
+                        for (int i = 0; i < (MK_NS + 1) * MK_XW; ++i)
+                            w[i] = __hip_atomic_load(
+                                e + i / MK_XW * 32 * MK_XW + i % MK_XW,
+                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                        for (int i = 0; i < (MK_NS + 1) * MK_XW; ++i)
+                            ready = ready && (int)(w[i] >> 32) >= step;
+                        if (ready) {
+#pragma unroll
+                            for (int i = 0; i <= MK_NS; ++i) {
+                                const Real v = (Real)__longlong_as_double(
+                                    (long long)(((w[i * MK_XW] & 0xffffffffull)
+                                                 << 32)
+                                                | (w[i * MK_XW + MK_XW - 1]
+                                                   & 0xffffffffull)));
+                                if (i < MK_NS) mu[i < MK_NS ? i : 0] = v;
+                                else ab = v;
+                            }
+                            break;
+                        }
+                        if (spins >= ln.spin_limit) {
+                            __hip_atomic_store(ln.err, 1, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                            bad = true;
+                            break;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                }
+                if (__any(bad)) return;
+            }
+#endif
+        }
+    }
+    if (own) {
+#pragma unroll
+        for (int i = 0; i < MK_NS; ++i) j.mu_out[i * np + c] = mu[i];
+        j.ab_out[c] = ab;
+#pragma unroll
+        for (int f = 0; f < MK_NF; ++f) j.gfield[f * np + c] += gf[f];
+        const int q = j.probe_of[c];
+        if (q >= 0) j.loss_acc[q] += loss;
+    } else {
+        cx = 0.0;
+    }
+#if MK_COUPLING == 1
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) cx += __shfl_down(cx, o, 64);
+    if (lane == 0) j.gx_acc[tile] += cx;
+#else
+    (void)cx; (void)sup; (void)left;
+#endif
+}
+#endif

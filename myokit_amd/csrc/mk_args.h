@@ -135,4 +135,20 @@ struct MkStrandT {
     R* traj;                  /* as MkSheetT */
 };
 
+/* Linear reverse pass of a line of cells or of uncoupled cells (the tiles of
+ * the strand driver). */
+template <typename R>
+struct MkLinT {
+    R* jac;                   /* [steps][entries][npad] of steps base.. */
+    unsigned long long* edges;  /* [2][tiles][2][states + 1][32]
+                                   [sizeof(R) / 4] mu and abar of each tile's
+                                   outer cells, tagged by exchange */
+    int* err;                 /* set to 1 if a neighbour wait timed out */
+    int base;                 /* first step whose entries jac holds */
+    int fresh;                /* the run's last step: mu and abar are 0 */
+    int tiles, width, halo;   /* as MkStrandT */
+    int g0;                   /* exchanges completed before this launch */
+    int spin_limit;           /* polls before a wait is abandoned */
+};
+
 #endif

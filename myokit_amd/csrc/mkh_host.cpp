@@ -73,7 +73,9 @@ struct Program {
     hipFunction_t f_chain = nullptr, f_strand = nullptr;
     hipFunction_t f_adj_step = nullptr, f_adj_block = nullptr,
                   f_adj_probe = nullptr, f_adj_sheet = nullptr,
-                  f_adj_gather = nullptr;
+                  f_adj_gather = nullptr, f_adj_jac = nullptr,
+                  f_adj_lin = nullptr;
+    int n_entries = 0;      /* of mk_adj_jac, per cell and step */
     /* mk_layout of the module: precision, states, fields, sheet / chain /
      * reverse-sheet cells per thread (have_layout false if absent) */
     int layout[6] = {0, 0, 0, 0, 0, 0};
@@ -1528,6 +1530,8 @@ struct Sim : SimBase {
             if (v) adj.release();
         } else if (k == "adj_sheet") {
             no_sheet_rev = v == 0;
+        } else if (k == "adj_linear") {
+            no_adj_linear = v == 0;
         } else if (k == "adj_overlap") {
             no_adj_overlap = v == 0;
         } else {
@@ -1573,6 +1577,11 @@ struct Sim : SimBase {
     /* "adj_overlap" option: 0 keeps the recomputation of earlier segments
      * in line with the reverse steps on small domains */
     bool no_adj_overlap = false;
+    /* "adj_linear" option: 0 keeps lines of cells on the kernels that apply
+     * the cell VJP step by step */
+    bool no_adj_linear = false;
+    /* most cells of the linear reverse pass */
+    static constexpr long long lin_cells = 8192;
     /* second stream (default priority) for overlapped recomputation */
     hipStream_t rc_stream = nullptr;
     hipEvent_t rc_ev[4] = {};
@@ -1582,6 +1591,9 @@ struct Sim : SimBase {
         DevBuf<R> ckpt, traj, traj2, work, work2, mu[2], ab[2];
         DevBuf<double> gfield, gx, gy, loss, target, trace;
         DevBuf<int> probe_of;
+        /* linear reverse pass: entries of a range of steps, tile edges */
+        DevBuf<R> jac;
+        DevBuf<unsigned long long> lin_edges;
         DevBuf<long long> probes;
         /* the probe list probe_of was built for */
         std::vector<long long> probe_key;
@@ -1604,6 +1616,8 @@ struct Sim : SimBase {
             target.release();
             trace.release();
             probe_of.release();
+            jac.release();
+            lin_edges.release();
             probes.release();
             probe_key.clear();
         }
@@ -1700,7 +1714,8 @@ struct Sim : SimBase {
                                   : 1,
                               driver == MKH_DRIVER_SHEET
                                   ? (size_t)adj_sheet_tiles()
-                                  : 1});
+                                  : 1,
+                              (size_t)st_tiles});
         DevBuf<Step>& dsteps = adj.steps;
         DevBuf<R>& ckpt = adj.ckpt;
         DevBuf<R>& traj = adj.traj;
@@ -1824,7 +1839,33 @@ struct Sim : SimBase {
                 for (auto& e : rc_ev) MKH_HIP(hipEventCreate(&e));
             }
         }
-        adj_rev_kind = sheet_rev ? MKH_ADJ_REV_SHEET
+        /* Lines of cells and uncoupled cells in double precision: the
+         * linear pass, while the entries of a step (one VJP per state and
+         * cell) take less time on the whole device than one VJP takes
+         * alone. */
+        const bool lin_rev = use_strand && prog->f_adj_lin &&
+                             n <= lin_cells && !no_adj_linear;
+        long long lin_steps = 0;        /* steps whose entries are held */
+        if (lin_rev) {
+            lin_steps = std::max<long long>(
+                16, std::min<long long>(
+                        256, (256LL << 20) /
+                                 (prog->n_entries * npad * (long long)
+                                  sizeof(R))));
+            lin_steps = std::min(lin_steps, Kl);
+            MKH_HIP(adj.jac.alloc((size_t)lin_steps * prog->n_entries *
+                                  npad));
+            if (st_halo > 0) {
+                MKH_HIP(adj.lin_edges.alloc((size_t)st_tiles * 4 *
+                                            (cfg.n_state + 1) * 32 * XW));
+                MKH_HIP(hipMemset(adj.lin_edges.p, 0,
+                                  adj.lin_edges.n *
+                                      sizeof(unsigned long long)));
+            }
+        }
+        long long lin_done = 0;
+        adj_rev_kind = lin_rev ? MKH_ADJ_REV_LINEAR
+                       : sheet_rev ? MKH_ADJ_REV_SHEET
                        : block_rev ? MKH_ADJ_REV_BLOCK
                        : overlap ? MKH_ADJ_REV_STEP_OVERLAP
                                  : MKH_ADJ_REV_STEP;
@@ -2044,6 +2085,55 @@ struct Sim : SimBase {
                 MKH_HIP(hipEventElapsedTime(&ms, ev[2], ev[3]));
                 recompute_ms += ms;
             }
+            if (lin_rev) {
+                /* the entries of a range of steps, then its products in
+                 * turn; mu and abar ping-pong between launches */
+                for (long long e1 = s1; e1 > s0;) {
+                    const long long e0 = std::max(s0, e1 - lin_steps);
+                    MkAdjT<R> js = j;
+                    js.yn = slot(e0 - s0);
+                    js.mu_in = mu_in;
+                    js.ab_in = ab_in;
+                    js.mu_out = mu_out;
+                    js.ab_out = ab_out;
+                    MkLinT<R> ln;
+                    std::memset(&ln, 0, sizeof(ln));
+                    ln.jac = adj.jac.p;
+                    ln.edges = adj.lin_edges.p;
+                    ln.err = st_err.p;
+                    ln.base = (int)e0;
+                    ln.fresh = mu_in == nullptr;
+                    ln.tiles = st_tiles;
+                    ln.width = st_width;
+                    ln.halo = st_halo;
+                    ln.g0 = (int)lin_done;
+                    ln.spin_limit = 1 << 20;
+                    int i0 = (int)e0, i1 = (int)e1;
+                    int tiles = (int)((n + 255) / 256);
+                    void* pj[] = {&a, &js, &ln, &i0, &tiles};
+                    MKH_HIP(hipModuleLaunchKernel(
+                        prog->f_adj_jac, (unsigned)(tiles * (e1 - e0)), 1, 1,
+                        256, 1, 1, 0, stream, pj, nullptr));
+                    void* pl_[] = {&a, &js, &ln, &i0, &i1};
+                    if (st_halo > 0) {
+                        MKH_HIP(hipModuleLaunchCooperativeKernel(
+                            prog->f_adj_lin, (unsigned)st_tiles, 1, 1, 64, 1,
+                            1, 0, stream, pl_));
+                        lin_done += (e1 - e0 - 1) / st_halo;
+                    } else {
+                        MKH_HIP(hipModuleLaunchKernel(
+                            prog->f_adj_lin, (unsigned)st_tiles, 1, 1, 64, 1,
+                            1, 0, stream, pl_, nullptr));
+                    }
+                    adj_rev_launches += 2;
+                    mu_in = mu_out;
+                    ab_in = ab_out;
+                    mu_out = (mu_out == muA.p) ? muB.p : muA.p;
+                    ab_out = (ab_out == abA.p) ? abB.p : abA.p;
+                    e1 = e0;
+                }
+                continue;
+            }
             if (sheet_rev) {
                 /* every reverse step of the segment in one cooperative
                  * launch; mu in LDS, carried in muA and abar in abA */
@@ -2094,7 +2184,7 @@ struct Sim : SimBase {
         }
         /* closing pass: conductance terms of step 0 (y_0 is slot 0); a
          * graph's are taken in the step itself */
-        if (!block_rev && !sheet_rev &&
+        if (!block_rev && !sheet_rev && !lin_rev &&
             cfg.coupling != MKH_COUPLING_GRAPH) {
             int e = reverse_step(nullptr, slot(0), 0, -1);
             if (e) return e;
@@ -2682,6 +2772,21 @@ int mkh_program_build(const char* source, const char* options,
                                  "mk_adj_sheet") != hipSuccess) {
             prog->f_adj_sheet = nullptr;
             (void)hipGetLastError();
+        }
+        /* the linear reverse pass: double precision, small models */
+        if (!prog->f_adj_step ||
+            hipModuleGetFunction(&prog->f_adj_jac, prog->module,
+                                 "mk_adj_jac") != hipSuccess ||
+            hipModuleGetFunction(&prog->f_adj_lin, prog->module,
+                                 "mk_adj_lin") != hipSuccess) {
+            prog->f_adj_jac = prog->f_adj_lin = nullptr;
+            (void)hipGetLastError();
+        } else {
+            hipDeviceptr_t ep = nullptr;
+            size_t esz = 0;
+            MKH_HIP(hipModuleGetGlobal(&ep, &esz, prog->module,
+                                       "mk_entries"));
+            MKH_HIP(hipMemcpyDtoH(&prog->n_entries, ep, sizeof(int)));
         }
         MKH_HIP(prog->query());
         hipDeviceptr_t lp = nullptr;
