@@ -12,6 +12,7 @@ appends at large cell counts.
 ``prepare_log`` follows ``myokit.prepare_log`` (``_datalog.py:1783-2193``):
 flags, lists of names, and existing logs, with the same checks.
 """
+import functools
 import os as _os
 import re
 from collections import OrderedDict
@@ -58,6 +59,12 @@ def dimco(*dims):
     grids = np.indices(tuple(reversed(dims))).reshape(len(dims), -1)
     for idx in grids.T:
         yield tuple(int(i) for i in reversed(idx))
+
+
+@functools.lru_cache(maxsize=4)
+def _cell_prefixes(dims):
+    """The key prefixes of every cell of a grid, 'x.' or 'x.y.'."""
+    return tuple('.'.join(str(i) for i in x) + '.' for x in dimco(*dims))
 
 
 def float_str(number, precision=DOUBLE_PRECISION):
@@ -244,18 +251,11 @@ def prepare_log(log, model, dims=None, global_vars=None,
     names, or an existing log (checked for compatibility)."""
     dtype = np.float64 if precision == DOUBLE_PRECISION else np.float32
     dims = tuple(dims) if dims else ()
-    _combos = []
 
     def dcombos():
         # Cell prefixes ('x.' or 'x.y.', first index fastest), built only
         # when a name is expanded over every cell
-        if not _combos:
-            if dims:
-                _combos.extend(
-                    '.'.join(str(i) for i in x) + '.' for x in dimco(*dims))
-            else:
-                _combos.append('')
-        return _combos
+        return _cell_prefixes(dims) if dims else ('',)
 
     def valid_index(kdims):
         # 'x.' or 'x.y.' with every index in range
@@ -294,8 +294,12 @@ def prepare_log(log, model, dims=None, global_vars=None,
             raise ValueError('This log does not support intermediary'
                              f' variables, got <{var}>.')
 
+    # an empty column: one array stands for all of them, since columns are
+    # replaced, never filled in place
+    empty = np.zeros(0, dtype=dtype)
+
     def new():
-        return np.zeros(0, dtype=dtype)
+        return empty
 
     if log is None:
         if if_empty & allowed_classes == if_empty:

@@ -388,12 +388,16 @@ class FiberTissueSimulation:
                 raise
             dtype = np.float64 if self._precision == DOUBLE_PRECISION \
                 else np.float32
+            nan = []
             for (sim, log, q, colmap, cols, g, ls), run in zip(parts, runs):
                 values, times, paces = sim._exec_end(run, ok)
                 sim._fill_log(log, values, times, paces, cols, g, dtype)
+                nan.append(np.isnan(values[-1]).any()
+                           if cols and len(times) else log.has_nan())
+        else:
+            nan = [logf.has_nan(), logt.has_nan()]
 
-        if report_nan and (arithmetic_error or logf.has_nan()
-                           or logt.has_nan()):
+        if report_nan and (arithmetic_error or any(nan)):
             self._report_nan(logf, logt)
         return logf, logt
 

@@ -290,6 +290,8 @@ class SimulationOpenCL:
         self._sources = {}
         # number of quantities -> column map of run_block (every cell)
         self._block_colmaps = {}
+        # the keys of the last log and their layout (_log_layout)
+        self._layout = None
         # device cell order of a set_connections graph (_cell_order) and
         # column maps permuted to it
         self._order_cache = None
@@ -1174,6 +1176,11 @@ class SimulationOpenCL:
             gnames[gtime.qname()] = 'time'
         if gpace is not None:
             gnames[gpace.qname()] = 'pace'
+        keys = tuple(log.keys())
+        hit = self._layout
+        if hit is not None and hit[0] == keys:
+            # the layout of a repeated run
+            return hit[1]
         quantities = []
         qindex = {}
         cols = []          # (key, q, cell)
@@ -1197,7 +1204,10 @@ class SimulationOpenCL:
         for col, (key, q, cell) in enumerate(cols):
             colmap[q, cell] = col
         logging_states = any(q.is_state() for q in quantities)
-        return quantities, colmap, cols, globals_, logging_states
+        colmap.setflags(write=False)
+        r = quantities, colmap, cols, globals_, logging_states
+        self._layout = (keys, r)
+        return r
 
     def _run(self, duration, log, log_interval, report_nan, progress, msg):
         if duration < 0:
@@ -1225,6 +1235,7 @@ class SimulationOpenCL:
                     ' myokit.ProgressReporter or None.')
 
         arithmetic_error = False
+        nan = None
         if duration > 0:
             quantities, colmap, cols, globals_, logging_states = \
                 self._log_layout(log)
@@ -1233,8 +1244,12 @@ class SimulationOpenCL:
                 log_interval, progress, msg)
             dtype = values.dtype
             self._fill_log(log, values, times, paces, cols, globals_, dtype)
-
-        if report_nan and (arithmetic_error or log.has_nan()):
+            if cols and len(times):
+                nan = np.isnan(values[-1]).any()
+        # as DataLog.has_nan: a NaN in the final row, which is this run's
+        # last one, if it has logged any
+        if report_nan and (arithmetic_error or (
+                log.has_nan() if nan is None else nan)):
             self._report_nan(log)
         return log
 

@@ -374,3 +374,21 @@ def test_library_releases_handles_at_exit():
                            __import__('os').path.dirname(__file__)))
     assert r.returncode == 0, r.stderr
     assert r.stdout.strip() == 'closed'
+
+
+def test_layout_of_a_repeated_log(model):
+    # the layout is that of the keys in their order, not of the log object
+    s = myokit.SimulationOpenCL(model, ncells=3)
+    logs = [['membrane.V'], ['0.membrane.V', '2.ica.ICa'],
+            ['2.ica.ICa', '0.membrane.V'], ['membrane.V']]
+    out = []
+    for names in logs:
+        log = myokit.prepare_log(names, s._model, dims=s._dims)
+        a = s._layout and s._layout[1]
+        b = s._log_layout(log)
+        assert b is s._log_layout(myokit.prepare_log(
+            names, s._model, dims=s._dims)) and b is not a
+        out.append(([q.qname() for q in b[0]], b[1].tolist()))
+    assert out[0] == out[3]
+    assert out[1] == (['membrane.V', 'ica.ICa'], [[0, -1, -1], [-1, -1, 1]])
+    assert out[2] == (['ica.ICa', 'membrane.V'], [[-1, -1, 0], [1, -1, -1]])
