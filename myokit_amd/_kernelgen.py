@@ -1289,6 +1289,11 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         '#define MK_CWAVES ' + str(cwaves),
         '#define MK_ACPT ' + str(acpt),
         '#define MK_GBLOCKS ' + str(gblocks),
+        # two steps per launch of the grid driver: single precision sheets of
+        # models whose state fits the registers six times
+        '#define MK_GRID2 ' + str(int(
+            precision == SINGLE_PRECISION and int(coupling) in (1, 2)
+            and len(cm.states) <= 12)),
         '#define MK_ADJ_SHEET ' + ('1' if adjoint and int(coupling) == 1
                                    and asg > 0 and persistent
                                    and adjoint_precision in (None, precision)

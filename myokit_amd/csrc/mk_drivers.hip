@@ -392,6 +392,121 @@ mk_grid(const MkArgs a, const Real* __restrict__ src, Real* __restrict__ dst,
     for (int i = 0; i < MK_NS; ++i) dst[(long long)i * a.npad + c] = y[i];
 }
 
+#if MK_GRID2
+/* ------------------------------------------------------------------------
+ * Two steps of a 2D sheet per launch (single precision): for sheets whose
+ * tiles cannot all be resident, where mk_grid is bound by reading and
+ * writing the whole state every step.
+ *
+ * A workgroup loads a tile of 64 x MK_G2H cells (MK_G2H = 4 * MK_G2C, thread
+ * (lx, w) the cells of rows w * MK_G2C + k), takes both steps of the rows
+ * they need, V in LDS between them, and stores the 60 x (MK_G2H - 4) inner
+ * cells; the outer two are recomputed by the neighbours' workgroups. With 4
+ * cells per thread a cell-step costs 1.16 of mk_grid's arithmetic and 39 B
+ * of its 64 B of state. LR1991, Rush-Larsen, us per step, mk_grid -> here:
+ * 2049 x 1501 43.7 -> 38.8 (with a conductance field 53.9 -> 43.3), 1100 x
+ * 1100 22.5 -> 19.1, 3000 x 200 13.8 -> 13.2; 6 and 8 cells per thread 39.4
+ * and 40.8 on the first. Both steps are unrolled: a loop over them spills
+ * (95 registers, 73 us).
+ *
+ * Only the second step may log (the host takes a step that logs first with
+ * mk_grid); the NaN test is the second step's.
+ * ---------------------------------------------------------------------- */
+#define MK_G2C 4
+#define MK_G2H (4 * MK_G2C)
+extern "C" __global__ void __launch_bounds__(256, 4)
+mk_grid2(const MkArgs a, const Real* __restrict__ src, Real* __restrict__ dst,
+         const int s)
+{
+    __shared__ Real vt[2][MK_G2H][66];
+    const MkStep p0 = a.steps[s], p1 = a.steps[s + 1];
+    if (mk_halted(a, p1.row)) return;
+    const int nx = (int)a.nx, ny = (int)a.ny;
+    const unsigned tiles_x = (unsigned)(nx + 59) / 60;
+    const unsigned b = (unsigned)mk_xcd_block(blockIdx.x, gridDim.x);
+    const unsigned ty = b / tiles_x, tx = b - ty * tiles_x;
+    const int lx = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int ix = (int)tx * 60 - 2 + lx;
+    const int gy0 = (int)ty * (MK_G2H - 4) - 2;
+    /* lanes and rows beyond the sheet hold a copy of its border cell, which
+     * no cell of the sheet reads */
+    const int xc = ix < 0 ? 0 : ix >= nx ? nx - 1 : ix;
+    const bool xin = lx >= 2 && lx < 62 && ix < nx;
+    Real y[MK_G2C][MK_NS];
+#pragma unroll
+    for (int k = 0; k < MK_G2C; ++k) {
+        const int r = w * MK_G2C + k, iy = gy0 + r;
+        const int yc = iy < 0 ? 0 : iy >= ny ? ny - 1 : iy;
+        const long long c = xc + (long long)yc * nx;
+#pragma unroll
+        for (int i = 0; i < MK_NS; ++i) y[k][i] = src[(long long)i * a.npad + c];
+        vt[0][r][lx + 1] = y[k][MK_IVM];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const Real (*v0)[66] = vt[h];
+#pragma unroll
+        for (int k = 0; k < MK_G2C; ++k) {
+            const int r = w * MK_G2C + k, iy = gy0 + r;
+            /* rows the second step's inner cells need, and the sheet's */
+            if (r >= 1 + h && r < MK_G2H - 1 - h && iy >= 0 && iy < ny) {
+                const long long c = xc + (long long)iy * nx;
+                const Real v = v0[r][lx + 1];
+                Real id;
+#if MK_COUPLING == 2
+                /* the sums of mk_hetero */
+                id = (Real)0;
+                if (nx > 1) {
+                    if (xc > 0)
+                        id += a.gx_field[c - iy - 1] * (v - v0[r][lx]);
+                    if (xc < nx - 1)
+                        id += a.gx_field[c - iy] * (v - v0[r][lx + 2]);
+                }
+                if (iy > 0) id += a.gy_field[c - nx] * (v - v0[r - 1][lx + 1]);
+                if (iy < ny - 1) id += a.gy_field[c] * (v - v0[r + 1][lx + 1]);
+#else
+                if (nx > 1) {
+                    if (xc == 0) id = a.gx * (v - v0[r][lx + 2]);
+                    else if (xc == nx - 1) id = a.gx * (v - v0[r][lx]);
+                    else id = a.gx * (((Real)2 * v - v0[r][lx])
+                                      - v0[r][lx + 2]);
+                } else {
+                    id = (Real)0;
+                }
+                if (iy == 0) id += a.gy * (v - v0[r + 1][lx + 1]);
+                else if (iy == ny - 1) id += a.gy * (v - v0[r - 1][lx + 1]);
+                else id += a.gy * (((Real)2 * v - v0[r - 1][lx + 1])
+                                   - v0[r + 1][lx + 1]);
+#endif
+                const Real pc = h == 0 ? p0.pace : p1.pace;
+                const Real pace = mk_is_paced<long long>(a, c, xc, iy)
+                                      ? pc : (Real)0;
+                Real fv[MK_NFA], q[MK_NQA];
+#pragma unroll
+                for (int f = 0; f < MK_NF; ++f)
+                    fv[f] = a.fields[(long long)f * a.npad + c];
+                if (h == 1 && p1.row >= 0 && xin && a.nan_check
+                    && c == a.nan_cell && y[k][0] != y[k][0])
+                    __atomic_store_n(a.halt, p1.row, __ATOMIC_RELAXED);
+                mk_cell<true>(y[k], h == 0 ? p0.t : p1.t,
+                              h == 0 ? p0.dt : p1.dt, pace, id, fv, q);
+                if (h == 0) {
+                    vt[1][r][lx + 1] = y[k][MK_IVM];
+                } else if (xin) {
+                    if (p1.row >= 0) mk_write_log(a, c, p1.row, q);
+#pragma unroll
+                    for (int i = 0; i < MK_NS; ++i)
+                        dst[(long long)i * a.npad + c] = y[k][i];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (h == 0) __syncthreads();
+    }
+}
+#endif
+
 /* ------------------------------------------------------------------------
  * Persistent 2D sheet: register-resident state, LDS halos, neighbour sync.
  *

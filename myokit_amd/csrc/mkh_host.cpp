@@ -68,7 +68,8 @@ int fail(int code, const std::string& msg)
 struct Program {
     int device = -1;
     hipModule_t module = nullptr;
-    hipFunction_t f_cells = nullptr, f_block = nullptr, f_grid = nullptr;
+    hipFunction_t f_cells = nullptr, f_block = nullptr, f_grid = nullptr,
+                  f_grid2 = nullptr;
     hipFunction_t f_sheet = nullptr, f_junction = nullptr;
     hipFunction_t f_chain = nullptr, f_strand = nullptr;
     hipFunction_t f_adj_step = nullptr, f_adj_block = nullptr,
@@ -1282,6 +1283,33 @@ struct Sim : SimBase {
         return emit_row(b, s);
     }
 
+    /* Sheets of at least this many cells take two steps per launch: on
+     * small ones a workgroup's cells, one after the other, take longer than
+     * a second launch (us per step, mk_grid and mk_grid2: 301 x 217 6.8 and
+     * 8.4, 3000 x 200 13.8 and 13.2, 1100 x 1100 22.5 and 19.1). */
+    static constexpr long long two_cells = 600000;
+
+    /* Steps s and s + 1 of the batch in one launch (mk_grid2). */
+    int grid2_launch(Batch& b, long long s)
+    {
+        Args a = base_args();
+        R* src = state[cur].p;
+        R* dst = state[cur ^ 1].p;
+        int si = (int)s;
+        void* params[] = {&a, &src, &dst, &si};
+        const long long tiles = (cfg.nx + 59) / 60 * ((cfg.ny + 11) / 12);
+        if (time_kernels) MKH_HIP(hipEventRecord(event(b.nev), stream));
+        MKH_HIP(hipModuleLaunchKernel(prog->f_grid2, (unsigned)tiles, 1, 1,
+                                      256, 1, 1, 0, stream, params, nullptr));
+        if (time_kernels) {
+            MKH_HIP(hipEventRecord(event(b.nev + 1), stream));
+            b.nev += 2;
+        }
+        launches++;
+        cur ^= 1;
+        return emit_row(b, s + 1);
+    }
+
     /* Waits for the batch; copies times and paces of its rows. Returns the
      * number of valid rows (all, or up to the one where the NaN check
      * halted the run) through `valid`. */
@@ -1362,8 +1390,13 @@ struct Sim : SimBase {
         const bool strand = driver == MKH_DRIVER_STRAND ||
                             (driver == MKH_DRIVER_CELLS && strand_for(driver));
         if (driver == MKH_DRIVER_GRID) {
+            const bool two = prog->f_grid2 && cfg.ny > 1 && n >= two_cells;
             for (long long s = 0; s < ns; ++s) {
-                e = grid_launch(b, s, nullptr);
+                if (two && s + 1 < ns && h_steps[s].row < 0) {
+                    e = grid2_launch(b, s++);
+                } else {
+                    e = grid_launch(b, s, nullptr);
+                }
                 if (e) return e;
             }
         } else if (driver == MKH_DRIVER_SHEET) {
@@ -2747,6 +2780,12 @@ int mkh_program_build(const char* source, const char* options,
         MKH_HIP(hipModuleGetFunction(&prog->f_chain, prog->module, "mk_chain"));
         MKH_HIP(hipModuleGetFunction(&prog->f_junction, prog->module,
                                      "mk_junction"));
+        /* two steps of a sheet per launch: small models, single precision */
+        if (hipModuleGetFunction(&prog->f_grid2, prog->module, "mk_grid2") !=
+            hipSuccess) {
+            prog->f_grid2 = nullptr;
+            (void)hipGetLastError();
+        }
         /* lines of cells and uncoupled cells, of models it can split */
         if (hipModuleGetFunction(&prog->f_strand, prog->module,
                                  "mk_strand") != hipSuccess) {

@@ -80,3 +80,20 @@ def test_reverse_sheet_edges_equal_one_step_kernel(shape, cpt):
     np.testing.assert_array_equal(res[0][1], res[1][1])
     assert res[0][2] == pytest.approx(res[1][2], rel=1e-12)
     assert res[0][3] == pytest.approx(res[1][3], rel=1e-12)
+
+
+@pytest.mark.parametrize('field', [False, True])
+@pytest.mark.parametrize('shape', [(1009, 601), (601, 1021)])
+def test_fp32_two_steps_per_launch_equal_one(shape, field):
+    # large sheets on the grid driver: a run that logs every step takes
+    # single steps, one that logs every 5 or never takes pairs and odd ones
+    out = []
+    for every in (1, 5, 1000):
+        s = _scenario(shape, field).product(32)
+        s.set_tuning(driver='grid')
+        b = s.run_block(0.21, ['membrane.V'], log_interval=every * 0.01)
+        assert s.engine_driver() == 'grid'
+        out.append((b['membrane.V'][::5 // min(every, 5)], np.array(s.state())))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    np.testing.assert_array_equal(out[0][1], out[2][1])
