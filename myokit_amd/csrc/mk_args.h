@@ -32,8 +32,8 @@ struct MkArgsT {
     const R* csr_g;             /* graph: conductance per entry */
     const R* gx_field;          /* hetero: (ny, nx - 1) */
     const R* gy_field;          /* hetero: (ny - 1, nx) */
-    const R* idiff_extra;       /* grid driver: current added to idiff where
-                                   nonzero (fiber-tissue junction), or NULL */
+    const R* jv;                /* grid driver: potentials of the other part of
+                                   a fiber-tissue junction, or NULL */
     const long long* dom_off;   /* block driver: domain offsets into dom_cells */
     const int* dom_cells;       /* block driver: cell ids, grouped by domain
                                    (NULL = identity order) */
@@ -55,6 +55,11 @@ struct MkArgsT {
                                    positions (q -> q * gcopies + c %
                                    gcopies); 1: a row per cell */
     R gx, gy;                   /* homogeneous conductances */
+    /* fiber-tissue junction: cell (jx, jy + k) of this part, k < jn, meets
+     * cell jo + k * js of the other */
+    long long jx, jy, jn, jo, js;
+    R jg;                       /* its conductance */
+    int jtissue;                /* this part is the tissue */
 };
 
 /* Discrete adjoint of one step (see mk_adjoint.hip). */

@@ -374,13 +374,24 @@ mk_grid(const MkArgs a, const Real* __restrict__ src, Real* __restrict__ dst,
 #else
     Real idiff = (Real)0;
 #endif
-    /* junction current of the fiber-tissue driver, added after the stencil
-     * as the reference adds it (diff_step_fiber_tissue, openclsim.cl:601-
-     * 628); zero elsewhere, where adding nothing keeps idiff bit for bit */
-    if (a.idiff_extra) {
-        const Real e = a.idiff_extra[c];
+#if MK_COUPLING == 1
+    /* junction of the fiber-tissue driver (diff_step_fiber_tissue,
+     * openclsim.cl:601-628): g (Vf - Vt) for the fiber's cell, its negative
+     * for the tissue's, from the potentials at t of both parts; added after
+     * the stencil as the reference adds it, and only where nonzero */
+    if (a.jv && ix == a.jx && iy >= a.jy && iy < a.jy + a.jn) {
+        const Real o = a.jv[a.jo + (iy - a.jy) * a.js];
+        const Real v = y[MK_IVM];
+        Real e;
+        if (a.jtissue) {
+            const Real i = a.jg * (o - v);
+            e = -i;
+        } else {
+            e = a.jg * (v - o);
+        }
         if (e != (Real)0) idiff += e;
     }
+#endif
     const Real pace = mk_is_paced(a, c, ix, iy) ? p.pace : (Real)0;
     if (p.row >= 0 && a.nan_check && c == a.nan_cell && y[0] != y[0])
         __atomic_store_n(a.halt, p.row, __ATOMIC_RELAXED);
@@ -1312,25 +1323,3 @@ mk_strand(const MkArgs a, const MkStrand st, const int s0, const int s1)
                        st, s0, s1, xs, vt, &flag);
 }
 #endif
-
-/* ------------------------------------------------------------------------
- * Fiber-tissue junction (diff_step_fiber_tissue, openclsim.cl:601-628):
- * fiber row k's last cell (nfx - 1, k) connects to tissue cell (ctx,
- * cty + k) with conductance gft. The current gft (Vf - Vt) is written for
- * the fiber cell and its negative for the tissue cell, into arrays that
- * are zero elsewhere; the grid driver adds them after its stencil.
- * ---------------------------------------------------------------------- */
-extern "C" __global__ void __launch_bounds__(64)
-mk_junction(const Real* __restrict__ vf, const Real* __restrict__ vt,
-            Real* __restrict__ jf, Real* __restrict__ jt, const long long nfx,
-            const long long nfy, const long long ntx, const long long ctx,
-            const long long cty, const Real gft)
-{
-    const long long k = (long long)blockIdx.x * 64 + threadIdx.x;
-    if (k >= nfy) return;
-    const long long iff = (nfx - 1) + k * nfx;
-    const long long ift = ctx + (cty + k) * ntx;
-    const Real i = gft * (vf[iff] - vt[ift]);
-    jf[iff] = i;
-    jt[ift] = -i;
-}
