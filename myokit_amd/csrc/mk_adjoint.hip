@@ -542,9 +542,15 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
     const long long np = a.npad;
     const long long SN = (long long)MK_NS * np;
     /* lanes beyond the last column compute a copy of its cell and keep it to
-     * themselves (waves of at most 8 active lanes are slow, see mk_sheet) */
+     * themselves (waves of at most 8 active lanes are slow, see mk_sheet);
+     * not with 8 cells per thread, where the sheet fills the device and the
+     * guards cost every tile 1% */
+#if MK_ACPT < 8
     const bool own = ix < nx;
     const int xc = own ? ix : nx - 1;
+#else
+    const int xc = ix;
+#endif
     const int nb[4] = {ty > 0 ? tile - sh.tiles_x : -1,
                        ty + 1 < sh.tiles_y ? tile + sh.tiles_x : -1,
                        tx > 0 ? tile - 1 : -1,
@@ -606,7 +612,11 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
 #pragma unroll 1
         for (int k = 0; k < MK_ACPT; ++k) {
             const int r = w * MK_ACPT + k, iy = gy0 + r;
+#if MK_ACPT < 8
             if (iy >= ny) continue;
+#else
+            if (!(ix < nx && iy < ny)) continue;
+#endif
             const int c = xc + iy * nx;
             Real lam[MK_NS], y[MK_NS], mu[MK_NS], fv[MK_NFA], fb[MK_NFA], abo;
 #pragma unroll
@@ -616,7 +626,11 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
             }
 #pragma unroll
             for (int f = 0; f < MK_NF; ++f) fv[f] = a.fields[f * np + c];
+#if MK_ACPT < 8
             Real lv = mk_adj_loss(j, c, V1[c], own ? s : -1);
+#else
+            Real lv = mk_adj_loss(j, c, V1[c], s);
+#endif
             Real ck = (Real)0;
 #pragma unroll
             for (int q = 0; q < MK_ACPT; ++q) if (q == k) ck = lc[q];
@@ -626,7 +640,9 @@ mk_adj_sheet(const MkArgs a, const MkAdj j, const MkSheet sh, const int s0,
 #pragma unroll
             for (int q = 0; q < MK_NS; ++q) mul[q][r][lx] = mu[q];
             at[r + 1][lx + 1] = abo;
+#if MK_ACPT < 8
             if (!own) continue;
+#endif
             if (r == 0) mk_tput(mk_adj_edge(sh, par, tile, 0, lx), abo, i + 1);
             if (r == MK_ATH - 1)
                 mk_tput(mk_adj_edge(sh, par, tile, 1, lx), abo, i + 1);
