@@ -1104,7 +1104,12 @@ mk_chain(const MkArgs a, const MkChain ch, const int s0, const int s1)
  *
  * The NaN test at a log step records the first row only; the host then
  * takes the steps up to that row again from the launch's start state (which
- * is in state_a, untouched), so that the run ends where it always did.
+ * is in state_a, untouched), so that the run ends where it always did. No
+ * workgroup looks at that record: a launch spans many rows, so one that
+ * starts late would find an early row of the same launch there and leave
+ * without its steps, while its neighbours wait for them. (The drivers that
+ * end a launch at each row skip the launches queued behind it with
+ * mk_halted; here the host has read the record before the next launch.)
  * ---------------------------------------------------------------------- */
 typedef MkStrandT<Real> MkStrand;
 
@@ -1310,15 +1315,12 @@ mk_strand(const MkArgs a, const MkStrand st, const int s0, const int s1)
     __shared__ Real xs[2][MK_NXS][64];
     __shared__ Real vt[2][66];
     __shared__ int flag;
-    if (threadIdx.x == 0) flag = mk_halted(a, a.steps[s1 - 1].row) ? 1 : 0;
+    if (threadIdx.x == 0) flag = 0;
     if (threadIdx.x < 2) {
         vt[threadIdx.x][0] = (Real)0;
         vt[threadIdx.x][65] = (Real)0;
     }
     __syncthreads();
-    const bool stop = flag;
-    __syncthreads();
-    if (stop) return;
     mk_strand_group<0>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), a,
                        st, s0, s1, xs, vt, &flag);
 }

@@ -108,3 +108,38 @@ def test_nan_ends_the_run_where_other_drivers_do(n):
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
     assert len(out[0][0]) < 20 and np.isnan(out[0][2]).any()
+
+
+def _nan_run(s, driver, st):
+    """The columns of a run of 40 steps from state ``st`` with a row every 4,
+    and the state it leaves."""
+    s.set_tuning(driver=driver)
+    s.reset()
+    s.set_state(st.reshape(-1))
+    d = s.run(40 * DT, log=['membrane.V', 'ica.ICa', 'engine.time'],
+              log_interval=4 * DT, report_nan=False)
+    return [np.asarray(v) for v in d.values()] + [np.array(s.state())]
+
+
+# a NaN in cell 0 that the first of the launch's rows finds, on lines of many
+# tiles (the largest with several per CU) and on uncoupled cells, each after
+# a run whose rows fill the log buffer
+@pytest.mark.parametrize('n,coupled', [
+    (65, True), (1000, True), (8193, True), (30000, True), (64, False),
+    (1000, False), (49152, False)])
+def test_nan_in_the_first_row(n, coupled):
+    sc = _scenario(n) if coupled else Scenario(
+        'lr1991', n, diffusion=False, dt=DT, events=((1, 0, 0.5, 1000, 0),))
+    s = sc.product(32)
+    st = np.array(s.state()).reshape(n, -1)
+    bad = st.copy()
+    bad[0] = np.nan
+    out = []
+    for driver in ('strand', 'grid') if coupled else ('auto', 'cells'):
+        _nan_run(s, driver, st)
+        out.append(_nan_run(s, driver, bad))
+    assert len(out[0]) == 2 * n + 2
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+    assert all(len(a) == 1 for a in out[0][:-1])
+    assert np.isnan(out[0][-1]).any() and np.isfinite(out[0][-1][-8:]).all()
