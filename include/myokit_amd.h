@@ -212,6 +212,9 @@ int mkh_sim_clean(void* sim);
  *   "adj_linear"    0: keep lines of cells and uncoupled cells in double
  *                   precision on the reverse kernels that apply the cell
  *                   VJP step by step (default 1)
+ *   "repeat_spins"  polls before a neighbour wait of the steps that the
+ *                   strand driver takes again after a NaN is abandoned
+ *                   (default 2^20; fewer make such a run fail)
  *   "graph_copies"  K: the next graph is K identical copies held
  *                   interleaved (cell p of copy k is cell p * K + k), the
  *                   copies' connection lists one after the other; if every

@@ -342,6 +342,7 @@ struct Sim : SimBase {
     DevBuf<int> st_err;
     int st_tiles = 0, st_width = 0, st_halo = 0;
     long long st_done = 0;        /* exchanges completed in this run */
+    int repeat_spins = 1 << 20;   /* "repeat_spins" option */
     int sh_tx = 0, sh_ty = 0, sh_capacity = 0;
     long long sh_steps = 0;
     long long max_domain = 0;
@@ -510,8 +511,9 @@ struct Sim : SimBase {
     }
 
     /* Steps [s0, s1) from state `src` to state `dst` (two buffers) in one
-     * launch; `trajp` as MkStrandT. */
-    int strand_launch(Args a, R* src, R* dst, int s0, int s1, R* trajp)
+     * launch; `trajp` and `spins` (its spin_limit) as MkStrandT. */
+    int strand_launch(Args a, R* src, R* dst, int s0, int s1, R* trajp,
+                      int spins = 1 << 20)
     {
         a.state_a = src;
         a.state_b = dst;
@@ -523,7 +525,7 @@ struct Sim : SimBase {
         st.width = st_width;
         st.halo = st_halo;
         st.g0 = (int)st_done;
-        st.spin_limit = 1 << 20;
+        st.spin_limit = spins;
         st.traj = trajp;
         void* params[] = {&a, &st, &s0, &s1};
         if (st_halo > 0) {
@@ -1326,6 +1328,27 @@ struct Sim : SimBase {
         return emit_row(b, s + 1);
     }
 
+    /* After the stream is idle: fails if a neighbour wait of the persistent
+     * drivers timed out. */
+    int exchange_error()
+    {
+        const bool strand = driver == MKH_DRIVER_STRAND && st_halo > 0;
+        const int* err = driver == MKH_DRIVER_SHEET   ? sh_err.p
+                         : driver == MKH_DRIVER_CHAIN ? ch_err.p
+                         : strand                     ? st_err.p
+                                                      : nullptr;
+        if (!err) return 0;
+        int e = 0;
+        MKH_HIP(hipMemcpy(&e, err, sizeof(int), hipMemcpyDeviceToHost));
+        if (!e) return 0;
+        running = false;
+        return fail(MKH_E_HIP, std::string(driver == MKH_DRIVER_SHEET
+                                               ? "sheet"
+                                           : strand ? "strand"
+                                                    : "chain") +
+                                   " driver: a neighbour exchange timed out");
+    }
+
     /* Waits for the batch; copies times and paces of its rows. Returns the
      * number of valid rows (all, or up to the one where the NaN check
      * halted the run) through `valid`. */
@@ -1337,23 +1360,8 @@ struct Sim : SimBase {
                                stream));
         MKH_HIP(hipStreamSynchronize(stream));
         MKH_HIP(hipStreamSynchronize(copy_stream));
-        const bool strand = driver == MKH_DRIVER_STRAND && st_halo > 0;
-        const int* err = driver == MKH_DRIVER_SHEET   ? sh_err.p
-                         : driver == MKH_DRIVER_CHAIN ? ch_err.p
-                         : strand                     ? st_err.p
-                                                      : nullptr;
-        if (err) {
-            int e = 0;
-            MKH_HIP(hipMemcpy(&e, err, sizeof(int), hipMemcpyDeviceToHost));
-            if (e) {
-                running = false;
-                return fail(MKH_E_HIP,
-                            std::string(driver == MKH_DRIVER_SHEET ? "sheet"
-                                        : strand ? "strand"
-                                                 : "chain") +
-                                " driver: a neighbour exchange timed out");
-            }
-        }
+        int e = exchange_error();
+        if (e) return e;
         valid = b.nr;
         halted = h;
         if (h >= 0) valid = h + 1;
@@ -1520,9 +1528,11 @@ struct Sim : SimBase {
             while (s + 1 < ns && h_steps[s].row != halted) ++s;
             if (s + 1 < ns) {
                 e = strand_launch(base_args(), state[cur ^ 1].p, state[cur].p,
-                                  0, (int)(s + 1), nullptr);
+                                  0, (int)(s + 1), nullptr, repeat_spins);
                 if (e) return e;
                 MKH_HIP(hipStreamSynchronize(stream));
+                e = exchange_error();
+                if (e) return e;
             }
         }
         return close_batch(b, valid, halted, tout, status);
@@ -1581,6 +1591,8 @@ struct Sim : SimBase {
             no_sheet_rev = v == 0;
         } else if (k == "adj_linear") {
             no_adj_linear = v == 0;
+        } else if (k == "repeat_spins") {
+            repeat_spins = (int)std::max(-1LL, std::min(v, 1LL << 20));
         } else if (k == "adj_overlap") {
             no_adj_overlap = v == 0;
         } else {

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import myokit_amd as myokit
+from myokit_amd._err import DeviceError
 from tests.helpers import Scenario, run_both
 
 pytestmark = pytest.mark.gpu
@@ -110,14 +111,14 @@ def test_nan_ends_the_run_where_other_drivers_do(n):
     assert len(out[0][0]) < 20 and np.isnan(out[0][2]).any()
 
 
-def _nan_run(s, driver, st):
-    """The columns of a run of 40 steps from state ``st`` with a row every 4,
-    and the state it leaves."""
+def _nan_run(s, driver, st, rows=4):
+    """The columns of a run of 10 ``rows`` steps from state ``st`` with a row
+    every ``rows``, and the state it leaves."""
     s.set_tuning(driver=driver)
     s.reset()
     s.set_state(st.reshape(-1))
-    d = s.run(40 * DT, log=['membrane.V', 'ica.ICa', 'engine.time'],
-              log_interval=4 * DT, report_nan=False)
+    d = s.run(10 * rows * DT, log=['membrane.V', 'ica.ICa', 'engine.time'],
+              log_interval=rows * DT, report_nan=False)
     return [np.asarray(v) for v in d.values()] + [np.array(s.state())]
 
 
@@ -143,3 +144,20 @@ def test_nan_in_the_first_row(n, coupled):
         np.testing.assert_array_equal(a, b)
     assert all(len(a) == 1 for a in out[0][:-1])
     assert np.isnan(out[0][-1]).any() and np.isfinite(out[0][-1][-8:]).all()
+
+
+def test_exchange_timeout_of_the_repeated_steps_is_reported():
+    # the steps up to a NaN's row are taken again: if a wait of theirs times
+    # out (no polls allowed; the first launch has them all), the state is not
+    # the run's, and the run must say so
+    n = 1000
+    s = _scenario(n).product(32)
+    st = np.array(s.state()).reshape(n, -1)
+    st[0, 7] = -1e-3
+    _nan_run(s, 'strand', st, 20)
+    s.set_engine_option('repeat_spins', 0)
+    with pytest.raises(DeviceError, match='timed out'):
+        _nan_run(s, 'strand', st, 20)
+    s.set_engine_option('repeat_spins', 1 << 20)
+    d = _nan_run(s, 'strand', st, 20)
+    assert len(d[0]) == 2 and np.isnan(d[-1]).any()
