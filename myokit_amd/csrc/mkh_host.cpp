@@ -376,6 +376,7 @@ struct Sim : SimBase {
     Step* h_steps = nullptr;       /* pinned staging */
     size_t h_steps_cap = 0;
     std::vector<double> row_t_after;
+    std::vector<int> row_cur;      /* `cur` after each row's launch, or -1 */
 
     /* timing */
     double kernel_ms = 0;
@@ -1235,18 +1236,22 @@ struct Sim : SimBase {
                 b.plog.push_back((double)(R)r.pace);
             }
         }
+        row_cur.assign((size_t)b.nr, -1);
         if (b.ns > 0)
             MKH_HIP(hipMemcpyAsync(steps.p, h_steps, b.ns * sizeof(Step),
                                    hipMemcpyHostToDevice, stream));
         return 0;
     }
 
-    /* After the launch that ends with step s: if s logs a row, copy the row
-     * to the caller's buffer on the copy stream. */
+    /* After the launch that ends with step s: if s logs a row, note where
+     * the state then is, and copy the row to the caller's buffer on the copy
+     * stream. */
     int emit_row(const Batch& b, long long s)
     {
         const int row = h_steps[s].row;
-        if (!(b.nr > 0 && ncols > 0 && dst_values) || row < 0) return 0;
+        if (row < 0) return 0;
+        row_cur[row] = cur;
+        if (!(b.nr > 0 && ncols > 0 && dst_values)) return 0;
         hipEvent_t e = row_ev[row % 16];
         MKH_HIP(hipEventRecord(e, stream));
         MKH_HIP(hipStreamWaitEvent(copy_stream, e, 0));
@@ -1364,7 +1369,12 @@ struct Sim : SimBase {
         if (e) return e;
         valid = b.nr;
         halted = h;
-        if (h >= 0) valid = h + 1;
+        if (h >= 0) {
+            /* the launches after the row's have done nothing, but each of
+             * those that swap the state buffers was counted */
+            valid = h + 1;
+            if (row_cur[h] >= 0) cur = row_cur[h];
+        }
         if (time_kernels) {
             for (size_t k = 0; k + 1 < b.nev; k += 2) {
                 float ms = 0;

@@ -187,3 +187,25 @@ def test_nan_in_user_cell_0_of_a_reordered_graph():
     s.reset()
     with pytest.raises(myokit.SimulationError, match='Time: +1.23'):
         s.run(5, log_interval=0.1)
+
+
+@pytest.mark.parametrize('rows', [3, 4])
+@pytest.mark.parametrize('shape', [200, (24, 24)])
+def test_state_left_by_a_nan_run_is_that_of_its_row(shape, rows):
+    # the launches queued behind the NaN's row do nothing: an odd number of
+    # them must not leave the state of the step before
+    from tests.helpers import Scenario
+    out = []
+    for driver in ('block', 'grid') + (('sheet',) if shape != 200 else ()):
+        s = Scenario('lr1991', shape).product(32)
+        s.set_tuning(driver=driver)
+        st = np.array(s.state()).reshape(s._ntotal, -1)
+        st[0] = np.nan
+        s.set_state(st.reshape(-1))
+        d = s.run(10 * rows * 0.005, log=['membrane.V', 'engine.time'],
+                  log_interval=rows * 0.005, report_nan=False)
+        assert s.engine_driver() == driver
+        out.append((len(d['engine.time']), np.array(s.state())))
+    for n, state in out:
+        assert n == 1
+        np.testing.assert_array_equal(state, out[0][1])
