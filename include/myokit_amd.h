@@ -212,6 +212,9 @@ int mkh_sim_clean(void* sim);
  *   "adj_linear"    0: keep lines of cells and uncoupled cells in double
  *                   precision on the reverse kernels that apply the cell
  *                   VJP step by step (default 1)
+ *   "step_tags"     lets the step tags of the persistent drivers' exchanges,
+ *                   which grow to 2^31 and start again, go on from this value
+ *                   if it is larger than theirs
  *   "repeat_spins"  polls before a neighbour wait of the steps that the
  *                   strand driver takes again after a NaN is abandoned
  *                   (default 2^20; fewer make such a run fail)

@@ -312,7 +312,10 @@ struct Sim : SimBase {
     int cur = 0;                  /* state buffer holding the current state */
     hipStream_t stream = nullptr;
     DevBuf<R> state[2], fields, csr_g, gxf, gyf, logbuf;
-    DevBuf<int> colmap, csr_ptr, csr_idx, dom_cells, halt;
+    DevBuf<int> colmap, csr_ptr, csr_idx, dom_cells;
+    /* halt[0]: the row of a NaN, or -1; halt[1]: set to 1 by a neighbour
+     * wait of the persistent drivers that timed out */
+    DevBuf<int> halt;
     DevBuf<long long> dom_off;
     DevBuf<unsigned char> pace_mask;
     DevBuf<Step> steps;
@@ -328,20 +331,17 @@ struct Sim : SimBase {
     /* tile edges as step-tagged words: one per 32 bits of a value */
     static constexpr int XW = (int)(sizeof(R) / 4);
     DevBuf<unsigned long long> sh_edges;
-    DevBuf<int> sh_err;
     /* chain driver (graphs whose every connection joins cells c, c + 1) */
     DevBuf<R> ch_gl, ch_gr;
     DevBuf<unsigned long long> ch_edges;
     DevBuf<unsigned char> ch_cf;
-    DevBuf<int> ch_err;
     bool is_chain = false;
     int ch_tiles = 0, ch_len = 0;
     long long ch_steps = 0;
     /* strand driver: lines of cells and uncoupled cells in few tiles */
     DevBuf<unsigned long long> st_edges;
-    DevBuf<int> st_err;
     int st_tiles = 0, st_width = 0, st_halo = 0;
-    long long st_done = 0;        /* exchanges completed in this run */
+    long long st_done = 0;        /* exchanges completed */
     int repeat_spins = 1 << 20;   /* "repeat_spins" option */
     int sh_tx = 0, sh_ty = 0, sh_capacity = 0;
     long long sh_steps = 0;
@@ -422,9 +422,9 @@ struct Sim : SimBase {
             MKH_HIP(fields.alloc((size_t)cfg.n_field * npad));
             MKH_HIP(hipMemset(fields.p, 0, fields.n * sizeof(R)));
         }
-        MKH_HIP(halt.alloc(1));
-        int m1 = -1;
-        MKH_HIP(hipMemcpy(halt.p, &m1, sizeof(int), hipMemcpyHostToDevice));
+        MKH_HIP(halt.alloc(2));
+        int e = reset_flags();
+        if (e) return e;
         long long off[2] = {0, n};
         MKH_HIP(dom_off.alloc(2));
         MKH_HIP(hipMemcpy(dom_off.p, off, sizeof(off), hipMemcpyHostToDevice));
@@ -444,13 +444,11 @@ struct Sim : SimBase {
                     (long long)sh_tx * sh_ty,
                     p->f_adj_sheet ? adj_sheet_tiles() : 0);
                 MKH_HIP(sh_edges.alloc(2 * nt * 4 * 64 * XW));
-                MKH_HIP(sh_err.alloc(1));
                 MKH_HIP(hipMemset(sh_edges.p, 0,
                                   sh_edges.n * sizeof(unsigned long long)));
-                MKH_HIP(hipMemset(sh_err.p, 0, sizeof(int)));
             }
         }
-        int e = build_strand_layout();
+        e = build_strand_layout();
         if (e) return e;
         choose_driver();
         return 0;
@@ -489,8 +487,6 @@ struct Sim : SimBase {
             break;
         }
         if (st_tiles == 0) return 0;
-        MKH_HIP(st_err.alloc(1));
-        MKH_HIP(hipMemset(st_err.p, 0, sizeof(int)));
         if (st_halo > 0) {
             MKH_HIP(st_edges.alloc((size_t)st_tiles * 4 * cfg.n_state * 32 *
                                    XW));
@@ -516,12 +512,16 @@ struct Sim : SimBase {
     int strand_launch(Args a, R* src, R* dst, int s0, int s1, R* trajp,
                       int spins = 1 << 20)
     {
+        if (st_halo > 0) {
+            int e = reserve_tags(st_edges, st_done, s1 - s0);
+            if (e) return e;
+        }
         a.state_a = src;
         a.state_b = dst;
         MkStrandT<R> st;
         std::memset(&st, 0, sizeof(st));
         st.edges = st_edges.p;
-        st.err = st_err.p;
+        st.err = halt.p + 1;
         st.tiles = st_tiles;
         st.width = st_width;
         st.halo = st_halo;
@@ -780,10 +780,8 @@ struct Sim : SimBase {
                           hipMemcpyHostToDevice));
         MKH_HIP(hipMemcpy(ch_cf.p, cf.data(), npad, hipMemcpyHostToDevice));
         MKH_HIP(ch_edges.alloc((size_t)tiles * 4 * XW));
-        MKH_HIP(ch_err.alloc(1));
         MKH_HIP(hipMemset(ch_edges.p, 0,
                           ch_edges.n * sizeof(unsigned long long)));
-        MKH_HIP(hipMemset(ch_err.p, 0, sizeof(int)));
         ch_steps = 0;
         ch_tiles = (int)tiles;
         ch_len = (int)len;
@@ -1066,8 +1064,8 @@ struct Sim : SimBase {
         if (nrows) *nrows = rows;
         dst_values = nullptr;
         dst_times = dst_paces = nullptr;
-        int m1 = -1;
-        MKH_HIP(hipMemcpy(halt.p, &m1, sizeof(int), hipMemcpyHostToDevice));
+        f = reset_flags();
+        if (f) return f;
         /* Device log buffer: whole run if it fits a budget, else batches */
         long long cap = log_rows_cap;
         if (cap <= 0) {
@@ -1080,25 +1078,6 @@ struct Sim : SimBase {
             MKH_HIP(logbuf.alloc((size_t)cap * ncols));
         }
         log_rows_cap_run = cap;
-        /* the step tags restart: old tags must not pass for new ones */
-        if (sh_edges.p) {
-            MKH_HIP(hipMemset(sh_edges.p, 0,
-                              sh_edges.n * sizeof(unsigned long long)));
-            MKH_HIP(hipMemset(sh_err.p, 0, sizeof(int)));
-            sh_steps = 0;
-        }
-        if (ch_edges.p) {
-            MKH_HIP(hipMemset(ch_edges.p, 0,
-                              ch_edges.n * sizeof(unsigned long long)));
-            MKH_HIP(hipMemset(ch_err.p, 0, sizeof(int)));
-            ch_steps = 0;
-        }
-        if (st_edges.p) {
-            MKH_HIP(hipMemset(st_edges.p, 0,
-                              st_edges.n * sizeof(unsigned long long)));
-            MKH_HIP(hipMemset(st_err.p, 0, sizeof(int)));
-            st_done = 0;
-        }
         size_t need = (size_t)batch_steps;
         MKH_HIP(steps.alloc(need));
         if (h_steps_cap < need) {
@@ -1162,7 +1141,7 @@ struct Sim : SimBase {
         MkSheetT<R> sh;
         std::memset(&sh, 0, sizeof(sh));
         sh.edges = sh_edges.p;
-        sh.err = sh_err.p;
+        sh.err = halt.p + 1;
         sh.tiles_x = sh_tx;
         sh.tiles_y = sh_ty;
         sh.spin_limit = 1 << 20;
@@ -1178,7 +1157,7 @@ struct Sim : SimBase {
         ch.gr = ch_gr.p;
         ch.cf = ch_cf.p;
         ch.edges = ch_edges.p;
-        ch.err = ch_err.p;
+        ch.err = halt.p + 1;
         ch.tiles = ch_tiles;
         ch.tile_len = ch_len;
         ch.spin_limit = 1 << 20;
@@ -1333,25 +1312,45 @@ struct Sim : SimBase {
         return emit_row(b, s + 1);
     }
 
-    /* After the stream is idle: fails if a neighbour wait of the persistent
-     * drivers timed out. */
-    int exchange_error()
+    /* Queues the copy of the flags and waits for the stream: the NaN's row
+     * or -1 in h; fails if a neighbour wait of the persistent drivers timed
+     * out. */
+    int read_flags(int& h)
     {
-        const bool strand = driver == MKH_DRIVER_STRAND && st_halo > 0;
-        const int* err = driver == MKH_DRIVER_SHEET   ? sh_err.p
-                         : driver == MKH_DRIVER_CHAIN ? ch_err.p
-                         : strand                     ? st_err.p
-                                                      : nullptr;
-        if (!err) return 0;
-        int e = 0;
-        MKH_HIP(hipMemcpy(&e, err, sizeof(int), hipMemcpyDeviceToHost));
-        if (!e) return 0;
+        int f[2] = {-1, 0};
+        MKH_HIP(hipMemcpyAsync(f, halt.p, sizeof(f), hipMemcpyDeviceToHost,
+                               stream));
+        MKH_HIP(hipStreamSynchronize(stream));
+        h = f[0];
+        if (!f[1]) return 0;
         running = false;
-        return fail(MKH_E_HIP, std::string(driver == MKH_DRIVER_SHEET
-                                               ? "sheet"
-                                           : strand ? "strand"
-                                                    : "chain") +
-                                   " driver: a neighbour exchange timed out");
+        return fail(MKH_E_HIP,
+                    std::string(driver == MKH_DRIVER_SHEET   ? "sheet"
+                                : driver == MKH_DRIVER_CHAIN ? "chain"
+                                                             : "strand") +
+                        " driver: a neighbour exchange timed out");
+    }
+
+    int reset_flags()
+    {
+        const int f[2] = {-1, 0};
+        MKH_HIP(hipMemcpy(halt.p, f, sizeof(f), hipMemcpyHostToDevice));
+        return 0;
+    }
+
+    /* Before a launch that takes the step tags done + 1 .. done + steps: the
+     * tags only grow, from run to run too, so that an old word never passes
+     * for a new one and nothing has to be cleared in between (a blocking
+     * call each, 10 us or more, in every run); before they would leave 31
+     * bits the words are cleared and the tags start again. */
+    int reserve_tags(DevBuf<unsigned long long>& edges, long long& done,
+                     long long steps)
+    {
+        if (done + steps < INT_MAX) return 0;
+        MKH_HIP(hipMemsetAsync(edges.p, 0,
+                               edges.n * sizeof(unsigned long long), stream));
+        done = 0;
+        return 0;
     }
 
     /* Waits for the batch; copies times and paces of its rows. Returns the
@@ -1361,11 +1360,8 @@ struct Sim : SimBase {
     {
         cell_steps += b.ns * n;
         int h = -1;
-        MKH_HIP(hipMemcpyAsync(&h, halt.p, sizeof(int), hipMemcpyDeviceToHost,
-                               stream));
-        MKH_HIP(hipStreamSynchronize(stream));
+        int e = read_flags(h);
         MKH_HIP(hipStreamSynchronize(copy_stream));
-        int e = exchange_error();
         if (e) return e;
         valid = b.nr;
         halted = h;
@@ -1442,6 +1438,8 @@ struct Sim : SimBase {
                     /* reads state[cur], writes state[cur ^ 1] */
                     Args a = base_args();
                     int i0 = (int)s0, i1 = (int)(s + 1);
+                    e = reserve_tags(sh_edges, sh_steps, i1 - i0);
+                    if (e) return e;
                     sh.g0 = (int)sh_steps;
                     void* params[] = {&a, &sh, &i0, &i1};
                     if (time_kernels)
@@ -1469,6 +1467,8 @@ struct Sim : SimBase {
                     /* reads state[cur], writes state[cur ^ 1] */
                     Args a = base_args();
                     int i0 = (int)s0, i1 = (int)(s + 1);
+                    e = reserve_tags(ch_edges, ch_steps, i1 - i0);
+                    if (e) return e;
                     ch.g0 = (int)ch_steps;
                     void* params[] = {&a, &ch, &i0, &i1};
                     if (time_kernels)
@@ -1540,8 +1540,8 @@ struct Sim : SimBase {
                 e = strand_launch(base_args(), state[cur ^ 1].p, state[cur].p,
                                   0, (int)(s + 1), nullptr, repeat_spins);
                 if (e) return e;
-                MKH_HIP(hipStreamSynchronize(stream));
-                e = exchange_error();
+                int h = -1;
+                e = read_flags(h);
                 if (e) return e;
             }
         }
@@ -1601,6 +1601,10 @@ struct Sim : SimBase {
             no_sheet_rev = v == 0;
         } else if (k == "adj_linear") {
             no_adj_linear = v == 0;
+        } else if (k == "step_tags") {
+            sh_steps = ch_steps = st_done =
+                std::max(std::max(sh_steps, ch_steps),
+                         std::max(st_done, std::min(v, (long long)INT_MAX)));
         } else if (k == "repeat_spins") {
             repeat_spins = (int)std::max(-1LL, std::min(v, 1LL << 20));
         } else if (k == "adj_overlap") {
@@ -1858,8 +1862,8 @@ struct Sim : SimBase {
             j.probe_of = probe_of.p;
             j.target = dtarget.p;
         }
-        int m1 = -1;
-        MKH_HIP(hipMemcpy(halt.p, &m1, sizeof(int), hipMemcpyHostToDevice));
+        f = reset_flags();
+        if (f) return f;
 
         Args a = base_args();
         a.steps = dsteps.p;
@@ -1961,6 +1965,8 @@ struct Sim : SimBase {
             } else if (driver == MKH_DRIVER_SHEET) {
                 R* wnext = wcur == work.p ? work2.p : work.p;
                 as.state_b = wnext;
+                int e = reserve_tags(sh_edges, sh_steps, s1 - s0);
+                if (e) return e;
                 MkSheetT<R> sh = sheet_args();
                 sh.g0 = (int)sh_steps;
                 sh.traj = trajp;
@@ -2171,7 +2177,7 @@ struct Sim : SimBase {
                     std::memset(&ln, 0, sizeof(ln));
                     ln.jac = adj.jac.p;
                     ln.edges = adj.lin_edges.p;
-                    ln.err = st_err.p;
+                    ln.err = halt.p + 1;
                     ln.base = (int)e0;
                     ln.fresh = mu_in == nullptr;
                     ln.tiles = st_tiles;
@@ -2218,9 +2224,9 @@ struct Sim : SimBase {
                 int i0 = (int)s0, i1 = (int)s1;
                 int flags = (sg == nseg - 1 ? 1 : 0) | (sg == 0 ? 2 : 0);
                 /* the reverse tags start at 1 in every launch: clear the
-                 * edge words (the forward's tags are larger, and they stay
-                 * above the reverse's: tags only grow until a run's init
-                 * clears the words) */
+                 * edge words (the forward's tags are larger, and those of
+                 * later forward steps stay above the reverse's, of which a
+                 * launch takes no more than the forward took) */
                 MKH_HIP(hipMemsetAsync(sh_edges.p, 0,
                                        sh_edges.n * sizeof(unsigned long long),
                                        stream));
@@ -2264,8 +2270,8 @@ struct Sim : SimBase {
         MKH_HIP(hipEventSynchronize(ev[3]));
         if (driver == MKH_DRIVER_SHEET || (use_strand && st_halo > 0)) {
             int e = 0;
-            MKH_HIP(hipMemcpy(&e, use_strand ? st_err.p : sh_err.p,
-                              sizeof(int), hipMemcpyDeviceToHost));
+            MKH_HIP(hipMemcpy(&e, halt.p + 1, sizeof(int),
+                              hipMemcpyDeviceToHost));
             if (e)
                 return fail(MKH_E_HIP,
                             std::string(use_strand ? "strand" : "sheet") +
@@ -2458,8 +2464,10 @@ struct Sim : SimBase {
             MKH_HIP(hipMemcpy(dprobes, probes,
                               (size_t)nprobe * sizeof(long long),
                               hipMemcpyHostToDevice));
-        const int m1 = -1;
-        MKH_HIP(hipMemcpy(halt.p, &m1, sizeof(int), hipMemcpyHostToDevice));
+        {
+            int e = reset_flags();
+            if (e) return e;
+        }
         MkAdjT<R> j;
         std::memset(&j, 0, sizeof(j));
         j.probes = dprobes;
@@ -2479,6 +2487,8 @@ struct Sim : SimBase {
                 Args as = a;
                 as.state_a = wa;
                 as.state_b = wb;
+                int e = reserve_tags(sh_edges, sh_steps, 1);
+                if (e) return e;
                 MkSheetT<R> sh = sheet_args();
                 sh.g0 = (int)sh_steps;
                 int i0 = sii, i1 = sii + 1;
@@ -2518,7 +2528,7 @@ struct Sim : SimBase {
         MKH_HIP(hipStreamSynchronize(stream));
         if (driver == MKH_DRIVER_SHEET) {
             int e = 0;
-            MKH_HIP(hipMemcpy(&e, sh_err.p, sizeof(int),
+            MKH_HIP(hipMemcpy(&e, halt.p + 1, sizeof(int),
                               hipMemcpyDeviceToHost));
             if (e)
                 return fail(MKH_E_HIP, "sheet driver: a neighbour exchange "

@@ -161,3 +161,30 @@ def test_exchange_timeout_of_the_repeated_steps_is_reported():
     s.set_engine_option('repeat_spins', 1 << 20)
     d = _nan_run(s, 'strand', st, 20)
     assert len(d[0]) == 2 and np.isnan(d[-1]).any()
+
+
+@pytest.mark.parametrize('driver', ['strand', 'sheet', 'chain'])
+def test_exchange_tags_start_again_before_they_overflow(driver):
+    # the tags go on from run to run; near 2^31 the words are cleared and
+    # they start again, in the first launch, a later one or a later run
+    def make():
+        if driver == 'chain':
+            s = Scenario('lr1991', 300, connections=[
+                (i, i + 1, 9.5) for i in range(299)],
+                paced_list=[0, 1]).product(32)
+        else:
+            s = _scenario(300 if driver == 'strand' else (30, 20)).product(32)
+        s.set_tuning(driver=driver)
+        s.run_block(20 * DT, ['membrane.V'], log_interval=DT * 10)
+        return s
+
+    def go(s):
+        b = [s.run_block(k * DT, ['membrane.V'], log_interval=DT * 20)
+             ['membrane.V'] for k in (60, 90, 40)]
+        assert s.engine_driver() == driver
+        return np.concatenate(b)
+    want = go(make())
+    for left in (5, 50, 100, 150, 300):
+        s = make()
+        s.set_engine_option('step_tags', 2 ** 31 - 1 - left)
+        np.testing.assert_array_equal(go(s), want)
