@@ -1403,6 +1403,37 @@ struct Sim : SimBase {
         return 0;
     }
 
+    /* Fewest steps of a batch that the strand driver takes by itself. Where
+     * tiles exchange, its launch is cooperative, which costs some 18 us more
+     * than an ordinary one. A step on it gains, single and double precision,
+     * 0.65 and 2.5 us over mk_block (which steps lines of at most 512 cells
+     * otherwise) and some 3 us over mk_grid. Rows cost it nothing, while each
+     * costs the others an event and a copy: a batch with one is the faster
+     * here from the first step (one step of 200 cells with its row 92 us per
+     * call, on mk_block 100), but for the longest lines (49,000 cells 117 and
+     * 110). */
+    long long strand_steps(const Batch& b) const
+    {
+        if (st_halo == 0 || forced_driver == MKH_DRIVER_STRAND) return 0;
+        if (b.nr > 0 && ncols > 0 && dst_values) return n <= 16384 ? 0 : 4;
+        if (n <= 512) return sizeof(R) == 4 ? 24 : 8;
+        return sizeof(R) == 4 ? 6 : 5;
+    }
+
+    /* Fewest steps of a launch (one per log row) of the sheet driver: its
+     * launches are cooperative. us per row, sheet and grid driver, rows every
+     * 4, 6, 8, 10 steps: single precision 64 x 64 61 and 61, 65 and 67, 69
+     * and 74, 72 and 78; 301 x 217 45 and 43, 49 and 52; 600 x 600 62 and 54,
+     * 69 and 69, 76 and 86; 1024 x 1024 118 and 114, 127 and 132; double
+     * precision 64 x 64 86 and 75, 98 and 90, 109 and 105, 107 and 106; 301 x
+     * 217 71 and 58, 87 and 78, 102 and 100, 117 and 120; 600 x 600 129 and
+     * 118, 167 and 164, 206 and 212. */
+    long long sheet_steps() const
+    {
+        if (forced_driver == MKH_DRIVER_SHEET) return 0;
+        return sizeof(R) == 4 ? 6 : n > 65536 ? 8 : 10;
+    }
+
     int step(double* tout, int* status) override
     {
         if (!running) return fail(MKH_E_STATE, "simulation not initialised");
@@ -1417,24 +1448,38 @@ struct Sim : SimBase {
         }
         /* Launch */
         const unsigned bt = (unsigned)cfg.block_threads;
-        const bool strand = driver == MKH_DRIVER_STRAND ||
+        const bool strand = (driver == MKH_DRIVER_STRAND &&
+                             ns >= strand_steps(b)) ||
                             (driver == MKH_DRIVER_CELLS && strand_for(driver));
-        if (driver == MKH_DRIVER_GRID) {
-            const bool two = prog->f_grid2 && cfg.ny > 1 && n >= two_cells;
-            for (long long s = 0; s < ns; ++s) {
-                if (two && s + 1 < ns && h_steps[s].row < 0) {
-                    e = grid2_launch(b, s++);
-                } else {
-                    e = grid_launch(b, s, nullptr);
-                }
+        /* batches too short for the strand's cooperative launch */
+        const int d = driver != MKH_DRIVER_STRAND || strand ? driver
+                      : n <= 512 ? MKH_DRIVER_BLOCK
+                                 : MKH_DRIVER_GRID;
+        const bool two = prog->f_grid2 && cfg.ny > 1 && n >= two_cells;
+        auto grid_steps = [&](long long s0, long long s1) -> int {
+            for (long long s = s0; s < s1; ++s) {
+                int e = two && s + 1 < s1 && h_steps[s].row < 0
+                            ? grid2_launch(b, s++)
+                            : grid_launch(b, s, nullptr);
                 if (e) return e;
             }
-        } else if (driver == MKH_DRIVER_SHEET) {
+            return 0;
+        };
+        if (d == MKH_DRIVER_GRID) {
+            e = grid_steps(0, ns);
+            if (e) return e;
+        } else if (d == MKH_DRIVER_SHEET) {
             MkSheetT<R> sh = sheet_args();
             const unsigned ntiles = (unsigned)(sh_tx * sh_ty);
             long long s0 = 0;
             for (long long s = 0; s < ns; ++s) {
                 if (h_steps[s].row >= 0 || s == ns - 1) {
+                    if (s + 1 - s0 < sheet_steps()) {
+                        e = grid_steps(s0, s + 1);
+                        if (e) return e;
+                        s0 = s + 1;
+                        continue;
+                    }
                     /* reads state[cur], writes state[cur ^ 1] */
                     Args a = base_args();
                     int i0 = (int)s0, i1 = (int)(s + 1);
@@ -1459,7 +1504,7 @@ struct Sim : SimBase {
                     if (e) return e;
                 }
             }
-        } else if (driver == MKH_DRIVER_CHAIN) {
+        } else if (d == MKH_DRIVER_CHAIN) {
             MkChainT<R> ch = chain_args();
             long long s0 = 0;
             for (long long s = 0; s < ns; ++s) {
@@ -1506,9 +1551,9 @@ struct Sim : SimBase {
                     stream));
             cur ^= 1;
         } else {
-            hipFunction_t f = driver == MKH_DRIVER_CELLS ? prog->f_cells
-                                                         : prog->f_block;
-            unsigned grid = driver == MKH_DRIVER_CELLS
+            hipFunction_t f = d == MKH_DRIVER_CELLS ? prog->f_cells
+                                                    : prog->f_block;
+            unsigned grid = d == MKH_DRIVER_CELLS
                                 ? (unsigned)((n + bt - 1) / bt)
                                 : (unsigned)ndom;
             Args a = base_args();

@@ -97,3 +97,28 @@ def test_fp32_two_steps_per_launch_equal_one(shape, field):
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_array_equal(out[0][1], out[1][1])
     np.testing.assert_array_equal(out[0][1], out[2][1])
+
+
+@pytest.mark.parametrize('shape,prec,row', [
+    ((40, 20), 32, 6), ((40, 20), 64, 10), ((200, 97), 32, 6),
+    ((257, 257), 64, 8)])
+@pytest.mark.parametrize('field', [False, True])
+def test_rows_too_close_for_a_sheet_launch(shape, prec, row, field):
+    # rows every `row` steps take a launch each (the first row's step one),
+    # closer ones one per step; equal results
+    dt = 1.0 / 128          # times are exact
+    for every, steps in ((row, 6 * row + 1), (row - 1, 6 * row - 5)):
+        out = []
+        for driver in ('auto', 'grid'):
+            s = _scenario(shape, field).product(prec)
+            s.set_tuning(driver=driver)
+            s.set_step_size(dt)
+            b = s.run_block(steps * dt, ['membrane.V'],
+                            log_interval=every * dt)
+            if driver == 'auto':
+                assert s.engine_driver() == 'sheet'
+                assert s.engine_timing()['launches'] == (
+                    1 + 6 if every == row else steps)
+            out.append((b['membrane.V'], np.array(s.state())))
+        for a, b in zip(*out):
+            np.testing.assert_array_equal(a, b)

@@ -64,7 +64,8 @@ def _run(s, steps, rows):
 @pytest.mark.parametrize('rl', [False, True])
 def test_fp32_equals_grid_across_run_lengths(n, rl):
     out = []
-    for driver in ('auto', 'grid'):
+    for driver in ('auto' if n > 49152 else 'strand', 'grid'):
+        # (asked for, the driver takes short batches too)
         s = _scenario(n, rl=rl).product(32)
         s.set_tuning(driver=driver)
         out.append(_run(s, (1, 15, 16, 17, 40, 33), 7))
@@ -188,3 +189,26 @@ def test_exchange_tags_start_again_before_they_overflow(driver):
         s = make()
         s.set_engine_option('step_tags', 2 ** 31 - 1 - left)
         np.testing.assert_array_equal(go(s), want)
+
+
+@pytest.mark.parametrize('n,prec,least', [
+    (200, 32, 24), (200, 64, 8), (1000, 32, 6), (1000, 64, 5), (20000, 32, 6),
+    (64, 32, 1)])
+def test_batches_too_short_for_a_cooperative_launch(n, prec, least):
+    # a run's last row ends a batch, the steps after it are another one: with
+    # a row at the first step only, one step and then steps - 1
+    for steps in (least, least + 1):
+        out = []
+        for driver in ('auto', 'strand'):
+            s = _scenario(n).product(prec)
+            s.set_tuning(driver=driver)
+            b = s.run_block(steps * DT, ['membrane.V'], log_interval=1000)
+            assert s.engine_driver() == 'strand' and len(b['time']) == 1
+            one = driver == 'strand' or steps > least or least == 1
+            # the other driver's launches: one per step, of mk_block (up to
+            # 512 cells) one per batch
+            assert s.engine_timing()['launches'] == (
+                min(steps, 2) if one or n <= 512 else steps)
+            out.append((b['membrane.V'], np.array(s.state())))
+        for a, b in zip(*out):
+            np.testing.assert_array_equal(a, b)
