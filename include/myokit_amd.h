@@ -205,13 +205,15 @@ int mkh_sim_clean(void* sim);
  *   "adj_release"   1: free the adjoint's trajectory and work buffers
  *   "adj_sheet"     0: on a persistent sheet, take the adjoint's reverse
  *                   sweep one launch per step instead of one persistent
- *                   launch per segment (default 1)
+ *                   launch per segment; 1: always one per segment (default:
+ *                   where segments are long enough to gain from it)
  *   "adj_overlap"   0: recompute earlier segments in line with the reverse
  *                   steps, also where a second stream could overlap them
  *                   (default 1)
  *   "adj_linear"    0: keep lines of cells and uncoupled cells in double
  *                   precision on the reverse kernels that apply the cell
- *                   VJP step by step (default 1)
+ *                   VJP step by step; 1: never (default: where segments are
+ *                   long enough to gain from it)
  *   "step_tags"     lets the step tags of the persistent drivers' exchanges,
  *                   which grow to 2^31 and start again, go on from this value
  *                   if it is larger than theirs

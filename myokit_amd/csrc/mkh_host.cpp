@@ -1643,9 +1643,9 @@ struct Sim : SimBase {
         } else if (k == "adj_release") {
             if (v) adj.release();
         } else if (k == "adj_sheet") {
-            no_sheet_rev = v == 0;
+            adj_sheet = v != 0;
         } else if (k == "adj_linear") {
-            no_adj_linear = v == 0;
+            adj_linear = v != 0;
         } else if (k == "step_tags") {
             sh_steps = ch_steps = st_done =
                 std::max(std::max(sh_steps, ch_steps),
@@ -1692,14 +1692,16 @@ struct Sim : SimBase {
     /* Adjoint work buffers, kept between calls (sizes permitting) and
      * released by the "adj_release" option or with the simulation. */
     /* "adj_sheet" option: 0 keeps the sheet's reverse sweep on the
-     * one-step kernel (mk_adj_step) */
-    bool no_sheet_rev = false;
+     * one-step kernel (mk_adj_step), 1 takes mk_adj_sheet wherever it can
+     * run, -1 where it is the faster one */
+    int adj_sheet = -1;
     /* "adj_overlap" option: 0 keeps the recomputation of earlier segments
      * in line with the reverse steps on small domains */
     bool no_adj_overlap = false;
     /* "adj_linear" option: 0 keeps lines of cells on the kernels that apply
-     * the cell VJP step by step */
-    bool no_adj_linear = false;
+     * the cell VJP step by step, 1 takes the linear pass wherever it can run,
+     * -1 where it is the faster one */
+    int adj_linear = -1;
     /* most cells of the linear reverse pass */
     static constexpr long long lin_cells = 8192;
     /* second stream (default priority) for overlapped recomputation */
@@ -1757,6 +1759,55 @@ struct Sim : SimBase {
      * last to first: recompute the segment's states from its checkpoint
      * (not needed for the last), then one fused reverse step per time step.
      * With K >= N nothing is recomputed. */
+    /* Whether the persistent reverse sheet can run: its tiles co-resident,
+     * and the edge words enough for them. */
+    bool adj_sheet_fits() const
+    {
+        const long long tiles = adj_sheet_tiles();
+        return cfg.adj_cpt > 0 && prog->f_adj_sheet && sh_edges.p &&
+               (size_t)tiles * 4 * 64 * 2 * XW <= sh_edges.n &&
+               (long long)prog->cu_adj_sheet * prog->ncu >= tiles;
+    }
+
+    /* Fewest steps of a segment that the adjoint of a line or of uncoupled
+     * cells takes on the strand kernel (`lin`: and the linear reverse pass).
+     * A segment costs two or three launches of some 19 us more than the
+     * ordinary ones where tiles exchange. us per step, this and the other
+     * kernels, 200 steps: linear pass, 1,000 cells, segments of 5 and 10
+     * steps 26.4 and 18.4, 15.4 and 17.6, 8,000 cells 27.5 and 19.7, 17.9 and
+     * 18.0, without exchange segments of 1, 2 and 5 54 and 40, 29 and 27, 13
+     * and 20; one-step kernel, 1,000 cells in single precision, segments of 5,
+     * 10 and 20 20.5 and 18.0, 14.4 and 15.9, 11.0 and 12.1, 20,000 in double
+     * 20 and 50 18.3 and 17.6, 15.6 and 17.1; mk_adj_block, 200 cells in
+     * single precision, 20, 50 and 100 8.0 and 6.9, 5.8 and 5.8, 4.9 and 5.2
+     * (Beeler-Reuter, 50: 5.4 and 5.0). */
+    long long adj_strand_steps(bool lin) const
+    {
+        if (st_halo == 0) return lin ? 3 : 0;
+        if (lin) return 10;
+        return n <= 512 ? 96 : sizeof(R) == 4 ? 16 : 32;
+    }
+
+    /* The same for the adjoint of a sheet: whether segments of K steps take
+     * the grid driver's kernels. Those can recompute a segment under the
+     * reverse steps of the next on sheets that leave room (`overlap_fits`),
+     * which outweighs the forward steps' gain where the reverse steps are the
+     * same either way, and hid them on the smallest sheets. us per step, this
+     * and the grid driver's kernels, segments of 10, 20, 50 and 100 steps: 24 x
+     * 24 in single precision 16.3 and 15.5, 11.8 and 14.2, 8.8 and 11.2, 7.4
+     * and 10.7, in double 26.3 and 18.4, 21.6 and 17.9, 18.0 and 17.6, 16.0
+     * and 17.3, with a conductance field (one-step reverse kernel) 25.9 and
+     * 17.3, 22.2 and 16.7, 19.5 and 16.5, 17.3 and 16.3; 301 x 217 with a field
+     * (no overlap) 18.2 and 17.3, 14.4 and 15.7 in single precision, 32.4 and
+     * 31.2, 28.1 and 29.4 in double. */
+    bool adj_short_sheet(long long K, bool overlap_fits) const
+    {
+        if (forced_driver == MKH_DRIVER_SHEET || adj_sheet >= 0) return false;
+        if (adj_sheet_fits())
+            return n <= 4096 && K < (sizeof(R) == 4 ? 16 : 64);
+        return overlap_fits || K < 16;
+    }
+
     int adj_run(double tmin, double tmax, double dt, const double* events,
                 long long nev, const long long* probes, long long nprobe,
                 const double* target, long long nrows, int K, double* loss,
@@ -1769,7 +1820,7 @@ struct Sim : SimBase {
                              trace_out, nrows, nullptr, 0);
         /* the chain layout's adjoint runs on the grid driver (its CSR is
          * built with it) */
-        const bool use_strand = strand_for(driver);
+        bool use_strand = strand_for(driver);
         DriverAs as_grid(driver, driver == MKH_DRIVER_CHAIN ||
                                          driver == MKH_DRIVER_STRAND
                                      ? MKH_DRIVER_GRID
@@ -1824,6 +1875,20 @@ struct Sim : SimBase {
         const unsigned bt = (unsigned)cfg.block_threads;
         const unsigned ggrid = grid_launch_size();
         const unsigned cgrid = (unsigned)((n + bt - 1) / bt);
+        /* Segments too short for the cooperative launches they would take
+         * keep the ordinary ones */
+        const bool lin_rev_fits = use_strand && prog->f_adj_lin &&
+                                  n <= lin_cells && adj_linear != 0;
+        if (use_strand && forced_driver != MKH_DRIVER_STRAND &&
+            !(lin_rev_fits && adj_linear == 1) &&
+            Kl < adj_strand_steps(lin_rev_fits))
+            use_strand = false;
+        const bool overlap_fits = nseg > 1 && !no_adj_overlap &&
+                                  (long long)ggrid + cgrid <= prog->ncu;
+        DriverAs as_short(driver, driver == MKH_DRIVER_SHEET &&
+                                          adj_short_sheet(Kl, overlap_fits)
+                                      ? MKH_DRIVER_GRID
+                                      : driver);
         /* conductance-gradient partial sums: one per workgroup of the
          * reverse kernel (per domain on the block layout, per tile on the
          * sheet) */
@@ -1935,23 +2000,15 @@ struct Sim : SimBase {
          * the kernel source), all co-resident */
         const int rtx = sh_tx;
         const int rty = sh_tx > 0 ? (int)(adj_sheet_tiles() / sh_tx) : 0;
-        bool sheet_rev = false;
-        if (driver == MKH_DRIVER_SHEET && cfg.adj_cpt > 0 &&
-            prog->f_adj_sheet &&
-            sh_edges.p && (size_t)rtx * rty * 4 * 64 * 2 * XW <= sh_edges.n &&
-            (size_t)rtx * rty <= nparts) {
-            sheet_rev = (long long)prog->cu_adj_sheet * prog->ncu >=
-                        (long long)rtx * rty && !no_sheet_rev;
-        }
+        const bool sheet_rev = driver == MKH_DRIVER_SHEET &&
+                               adj_sheet_fits() && adj_sheet != 0;
         /* Small domains on the one-step kernels: segment sg - 1 is
          * recomputed on a second stream while the reverse steps of segment
          * sg run, the two segments' states in two trajectory buffers. Only
          * where the workgroups of both kernels fit on the device at once
          * (otherwise each would only slow the other). Same kernels, same
          * inputs: the results are those of the in-line order. */
-        const int ncu = prog->ncu;
-        const bool overlap = !use_pers && nseg > 1 && !no_adj_overlap &&
-                             (long long)ggrid + cgrid <= ncu;
+        const bool overlap = !use_pers && overlap_fits;
         if (overlap) {
             MKH_HIP(adj.traj2.alloc((size_t)tslots * SN));
             if (!rc_stream) {
@@ -1963,8 +2020,7 @@ struct Sim : SimBase {
          * linear pass, while the entries of a step (one VJP per state and
          * cell) take less time on the whole device than one VJP takes
          * alone. */
-        const bool lin_rev = use_strand && prog->f_adj_lin &&
-                             n <= lin_cells && !no_adj_linear;
+        const bool lin_rev = use_strand && lin_rev_fits;
         long long lin_steps = 0;        /* steps whose entries are held */
         if (lin_rev) {
             lin_steps = std::max<long long>(

@@ -64,3 +64,55 @@ def test_conductance_field_uncoupled_and_other_model():
     _both(sc, {'ina.gNa': 16 * rng.uniform(0.8, 1.2, 100)}, [0, 99], 2.0, 90)
     sc = Scenario('br1977', 70, dt=0.005, gx=9.5, paced=(4, 1, 0, 0))
     _both(sc, {}, [0, 69], 2.0, 90)
+
+
+# below the shortest segments whose gain outweighs their cooperative launches
+# a gradient takes the kernels without those, and on small sheets with a
+# conductance field wherever segments are recomputed
+@pytest.mark.parametrize('shape,prec,field,kinds', [
+    (40, 64, False, {2: 'block', 3: 'linear'}),
+    (200, 64, False, {9: 'block', 10: 'linear'}),
+    (1000, 64, True, {9: 'step-overlap', 10: 'linear'}),
+    (1000, 32, False, {15: 'step-overlap', 16: 'step'}),
+    ((40, 20), 32, False, {15: 'step-overlap', 16: 'sheet'}),
+    ((40, 20), 64, False, {63: 'step-overlap', 64: 'sheet'}),
+    ((40, 20), 64, True, {64: 'step-overlap', 300: 'step'}),
+    ((300, 130), 64, True, {15: 'step', 16: 'step'}),
+])
+def test_segment_lengths(shape, prec, field, kinds):
+    rng = np.random.default_rng(3)
+    n = int(np.prod(shape))
+    if not field:
+        g = None
+    elif isinstance(shape, tuple):
+        g = (rng.uniform(2, 12, (shape[1], shape[0] - 1)),
+             rng.uniform(2, 12, (shape[1] - 1, shape[0])))
+    else:
+        g = (rng.uniform(2, 12, n - 1), None)
+    res = []
+    for K, kind in list(kinds.items()) + [(7, None)]:
+        s = Scenario('lr1991', shape, dt=0.005, gx=9.5, gy=6.0,
+                     paced=(4, 20, 0, 0), conductance_field=g).product(prec)
+        s.set_field('ina.gNa', 16 * np.linspace(0.8, 1.2, n).reshape(
+            shape[::-1] if isinstance(shape, tuple) else (n,)))
+        if kind is None:
+            s.set_tuning(driver='grid')
+            s.set_engine_option('adj_linear', 0)
+        probe = [(0, 0)] if isinstance(shape, tuple) else [0]
+        adj = TissueAdjoint(s, probe, checkpoint_every=K)
+        target = np.full((adj.n_steps(1.0), 1), -60.0)
+        loss, grad, dgx, dgy = adj.loss_and_gradient(1.0, target)
+        if kind is not None:
+            assert adj.reverse_kernel()[0] == kind
+        res.append((loss, dgx, dgy, np.array(grad['ina.gNa'])))
+    # against the one-step kernels on the grid driver: sums in another order
+    # (single precision: states and adjoints of 200 steps, rounded at 6e-8)
+    rel = 1e-9 if prec == 64 else 1e-4
+    for l, x, y, g in res[:-1]:
+        l0, x0, y0, g0 = res[-1]
+        assert l == pytest.approx(l0, rel=rel)
+        np.testing.assert_allclose(g, g0, rtol=0,
+                                   atol=rel * np.max(np.abs(g0)))
+        # (the conductances' gradients cancel over the cells)
+        assert x == pytest.approx(x0, rel=100 * rel, abs=1e-9)
+        assert y == pytest.approx(y0, rel=100 * rel, abs=1e-9)
