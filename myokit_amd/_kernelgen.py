@@ -876,6 +876,8 @@ def _text_cost(text, precision):
 
 # Groups of waves that share one cell step in the strand driver
 STRAND_GROUPS = 4
+# a kernel text without it
+NO_GROUPS = '#define MK_NG 0\n#define MK_SWORK 0\n'
 
 
 def strand_cells(coupling, dims):
@@ -903,6 +905,8 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
     sums of :func:`_deferred` and advances the states that depend on the
     diffusion current, in every group alike.
 
+    ``MK_SWORK``: what all groups together evaluate, in percent of the
+    cell step (equations that several groups need count in each).
     ``mk_gown[i]``: group that advances state i (-1: all, in part B);
     ``mk_gheld[g]``: bit i set if group g holds state i; ``mk_gq[k]``: group
     that logs quantity k. MK_NG is 0 (no such functions) for models of more
@@ -910,7 +914,7 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
     import re
     ns = len(cm.states)
     if ns > 64:
-        return '#define MK_NG 0\n'
+        return NO_GROUPS
     a_lines, b_lines, declared, qa, qb, qpart, ua, ub, in_y = _split_lines(
         cm, precision, native_maths, _deferred(cm))
     word = re.compile(r'[A-Za-z_][A-Za-z0-9_]*')
@@ -948,6 +952,11 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
         mine[g].append(r[:3])
         have[g] |= r[3]
         load[g] = after[g]
+    once = sum(_text_cost(t, precision)
+               for t in b_lines + qb + list(ub.values()))
+    work = sum(load) + groups * once
+    whole = sum(cost[n] for n in set().union(*have)) \
+        + sum(r[4] for r in roots) + once
     own = [-1] * ns
     qown = [0] * max(1, len(cm.quantities))
     for g in range(groups):
@@ -969,6 +978,7 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
             slot[i] = len(slot)
     tab = '    '
     out = ['#define MK_NG ' + str(groups),
+           '#define MK_SWORK ' + str(round(100 * work / max(1, whole))),
            '#define MK_NXS ' + str(max(1, len(slot))),
            '__device__ constexpr int mk_gown[MK_NS] = {'
            + ', '.join(str(x) for x in own) + '};',
@@ -1311,7 +1321,7 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         generate_cell_function(cm, precision, native_maths),
         generate_split_cell_function(cm, precision, native_maths),
         generate_group_cell_functions(cm, precision, native_maths)
-        if strand and int(coupling) != 3 else '#define MK_NG 0\n',
+        if strand and int(coupling) != 3 else NO_GROUPS,
         _read('mk_drivers.hip'),
     ]
     if adjoint:

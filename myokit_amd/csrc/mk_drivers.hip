@@ -49,10 +49,12 @@ typedef MkStepT<Real> MkStep;
 
 /* The layout this text was generated for: precision (bits), states,
  * fields, and the cells per thread of the sheet, chain and reverse-sheet
- * tiles. The host library reads it when it loads the module and rejects a
+ * tiles; last the strand driver's work (mkh_host.cpp, build_strand_layout).
+ * The host library reads it when it loads the module and rejects a
  * simulation configured for another layout. */
-extern "C" __device__ const int mk_layout[6] = {
-    (int)(sizeof(Real) * 8), MK_NS, MK_NF, MK_SCPT, MK_CCPT, MK_ACPT};
+extern "C" __device__ const int mk_layout[7] = {
+    (int)(sizeof(Real) * 8), MK_NS, MK_NF, MK_SCPT, MK_CCPT, MK_ACPT,
+    MK_SWORK};
 
 #define MK_NFA (MK_NF > 0 ? MK_NF : 1)
 #define MK_NQA (MK_NQ > 0 ? MK_NQ : 1)

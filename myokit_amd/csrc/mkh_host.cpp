@@ -78,8 +78,9 @@ struct Program {
                   f_adj_lin = nullptr;
     int n_entries = 0;      /* of mk_adj_jac, per cell and step */
     /* mk_layout of the module: precision, states, fields, sheet / chain /
-     * reverse-sheet cells per thread (have_layout false if absent) */
-    int layout[6] = {0, 0, 0, 0, 0, 0};
+     * reverse-sheet cells per thread, the strand driver's work (have_layout
+     * false if absent) */
+    int layout[7] = {0, 0, 0, 0, 0, 0, 0};
     bool have_layout = false;
     std::vector<char> code;
     /* The device's CUs and the workgroups of each persistent kernel that
@@ -458,13 +459,22 @@ struct Sim : SimBase {
      * cells, or 64 - 2 h cells of a longer one with h more on each side and
      * an exchange every h steps. h = 16, or 8 where the tiles would then
      * outnumber the CUs. As many tiles per CU as leave the split of a step
-     * over four waves the faster way: uncoupled cells 3 (LR1991 forward
-     * Euler, us per step, split and one thread per cell: single precision
-     * 16,384 cells 0.36 and 0.65, 32,768 0.44 and 0.67, 49,152 0.57 and
-     * 0.68, 65,536 0.74 and 0.69; double precision 1.29 and 3.40, 2.03 and
-     * 3.42, 2.67 and 3.48, 3.38 and 3.54), a line 4 (strand and grid driver:
-     * 1,000 cells 0.63 and 6.3, 12,000 0.70 and 6.4, 49,000 1.2 and 6.4;
-     * double precision 1.5 and 8.2, 1.6 and 8.4, 4.4 and 8.7). */
+     * over four waves the faster way. Uncoupled cells: k tiles issue k/4 of
+     * what the four groups evaluate together (layout[6], percent of the cell
+     * step, as equations that several groups need count in each), where one
+     * thread per cell issues the cell step once; so up to 3, while k times
+     * that is at most 350. Forward Euler, us per step, split and one thread
+     * per cell, 1, 2 and 3 tiles: LR1991 in single precision (112) 0.36 and
+     * 0.65, 0.44 and 0.67, 0.57 and 0.68 (4 tiles 0.74 and 0.69), in double
+     * (108) 1.29 and 3.40, 2.03 and 3.42, 2.67 and 3.48; DiFrancesco-Noble
+     * (177, 179) 1.15 and 1.51, 1.61 and 1.52, 2.26 and 1.56, in double 2.99
+     * and 5.09, 4.75 and 5.13, 6.19 and 5.16; the same with 8 more gates
+     * (158, 156) 1.21 and 1.77, 1.69 and 1.82, 2.33 and 1.85, in double 3.50
+     * and 6.58, 5.34 and 6.63, 7.40 and 6.71. A line: 4 (strand and grid
+     * driver: 1,000 cells 0.63 and 6.3, 12,000 0.70 and 6.4, 49,000 1.2 and
+     * 6.4; double precision 1.5 and 8.2, 1.6 and 8.4, 4.4 and 8.7;
+     * DiFrancesco-Noble, 49,000 cells in single precision 3.4 and 4.5, 30,000
+     * in double 5.6 and 9.5). */
     int build_strand_layout()
     {
         st_tiles = 0;
@@ -475,11 +485,15 @@ struct Sim : SimBase {
             return 0;
         const int per_cu = prog->cu_strand, ncu = prog->ncu;
         if (per_cu < 1) return 0;
+        const int work = std::max(100, prog->layout[6]);
         for (int h : {0, 16, 8}) {
-            if (h == 0 && coupled && n > 64) continue;
+            /* (one tile without exchange, or tiles with) */
+            if (coupled ? h == 0 && n > 64 : h > 0) continue;
             const long long width = 64 - 2 * h;
             const long long tiles = (n + width - 1) / width;
-            const int most = h == 0 ? 3 : h == 16 ? 1 : 4;
+            const int most = h == 0    ? std::min(3, std::max(1, 350 / work))
+                             : h == 16 ? 1
+                                       : 4;
             if (tiles > (long long)std::min(most, per_cu) * ncu) continue;
             st_halo = h;
             st_width = (int)width;

@@ -212,3 +212,25 @@ def test_batches_too_short_for_a_cooperative_launch(n, prec, least):
             out.append((b['membrane.V'], np.array(s.state())))
         for a, b in zip(*out):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize('n', [16384, 16385])
+def test_uncoupled_cells_of_a_model_that_splits_badly(n):
+    # a model whose four groups share much of the work (nearly twice the cell
+    # step in all) takes one tile per CU, then one thread per cell
+    out = []
+    for driver in ('auto', 'cells'):
+        s = myokit.SimulationOpenCL(
+            myokit.load_model('tests/data/dn-1985-normalised.mmt'),
+            myokit.pacing.blocktrain(1000, 0.5), ncells=n, diffusion=False)
+        s.set_step_size(DT)
+        s.set_tuning(driver=driver)
+        b = s.run_block(20 * DT, ['membrane.V'], log_interval=5 * DT)
+        # one launch for the batch of all rows and one for the steps after
+        # the last, or one per row
+        rows = len(b['time'])
+        assert s.engine_timing()['launches'] == (
+            2 if driver == 'auto' and n == 16384 else rows + 1)
+        out.append([b['membrane.V'], np.array(s.state())])
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
