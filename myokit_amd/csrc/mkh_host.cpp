@@ -87,6 +87,8 @@ struct Program {
      * are resident on one (0: no such kernel), asked once when the module is
      * loaded: the queries take about a millisecond each. */
     int ncu = 0, cu_sheet = 0, cu_strand = 0, cu_chain = 0, cu_adj_sheet = 0;
+    /* bytes of scratch memory per thread that spilled registers take */
+    int spill_sheet = 0, spill_grid = 0;
 
     hipError_t query()
     {
@@ -101,6 +103,13 @@ struct Program {
         ask(&cu_strand, f_strand, 256);
         ask(&cu_chain, f_chain, 64);
         ask(&cu_adj_sheet, f_adj_sheet, 256);
+        auto spill = [&](int* bytes, hipFunction_t f) {
+            if (e == hipSuccess && f)
+                e = hipFuncGetAttribute(
+                    bytes, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, f);
+        };
+        spill(&spill_sheet, f_sheet);
+        spill(&spill_grid, f_grid);
         return e;
     }
 };
@@ -592,6 +601,21 @@ struct Sim : SimBase {
         }
     }
 
+    /* Whether the sheet kernel spills so much that the grid kernel is the
+     * faster one: large cell models whose tiles of 4 cells per thread exceed
+     * the registers. Scratch bytes per thread of both and us per step, sheet
+     * and grid driver: DiFrancesco-Noble (16 states), single precision 725 x
+     * 725 204 and 0 B, 18.0 and 18.3 us, double 600 x 600 520 and 68 B, 47 and
+     * 35 us; with 8 more gates, single 468 and 0 B, 34 and 23 us, double 1200
+     * and 260 B, 119 and 60 us; with 24 more, single 600 x 600 (2 cells per
+     * thread) 320 and 0 B, 21 and 25 us, 725 x 725 1028 and 0 B, 111 and 35 us,
+     * double 600 x 600 1520 and 716 B, 108 and 190 us. */
+    bool sheet_spills() const
+    {
+        return prog->spill_sheet > 400 &&
+               prog->spill_sheet > 3 * prog->spill_grid;
+    }
+
     void choose_driver()
     {
         if (forced_driver >= 0 && feasible(forced_driver)) {
@@ -604,7 +628,8 @@ struct Sim : SimBase {
             /* (the adjoint keeps the layouts of its reverse kernels; its
              * forward steps take the strand kernel, strand_for) */
             driver = MKH_DRIVER_STRAND;
-        } else if (n > sheet_cells && feasible(MKH_DRIVER_SHEET)) {
+        } else if (n > sheet_cells && feasible(MKH_DRIVER_SHEET) &&
+                   !sheet_spills()) {
             driver = MKH_DRIVER_SHEET;
         } else if (max_domain <= max_block_cells &&
                    (ndom >= 64 || max_domain <= 512)) {

@@ -122,3 +122,30 @@ def test_rows_too_close_for_a_sheet_launch(shape, prec, row, field):
             out.append((b['membrane.V'], np.array(s.state())))
         for a, b in zip(*out):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize('shape,field,driver', [
+    ((600, 600), False, 'grid'), ((600, 600), True, 'grid'),
+    ((301, 217), True, 'sheet')])
+def test_sheet_tiles_that_spill_leave_the_grid_driver(shape, field, driver):
+    # 16 states in double precision: with 4 cells per thread the sheet kernel
+    # keeps half its registers in scratch memory; asked for, it runs
+    nx, ny = shape
+    out = []
+    for d in ('auto', 'sheet'):
+        s = myokit.SimulationOpenCL(
+            myokit.load_model('tests/data/dn-1985-normalised.mmt'),
+            myokit.pacing.blocktrain(1000, 2), ncells=shape, precision=64)
+        s.set_step_size(0.005)
+        s.set_paced_cells(4, ny, 0, 0)
+        if field:
+            s.set_conductance_field(np.full((ny, nx - 1), 2.0),
+                                    np.full((ny - 1, nx), 1.5))
+        else:
+            s.set_conductance(2.0, 1.5)
+        s.set_tuning(driver=d)
+        b = s.run_block(0.1, ['membrane.V'], log_interval=0.06)
+        assert s.engine_driver() == (driver if d == 'auto' else 'sheet')
+        out.append((b['membrane.V'], np.array(s.state())))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
