@@ -1144,7 +1144,7 @@ def adjoint_waves_default(cm, precision, adjoint_precision=None):
     return 1
 
 
-def sheet_cpt(precision, dims=None, n_states=8):
+def sheet_cpt(precision, dims=None, n_states=8, waves=None):
     """Cells per thread of the persistent sheet driver (tiles of 64 x 4 cpt
     cells for a 256-thread workgroup) on a sheet of ``dims`` (nx, ny) cells:
     the fewest (1, 2 or 4) whose tiles are all resident within the register
@@ -1156,13 +1156,13 @@ def sheet_cpt(precision, dims=None, n_states=8):
     1024 x 1024 20.6, -, -, 10.5; double precision 64 x 64 9.1, 6.0, 10.4,
     18.8; 400 x 400 16.5, 11.9, 16.1, 18.8; 600 x 600 27.6, -, 22.7, 30.0.
     4 for a sheet that fits with none of them; without ``dims``, the tile of
-    a small sheet."""
+    a small sheet. ``waves``: the budget that is given in their place."""
     if dims is None:
         return 1
     for cpt in (1, 2):
         tiles = -(-dims[0] // 64) * -(-dims[-1] // (4 * cpt))
-        if len(dims) == 2 and tiles <= 256 * sheet_waves(precision, cpt,
-                                                         n_states):
+        if len(dims) == 2 and tiles <= 256 * (
+                waves or sheet_waves(precision, cpt, n_states)):
             return cpt
     return 4
 

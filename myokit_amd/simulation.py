@@ -918,7 +918,8 @@ class SimulationOpenCL:
         """Cells per thread of the persistent sheet: the value given to
         :meth:`set_tuning`, else the one for this sheet's size."""
         return self._tuning.get('sheet_cpt') or _kernelgen.sheet_cpt(
-            self._precision, self._dims, self._nstate)
+            self._precision, self._dims, self._nstate,
+            self._tuning.get('sheet_waves'))
 
     def _adjoint_cpt(self):
         """Cells per thread of the persistent reverse sheet: the value given

@@ -149,3 +149,13 @@ def test_sheet_tiles_that_spill_leave_the_grid_driver(shape, field, driver):
         out.append((b['membrane.V'], np.array(s.state())))
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize('waves', [1, 2, 3])
+def test_tile_follows_a_given_register_budget(waves):
+    # 1,024 tiles of 64 x 4 cells need the rule's four waves: a smaller budget
+    # takes larger tiles, so that the driver asked for is not refused
+    s = _scenario((512, 512), False).product(64)
+    s.set_tuning(driver='sheet', sheet_waves=waves)
+    s.run_block(0.2, ['membrane.V'], log_interval=1)
+    assert s.engine_driver() == 'sheet'

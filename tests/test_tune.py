@@ -138,6 +138,12 @@ def test_sheet_tiles_follow_the_size():
         assert k.sheet_waves(prec, 1, 30) == k.sheet_waves(prec, 4, 30) \
             == k.sheet_waves(prec, 4)
     assert sim((100, 70)).tuning()['sheet_cpt'] == 1
+    # a register budget that is given counts in place of the rule's
+    s = sim((600, 600))
+    assert s.tuning()['sheet_cpt'] == 1
+    for waves, cpt in ((3, 2), (2, 4), (6, 1)):
+        s.set_tuning(sheet_waves=waves)
+        assert s.tuning()['sheet_cpt'] == cpt
     assert sim((1024, 1024)).tuning()['sheet_cpt'] == 4
 
 
