@@ -61,10 +61,15 @@ def dimco(*dims):
         yield tuple(int(i) for i in reversed(idx))
 
 
-@functools.lru_cache(maxsize=4)
 def _cell_prefixes(dims):
     """The key prefixes of every cell of a grid, 'x.' or 'x.y.'."""
     return tuple('.'.join(str(i) for i in x) + '.' for x in dimco(*dims))
+
+
+# Grids of at most this many cells keep their prefixes (about 60 bytes each,
+# 4 MB) for the process's next logs, of the four last sizes
+PREFIX_CELLS = 65536
+_kept_prefixes = functools.lru_cache(maxsize=4)(_cell_prefixes)
 
 
 def float_str(number, precision=DOUBLE_PRECISION):
@@ -252,10 +257,16 @@ def prepare_log(log, model, dims=None, global_vars=None,
     dtype = np.float64 if precision == DOUBLE_PRECISION else np.float32
     dims = tuple(dims) if dims else ()
 
+    _combos = []
+
     def dcombos():
         # Cell prefixes ('x.' or 'x.y.', first index fastest), built only
         # when a name is expanded over every cell
-        return _cell_prefixes(dims) if dims else ('',)
+        if not _combos:
+            keep = int(np.prod(dims)) <= PREFIX_CELLS
+            _combos.extend([''] if not dims else _kept_prefixes(dims) if keep
+                           else _cell_prefixes(dims))
+        return _combos
 
     def valid_index(kdims):
         # 'x.' or 'x.y.' with every index in range

@@ -27,8 +27,8 @@ from . import _expressions as ex
 from . import _kernelgen
 from . import _native
 from ._datalog import (DOUBLE_PRECISION, LOG_BOUND, LOG_INTER, LOG_NONE,
-                       LOG_STATE, SINGLE_PRECISION, dimco, float_str,
-                       prepare_log, split_key)
+                       LOG_STATE, PREFIX_CELLS, SINGLE_PRECISION, dimco,
+                       float_str, prepare_log, split_key)
 from ._err import (FindNanError, NumericalError, SimulationCancelledError,
                    SimulationError, SimultaneousProtocolEventError)
 from ._model import Variable
@@ -1207,7 +1207,9 @@ class SimulationOpenCL:
         logging_states = any(q.is_state() for q in quantities)
         colmap.setflags(write=False)
         r = quantities, colmap, cols, globals_, logging_states
-        self._layout = (keys, r)
+        # (some 15 MB at most, most of it keys)
+        self._layout = (keys, r) \
+            if max(len(keys), colmap.size // 16) <= PREFIX_CELLS else None
         return r
 
     def _run(self, duration, log, log_interval, report_nan, progress, msg):

@@ -392,3 +392,25 @@ def test_layout_of_a_repeated_log(model):
     assert out[0] == out[3]
     assert out[1] == (['membrane.V', 'ica.ICa'], [[0, -1, -1], [-1, -1, 1]])
     assert out[2] == (['ica.ICa', 'membrane.V'], [[-1, -1, 0], [1, -1, -1]])
+
+
+def test_large_grids_keep_no_keys(model):
+    # what outlives a log is bounded: the cell prefixes and the column layout
+    # of a grid beyond the limit go with it
+    from myokit_amd import _datalog
+    n = _datalog.PREFIX_CELLS
+    for cells, kept in ((n, 1), (n + 1, 0)):
+        _datalog._kept_prefixes.cache_clear()
+        s = myokit.SimulationOpenCL(model, ncells=cells)
+        log = myokit.prepare_log(['membrane.V'], s._model, dims=s._dims)
+        assert len(log) == cells and str(cells - 1) + '.membrane.V' in log
+        assert _datalog._kept_prefixes.cache_info().currsize == kept
+        a = s._log_layout(log)
+        assert (a is s._log_layout(log)) == bool(kept)
+        assert (s._layout is not None) == bool(kept)
+    # the same for a column map of many cells with few columns
+    s = myokit.SimulationOpenCL(model, ncells=(2048, 1024))
+    log = myokit.prepare_log(['3.5.membrane.V'], s._model, dims=s._dims)
+    assert s._log_layout(log)[1].shape == (1, 2048 * 1024)
+    assert s._layout is None
+    _datalog._kept_prefixes.cache_clear()
