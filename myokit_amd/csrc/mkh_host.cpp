@@ -372,6 +372,7 @@ struct Sim : SimBase {
 
     /* options */
     long long batch_steps = 1 << 16;
+    long long run_steps = 0;       /* planned in this run */
     long long log_rows_cap = 0;   /* 0 = automatic */
     bool time_kernels = false;
     int forced_driver = -1;
@@ -528,6 +529,14 @@ struct Sim : SimBase {
     {
         return st_tiles > 0 && ndom == 1 &&
                (d == MKH_DRIVER_STRAND || forced_driver < 0);
+    }
+
+    /* Whether a run's batches (but short ones, strand_steps) take the strand
+     * kernel. */
+    bool takes_strand() const
+    {
+        return driver == MKH_DRIVER_STRAND ||
+               (driver == MKH_DRIVER_CELLS && strand_for(driver));
     }
 
     /* Steps [s0, s1) from state `src` to state `dst` (two buffers) in one
@@ -1100,6 +1109,7 @@ struct Sim : SimBase {
         }
         total_rows = rows;
         rows_done = 0;
+        run_steps = 0;
         if (nrows) *nrows = rows;
         dst_values = nullptr;
         dst_times = dst_paces = nullptr;
@@ -1239,7 +1249,15 @@ struct Sim : SimBase {
         b = Batch();
         row_t_after.clear();
         StepRec r;
-        while (!plan.done && b.ns < batch_steps && b.nr < log_rows_cap_run) {
+        /* The strand driver takes a whole batch in one launch, which a NaN
+         * does not end: no more than the run has taken, at least 4,096, so
+         * that a run that meets one takes at most about twice its time (a
+         * batch costs some 50 us, 4,096 steps 2.6 ms and more) */
+        const long long most =
+            takes_strand() ? std::min(batch_steps,
+                                      std::max(4096LL, run_steps))
+                           : batch_steps;
+        while (!plan.done && b.ns < most && b.nr < log_rows_cap_run) {
             int f = plan.next(r);
             if (f) return pacing_error(f);
             Step& st = h_steps[b.ns++];
@@ -1254,6 +1272,7 @@ struct Sim : SimBase {
                 b.plog.push_back((double)(R)r.pace);
             }
         }
+        run_steps += b.ns;
         row_cur.assign((size_t)b.nr, -1);
         if (b.ns > 0)
             MKH_HIP(hipMemcpyAsync(steps.p, h_steps, b.ns * sizeof(Step),
@@ -1487,9 +1506,7 @@ struct Sim : SimBase {
         }
         /* Launch */
         const unsigned bt = (unsigned)cfg.block_threads;
-        const bool strand = (driver == MKH_DRIVER_STRAND &&
-                             ns >= strand_steps(b)) ||
-                            (driver == MKH_DRIVER_CELLS && strand_for(driver));
+        const bool strand = takes_strand() && ns >= strand_steps(b);
         /* batches too short for the strand's cooperative launch */
         const int d = driver != MKH_DRIVER_STRAND || strand ? driver
                       : n <= 512 ? MKH_DRIVER_BLOCK

@@ -234,3 +234,20 @@ def test_uncoupled_cells_of_a_model_that_splits_badly(n):
         out.append([b['membrane.V'], np.array(s.state())])
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+def test_launches_grow_with_the_run():
+    # a launch of the strand driver takes no more steps than the run before
+    # it, at least 4,096: a NaN early in a long run does not cost the rest of
+    # a full batch
+    s = _scenario(65).product(32)
+    s.run_block(40000 * DT, ['membrane.V'], log_interval=39999 * DT)
+    # 4,096, 4,096, 8,192, 16,384 and 7,232 steps up to or past the last row,
+    # which ends a batch
+    assert s.engine_driver() == 'strand'
+    assert s.engine_timing()['launches'] in (5, 6)
+    s = _scenario(65).product(32)
+    s.set_engine_option('batch_steps', 1000)
+    s.run_block(4000 * DT, ['membrane.V'], log_interval=1e6)
+    # the first row ends a batch of one step
+    assert s.engine_timing()['launches'] == 5
