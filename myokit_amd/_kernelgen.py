@@ -876,7 +876,9 @@ def _text_cost(text, precision):
 
 # Groups of waves that share one cell step in the strand driver
 STRAND_GROUPS = 4
-# a kernel text without it
+# LDS of a workgroup on gfx950
+LDS_BYTES = 160 * 1024
+# a kernel text without the strand driver
 NO_GROUPS = '#define MK_NG 0\n#define MK_SWORK 0\n'
 
 
@@ -910,7 +912,8 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
     ``mk_gown[i]``: group that advances state i (-1: all, in part B);
     ``mk_gheld[g]``: bit i set if group g holds state i; ``mk_gq[k]``: group
     that logs quantity k. MK_NG is 0 (no such functions) for models of more
-    than 64 states."""
+    than 64 states and for those whose exchange area does not fit into LDS
+    twice (the strand driver's two buffers)."""
     import re
     ns = len(cm.states)
     if ns > 64:
@@ -976,6 +979,9 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
         if own[i] >= 0 and any(i in held[g] for g in range(groups)
                                if g != own[i]):
             slot[i] = len(slot)
+    size = 8 if precision == DOUBLE_PRECISION else 4
+    if 2 * size * (64 * max(1, len(slot)) + 66) + 16 > LDS_BYTES:
+        return NO_GROUPS
     tab = '    '
     out = ['#define MK_NG ' + str(groups),
            '#define MK_SWORK ' + str(round(100 * work / max(1, whole))),

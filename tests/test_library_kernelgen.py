@@ -137,3 +137,42 @@ def test_constants_evaluated_on_host():
     assert cons['cell.RTF'] == pytest.approx(8314 * 310 / 96500, rel=1e-15)
     assert cons['ina.ENa'] == pytest.approx(
         8314 * 310 / 96500 * math.log(140 / 10), rel=1e-15)
+
+
+def _compiles(src, precision):
+    prog = ctypes.c_void_p()
+    log = ctypes.create_string_buffer(1 << 16)
+    r = _native.lib().mkh_program_build(
+        src.encode(), _kernelgen.compile_options(precision).encode(), None,
+        -1, ctypes.byref(prog), log, 1 << 16)
+    if r == 0:
+        _native.lib().mkh_program_free(prog)
+    return r == 0
+
+
+def _currents(n):
+    """The LR1991 model with n more currents, each a product (so that none
+    is folded into a sum of other variables)."""
+    m = myokit.load_model('example').clone()
+    mem, tot = m.get('membrane'), m.get('membrane.i_ion')
+    terms = [tot.rhs().code()]
+    for k in range(n):
+        v = mem.add_variable('extra' + str(k))
+        v.set_rhs(f'{1e-5 * (k + 1)!r} * (V + {50 + k}) * exp(V / {100 + k})')
+        terms.append(v.name())
+    tot.set_rhs(' + '.join(terms))
+    m.validate()
+    return m
+
+
+@pytest.mark.parametrize('n,strand', [(120, True), (170, False)])
+def test_models_whose_exchange_area_exceeds_lds_have_no_strand(n, strand):
+    # the groups exchange one value per current: 170 doubles of 64 cells twice
+    # are 170 KiB
+    cm = _prepare_cell_model(_currents(n), rl=False, diffusion=True,
+                             fields=[], quantities=['membrane.V'])
+    src = _kernelgen.generate_kernel(cm, 64, 1)
+    assert ('#define MK_NG 0' not in src) == strand
+    assert _compiles(src, 64)
+    # half the bytes in single precision
+    assert '#define MK_NG 0' not in _kernelgen.generate_kernel(cm, 32, 1)
