@@ -1173,6 +1173,21 @@ def sheet_cpt(precision, dims=None, n_states=8, waves=None):
     return 4
 
 
+def sheet_fits(split, precision, coupling, cpt):
+    """Whether the sheet kernel's tile fits into LDS: the potentials of two
+    steps with a halo, the values that a cell step's part A (the text ``split``)
+    hands to part B, and with a conductance field the tile's
+    conductances."""
+    import re
+    carry = int(re.search(r'#define MK_NCARRY (\d+)', split).group(1))
+    rows = 4 * cpt
+    values = 2 * (rows + 2) * 66 + carry * cpt * 256
+    if int(coupling) == 2:
+        values += rows * 65 + (rows + 1) * 64
+    size = 8 if precision == DOUBLE_PRECISION else 4
+    return size * values + 16 <= LDS_BYTES
+
+
 def sheet_waves(precision, cpt=4, n_states=8):
     """Waves per SIMD the sheet kernel's register budget must allow, which
     is also the workgroups per CU that are sure to be resident. 4 cells per
@@ -1275,6 +1290,7 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
     i_vm = vm.index() if (vm is not None and vm.is_state()) else 0
     bcells = 2048 if precision == DOUBLE_PRECISION else 4096
     real = 'double' if precision == DOUBLE_PRECISION else 'float'
+    split = generate_split_cell_function(cm, precision, native_maths)
     acpt = adjoint_sheet_cpt(precision) if adjoint_cpt is None \
         else int(adjoint_cpt)
     # 0: the reverse pass takes the one-step kernel
@@ -1305,6 +1321,8 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         '#define MK_CWAVES ' + str(cwaves),
         '#define MK_ACPT ' + str(acpt),
         '#define MK_GBLOCKS ' + str(gblocks),
+        '#define MK_SHEET ' + str(int(sheet_fits(split, precision, coupling,
+                                                 cpt))),
         # two steps per launch of the grid driver: single precision sheets of
         # models whose state fits the registers six times
         '#define MK_GRID2 ' + str(int(
@@ -1325,7 +1343,7 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         _read('mk_args.h'),
         _FLOAT_HELPERS,
         generate_cell_function(cm, precision, native_maths),
-        generate_split_cell_function(cm, precision, native_maths),
+        split,
         generate_group_cell_functions(cm, precision, native_maths)
         if strand and int(coupling) != 3 else NO_GROUPS,
         _read('mk_drivers.hip'),

@@ -622,6 +622,7 @@ __device__ __forceinline__ MkXWord* mk_edge(const MkSheet& sh, int par,
                         + e) * 64 + k) * MK_XW;
 }
 
+#if MK_SHEET
 extern "C" __global__ void __launch_bounds__(256, MK_SWAVES)
 mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
 {
@@ -879,6 +880,7 @@ mk_sheet(const MkArgs a, const MkSheet sh, const int s0, const int s1)
         }
     }
 }
+#endif
 
 /* ------------------------------------------------------------------------
  * Persistent chains: disjoint chains of cells (cables built with

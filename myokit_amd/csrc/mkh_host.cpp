@@ -2983,7 +2983,12 @@ int mkh_program_build(const char* source, const char* options,
         MKH_HIP(hipModuleGetFunction(&prog->f_cells, prog->module, "mk_cells"));
         MKH_HIP(hipModuleGetFunction(&prog->f_block, prog->module, "mk_block"));
         MKH_HIP(hipModuleGetFunction(&prog->f_grid, prog->module, "mk_grid"));
-        MKH_HIP(hipModuleGetFunction(&prog->f_sheet, prog->module, "mk_sheet"));
+        /* sheets, of models whose tiles fit into LDS */
+        if (hipModuleGetFunction(&prog->f_sheet, prog->module, "mk_sheet") !=
+            hipSuccess) {
+            prog->f_sheet = nullptr;
+            (void)hipGetLastError();
+        }
         MKH_HIP(hipModuleGetFunction(&prog->f_chain, prog->module, "mk_chain"));
         /* two steps of a sheet per launch: small models, single precision */
         if (hipModuleGetFunction(&prog->f_grid2, prog->module, "mk_grid2") !=

@@ -176,3 +176,31 @@ def test_models_whose_exchange_area_exceeds_lds_have_no_strand(n, strand):
     assert _compiles(src, 64)
     # half the bytes in single precision
     assert '#define MK_NG 0' not in _kernelgen.generate_kernel(cm, 32, 1)
+
+
+def _carried(n):
+    """The LR1991 model with n values that a cell step computes before it
+    knows the diffusion current and needs after."""
+    m = myokit.load_model('example').clone()
+    mem, v = m.get('membrane'), m.get('membrane.V')
+    terms = [v.rhs().code()]
+    for k in range(n):
+        a = mem.add_variable('extra' + str(k))
+        a.set_rhs(f'{1e-9 * (k + 1)!r} * exp(V / {100 + k})')
+        terms.append(a.name() + ' * i_diff')
+    v.set_rhs(' + '.join(terms))
+    m.validate()
+    return m
+
+
+@pytest.mark.parametrize('n,coupling,sheet', [
+    (14, 1, True), (14, 2, False), (12, 2, True), (20, 1, False)])
+def test_models_whose_sheet_tile_exceeds_lds_have_no_sheet(n, coupling,
+                                                           sheet):
+    # 16 x 256 doubles (8 KiB) per value of a tile of 4 cells per thread, and
+    # with a field 17 KiB of conductances
+    cm = _prepare_cell_model(_carried(n), rl=False, diffusion=True,
+                             fields=[], quantities=['membrane.V'])
+    src = _kernelgen.generate_kernel(cm, 64, coupling, tile_cpt=4)
+    assert ('#define MK_SHEET 1' in src) == sheet
+    assert _compiles(src, 64)
