@@ -1353,9 +1353,10 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
         parts.append(_adjointgen.generate_vjp_function(cm, precision,
                                                        adjoint_precision))
         # the linear reverse pass: double precision, where the strand driver
-        # may run
+        # may run (masks of 64 bits)
         lin = precision == DOUBLE_PRECISION and strand \
-            and int(coupling) != 3 and len(cm.states) <= 64
+            and int(coupling) != 3 and len(cm.states) <= 64 \
+            and len(cm.fields) <= 64
         if lin:
             tables, entries = _adjointgen.generate_jacobian_tables(cm)
             lin = entries <= _adjointgen.LINEAR_ENTRIES

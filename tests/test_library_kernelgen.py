@@ -204,3 +204,21 @@ def test_models_whose_sheet_tile_exceeds_lds_have_no_sheet(n, coupling,
     src = _kernelgen.generate_kernel(cm, 64, coupling, tile_cpt=4)
     assert ('#define MK_SHEET 1' in src) == sheet
     assert _compiles(src, 64)
+
+
+@pytest.mark.parametrize('n', [64, 65])
+def test_gradients_by_many_fields_compile(n):
+    # the last field, whose bit the linear pass's masks hold up to 64, is the
+    # one that matters
+    m = myokit.load_model('example').clone()
+    c = m.get('ina')
+    for k in range(n):
+        c.add_variable('extra' + str(k)).set_rhs(k + 1)
+    c.get('INa').set_rhs(c.get('INa').rhs().code()
+                         + f' + 1e-9 * extra{n - 1}')
+    m.validate()
+    cm = _prepare_cell_model(m, rl=False, diffusion=True, quantities=[],
+                             fields=['ina.extra' + str(k) for k in range(n)])
+    src = _kernelgen.generate_kernel(cm, 64, 1, adjoint=True)
+    assert ('#define MK_ADJ_LIN 1' in src) == (n == 64)
+    assert _compiles(src, 64)
