@@ -391,9 +391,8 @@ class FiberTissueSimulation:
             nan = []
             for (sim, log, q, colmap, cols, g, ls), run in zip(parts, runs):
                 values, times, paces = sim._exec_end(run, ok)
-                sim._fill_log(log, values, times, paces, cols, g, dtype)
-                nan.append(np.isnan(values[-1]).any()
-                           if cols and len(times) else log.has_nan())
+                nan.append(sim._fill_log(log, values, times, paces, cols, g,
+                                         dtype))
         else:
             nan = [logf.has_nan(), logt.has_nan()]
 

@@ -1238,7 +1238,6 @@ class SimulationOpenCL:
                     ' myokit.ProgressReporter or None.')
 
         arithmetic_error = False
-        nan = None
         if duration > 0:
             quantities, colmap, cols, globals_, logging_states = \
                 self._log_layout(log)
@@ -1246,13 +1245,11 @@ class SimulationOpenCL:
                 tmin, tmax, quantities, colmap, len(cols), logging_states,
                 log_interval, progress, msg)
             dtype = values.dtype
-            self._fill_log(log, values, times, paces, cols, globals_, dtype)
-            if cols and len(times):
-                nan = np.isnan(values[-1]).any()
-        # as DataLog.has_nan: a NaN in the final row, which is this run's
-        # last one, if it has logged any
-        if report_nan and (arithmetic_error or (
-                log.has_nan() if nan is None else nan)):
+            nan = self._fill_log(log, values, times, paces, cols, globals_,
+                                 dtype)
+        else:
+            nan = log.has_nan()
+        if report_nan and (arithmetic_error or nan):
             self._report_nan(log)
         return log
 
@@ -1429,6 +1426,9 @@ class SimulationOpenCL:
         _native.check(code, 'mkh_sim_step')
 
     def _fill_log(self, log, values, times, paces, cols, globals_, dtype):
+        """Puts a run's rows into ``log``; returns ``log.has_nan()``, from the
+        run's last row at once where it has one (each of the log's columns
+        then ends with it)."""
         import collections
         new = {}
         for key, what in globals_:
@@ -1441,6 +1441,10 @@ class SimulationOpenCL:
                 collections.OrderedDict.__setitem__(log, key, arr)
             else:
                 log.extend_column(key, arr)
+        if not len(times):
+            return log.has_nan()
+        return bool((cols and np.isnan(values[-1]).any())
+                    or any(np.isnan(new[key][-1]) for key, _ in globals_))
 
     def _report_nan(self, log):
         """Raises SimulationError describing the first numerical error, as

@@ -414,3 +414,29 @@ def test_large_grids_keep_no_keys(model):
     assert s._log_layout(log)[1].shape == (1, 2048 * 1024)
     assert s._layout is None
     _datalog._kept_prefixes.cache_clear()
+
+
+def test_nan_of_a_runs_last_row(model):
+    # as has_nan: any column of the log counts, those of time and pacing too,
+    # and a run without rows leaves the earlier last row
+    s = myokit.SimulationOpenCL(model, ncells=2)
+    nan = float('nan')
+    for values, pace, want in (([[1, 2]], [0], False), ([[nan, 2]], [0], True),
+                               ([[nan, 2], [1, 2]], [nan, 0], False),
+                               ([[1, 2]], [nan], True)):
+        log = myokit.prepare_log(['membrane.V', 'engine.pace'], s._model,
+                                 dims=s._dims, global_vars=['engine.pace'])
+        _, _, cols, g, _ = s._log_layout(log)
+        v = np.array(values, dtype=float)
+        t = np.arange(len(v), dtype=float)
+        assert s._fill_log(log, v, t, np.array(pace, dtype=float), cols, g,
+                           np.float64) is want
+        assert log.has_nan() is want
+        assert s._fill_log(log, v[:0], t[:0], t[:0], cols, g,
+                           np.float64) is want
+    log = myokit.prepare_log(['engine.pace'], s._model, dims=s._dims,
+                             global_vars=['engine.pace'])
+    _, _, cols, g, _ = s._log_layout(log)
+    # (a run without columns has one of no meaning)
+    assert s._fill_log(log, np.full((1, 1), nan), np.zeros(1), np.zeros(1),
+                       cols, g, np.float64) is False

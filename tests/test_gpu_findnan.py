@@ -209,3 +209,18 @@ def test_state_left_by_a_nan_run_is_that_of_its_row(shape, rows):
     for n, state in out:
         assert n == 1
         np.testing.assert_array_equal(state, out[0][1])
+
+
+def test_nan_in_the_pacing_level_is_reported():
+    # the cells logged have none
+    p = myokit.Protocol()
+    p.schedule(float('nan'), 0.5, 10)
+    s = myokit.SimulationOpenCL(myokit.load_model('example'), p, ncells=40)
+    s.set_paced_cells(1, 1, 20, 0)
+    log = ['engine.pace', '39.membrane.V']
+    d = s.run(0.53, log=log, log_interval=0.01, report_nan=False)
+    assert np.isnan(d['engine.pace'][-1])
+    assert np.isfinite(d['39.membrane.V']).all()
+    s.reset()
+    with pytest.raises(myokit.SimulationError, match='Numerical error'):
+        s.run(0.53, log=log, log_interval=0.01)
