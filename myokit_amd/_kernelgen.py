@@ -1093,11 +1093,16 @@ def adjoint_sheet_cpt(precision, dims=None):
     resident (:func:`adjoint_sheet_waves` per CU of 256). Measured on LR1991
     (us per reverse step; 1, 2, 8 cells per thread, one-step kernel): single
     precision 64 x 40 3.8, 6.9, 22.4, 6.2; 301 x 217 4.5, 7.1, 24.3, 7.0;
-    400 x 400 6.0, 9.3, 25.6, 10.2; 800 x 800 -, -, 32.7, 24.4; 1024 x 1024
-    -, -, 33.7, 35.8 (8 cells per thread fill every tile there: mu of 4,096
-    cells per CU in LDS); double precision 200 x 150 8.5, 15.6, 57, 10.8;
-    301 x 217 12.2, 15.9, 57, 11.8; 400 x 400 -, 23.5, 61, 23.8. Without
-    ``dims``, the tile of a small sheet."""
+    400 x 400 6.0, 9.3, 25.6, 10.2; double precision 200 x 150 8.5, 15.6, 57,
+    10.8; 301 x 217 12.2, 15.9, 57, 11.8; 400 x 400 -, 23.5, 61, 23.8. The
+    tiles of 8 cells per thread take the same time on any sheet that more
+    than half fills the device with them (mu of 4,096 cells per CU in LDS),
+    the one-step kernel time by cells: 832 x 832 31.4 and 26.1, 896 x 896
+    31.8 and 29.2, 960 x 896 31.8 and 30.6, 960 x 960 32.1 and 33.0, 992 x 992
+    32.1 and 33.6, 1024 x 1024 31.9 and 35.8 (Beeler-Reuter 29.5 and 26.0 on
+    960 x 896, 29.3 and 28.9 on 1024 x 992, 29.1 and 31.1 on 1024 x 1024), so
+    they take over at 900,000 cells. Without ``dims``, the tile of a small
+    sheet."""
     if dims is None:
         return 1
     if len(dims) == 2:
@@ -1110,7 +1115,7 @@ def adjoint_sheet_cpt(precision, dims=None):
             if fits(cpt):
                 return cpt
         if precision != DOUBLE_PRECISION and fits(8) \
-                and dims[0] * dims[1] >= 1000000:
+                and dims[0] * dims[1] >= 900000:
             return 8
     return 0
 

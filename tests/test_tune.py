@@ -160,6 +160,9 @@ def test_reverse_sheet_tiles_follow_the_size():
     assert k.adjoint_sheet_cpt(32, (65, 2049)) == 0
     assert k.adjoint_sheet_cpt(32, (1024, 1024)) == 8
     assert k.adjoint_sheet_cpt(32, (1025, 1024)) == 0
+    # the tiles of 8 cells per thread are the faster from 900,000 cells on
+    assert k.adjoint_sheet_cpt(32, (960, 960)) == 8
+    assert k.adjoint_sheet_cpt(32, (960, 896)) == 0
     # 0 leaves the persistent kernel out of the text
     s = sim((800, 800), rl=True)
     assert s.tuning()['adjoint_cpt'] is None
