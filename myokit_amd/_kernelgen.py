@@ -908,7 +908,8 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
     diffusion current, in every group alike.
 
     ``MK_SWORK``: what all groups together evaluate, in percent of the
-    cell step (equations that several groups need count in each).
+    cell step (equations that several groups need count in each; logged
+    quantities are left out).
     ``mk_gown[i]``: group that advances state i (-1: all, in part B);
     ``mk_gheld[g]``: bit i set if group g holds state i; ``mk_gq[k]``: group
     that logs quantity k. MK_NG is 0 (no such functions) for models of more
@@ -955,11 +956,14 @@ def generate_group_cell_functions(cm, precision, native_maths=False,
         mine[g].append(r[:3])
         have[g] |= r[3]
         load[g] = after[g]
-    once = sum(_text_cost(t, precision)
-               for t in b_lines + qb + list(ub.values()))
-    work = sum(load) + groups * once
-    whole = sum(cost[n] for n in set().union(*have)) \
-        + sum(r[4] for r in roots) + once
+    # the work of a step without its logged quantities, which are evaluated
+    # where a row is
+    once = sum(_text_cost(t, precision) for t in b_lines + list(ub.values()))
+    step = [set().union(*[closure(t) for kind, _, t in m if kind != 'q'])
+            for m in mine]
+    ends = sum(r[4] for r in roots if r[0] != 'q')
+    work = sum(cost[n] for h in step for n in h) + ends + groups * once
+    whole = sum(cost[n] for n in set().union(*step)) + ends + once
     own = [-1] * ns
     qown = [0] * max(1, len(cm.quantities))
     for g in range(groups):

@@ -222,3 +222,19 @@ def test_gradients_by_many_fields_compile(n):
     src = _kernelgen.generate_kernel(cm, 64, 1, adjoint=True)
     assert ('#define MK_ADJ_LIN 1' in src) == (n == 64)
     assert _compiles(src, 64)
+
+
+def test_split_ratio_leaves_logged_quantities_out():
+    # logging does not change how many tiles of uncoupled cells share a CU
+    def work(quantities, precision):
+        cm = _prepare_cell_model(
+            myokit.load_model('example'), rl=False, diffusion=False,
+            fields=[], quantities=quantities)
+        return int(re.search(
+            r'#define MK_SWORK (\d+)',
+            _kernelgen.generate_group_cell_functions(cm, precision)).group(1))
+    for precision in (32, 64):
+        w = work([], precision)
+        assert 100 <= w <= 116
+        assert work(['membrane.V', 'ica.ICa', 'ina.INa', 'ik.IK'],
+                    precision) <= 116
