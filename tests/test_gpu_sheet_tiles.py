@@ -93,6 +93,11 @@ def test_fp32_two_steps_per_launch_equal_one(shape, field):
         s.set_tuning(driver='grid')
         b = s.run_block(0.21, ['membrane.V'], log_interval=every * 0.01)
         assert s.engine_driver() == 'grid'
+        # 21 steps: one launch each where all log; the first alone and ten
+        # pairs where none but the first does
+        launches = s.engine_timing()['launches']
+        assert launches == {1: 21, 5: launches, 1000: 11}[every]
+        assert every != 5 or 13 <= launches <= 15
         out.append((b['membrane.V'][::5 // min(every, 5)], np.array(s.state())))
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_array_equal(out[0][1], out[1][1])

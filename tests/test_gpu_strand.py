@@ -46,6 +46,7 @@ def test_fp64_other_model_and_uncoupled():
                   events=((1, 0, 0.5, 1000, 0),),
                   fields={'ina.gNa': 16 * rng.uniform(0.5, 2, 131)})
     P, O = run_both(sc, 4.0, myokit.DOUBLE_PRECISION)
+    assert P['sim'].engine_timing()['launches'] == 2
     np.testing.assert_array_equal(P['V'], O['V'])
     np.testing.assert_array_equal(P['state'], O['state'])
 
@@ -87,7 +88,12 @@ def test_fp32_uncoupled_equals_cells(n):
         s.set_field('ina.gNa', 16 * rng.uniform(0.5, 2, n))
         s.set_tuning(driver=driver)
         b = s.run_block(1.0, ['membrane.V', 'ica.ICa'], log_interval=0.2)
+        # (the name of the layout, whichever kernel runs: one launch up to
+        # the last row and one after it, or one per row)
         assert s.engine_driver() == 'cells'
+        rows = len(b['time'])
+        assert s.engine_timing()['launches'] == (
+            2 if driver == 'auto' and n <= 49152 else rows + 1)
         out.append([b['membrane.V'], b['ica.ICa'], np.array(s.state())])
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
