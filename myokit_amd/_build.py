@@ -41,9 +41,12 @@ def build_library(verbose=False):
 
 
 def check_kernel_compiles(precision=32, coupling=1, adjoint=False, rl=True,
-                          fields=(), adjoint_precision=None):
+                          fields=(), adjoint_precision=None, tile_cpt=None,
+                          adjoint_cpt=None):
     """Generates the LR1991 kernel (with the adjoint kernels if ``adjoint``)
-    and compiles it for gfx950 with hiprtc (no device needed)."""
+    and compiles it for gfx950 with hiprtc (no device needed). ``tile_cpt``
+    and ``adjoint_cpt``: the tiles of the sheet kernels (default: those of a
+    small sheet)."""
     import ctypes
     from . import _native, _kernelgen
     from .simulation import _prepare_cell_model
@@ -52,8 +55,9 @@ def check_kernel_compiles(precision=32, coupling=1, adjoint=False, rl=True,
     cm = _prepare_cell_model(model, rl=rl, diffusion=True,
                              fields=list(fields), quantities=['membrane.V'])
     src = _kernelgen.generate_kernel(cm, precision, coupling,
-                                     adjoint=adjoint,
-                                     adjoint_precision=adjoint_precision)
+                                     adjoint=adjoint, tile_cpt=tile_cpt,
+                                     adjoint_precision=adjoint_precision,
+                                     adjoint_cpt=adjoint_cpt)
     prog = ctypes.c_void_p()
     log = ctypes.create_string_buffer(1 << 16)
     _native.check(_native.lib().mkh_program_build(
@@ -63,9 +67,18 @@ def check_kernel_compiles(precision=32, coupling=1, adjoint=False, rl=True,
     return True
 
 
+def check_kernels():
+    """The kernels of small sheets, and of sheets that fill the device (tiles
+    of 4 cells per thread, in the reverse pass of 8), both precisions."""
+    for p in (32, 64):
+        check_kernel_compiles(p)
+        check_kernel_compiles(p, tile_cpt=4)
+    check_kernel_compiles(64, adjoint=True)
+    check_kernel_compiles(32, adjoint=True, tile_cpt=4, adjoint_cpt=8)
+
+
 if __name__ == '__main__':
     print(build_library(verbose=True))
     if '--check' in sys.argv:
-        for p in (32, 64):
-            check_kernel_compiles(p)
+        check_kernels()
         print('kernels compile for gfx950')

@@ -1341,7 +1341,6 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
                                    and asg > 0 and persistent
                                    and adjoint_precision in (None, precision)
                                    else '0'),
-        '#define MK_ADJ_SWAVES ' + str(max(1, asg)),
         '#define MK_ADJ_SREG ' + str(max(1, min(asg, adjoint_sheet_waves(
             precision)))),
         '#define MK_ADJ_WAVES ' + str(max(1, int(

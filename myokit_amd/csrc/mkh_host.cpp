@@ -583,8 +583,11 @@ struct Sim : SimBase {
 
     /* Whether driver d can run this geometry and coupling: the block
      * driver needs every domain in one workgroup's LDS, the sheet a 2D
-     * homogeneous stencil whose tiles are co-resident, the cells driver
-     * uncoupled cells. */
+     * stencil (one pair of conductances or a field) whose tiles are
+     * co-resident and fit into LDS, the strand a line of cells in few tiles of
+     * a model that can be split, the chain a graph of chains, the cells driver
+     * uncoupled cells (which take the strand's kernel where it is the faster
+     * one, strand_for). */
     bool feasible(int d) const
     {
         switch (d) {

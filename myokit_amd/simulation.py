@@ -807,13 +807,14 @@ class SimulationOpenCL:
         """Launch configuration of the device engine (chosen automatically
         by default; :func:`myokit_amd.tune.autotune` measures and picks
         one). ``driver``: ``'auto'``, ``'cells'``, ``'block'``, ``'grid'``,
-        ``'sheet'``, ``'chain'`` or ``'strand'``; ``block_threads``: threads per
-        workgroup of the cells, block and grid kernels (multiple of 64);
-        ``sheet_cpt``: cells per thread of the persistent sheet (tile
-        64 x 4*cpt); ``sheet_waves``: waves per SIMD its register budget
-        allows; ``chain_cpt`` and ``chain_waves``: the same for the chain
-        driver (graphs of disjoint chains; one-wave tiles of at most
-        64*cpt cells); ``adjoint_waves``: the waves per SIMD of the reverse
+        ``'sheet'``, ``'chain'`` or ``'strand'`` (the sheet or strand driver,
+        asked for, takes every step, else only runs long enough to gain);
+        ``block_threads``: threads per workgroup of the cells, block and grid
+        kernels (multiple of 64); ``sheet_cpt``: cells per thread of the
+        persistent sheet (tile 64 x 4*cpt); ``sheet_waves``: waves per SIMD
+        its register budget allows; ``chain_cpt`` and ``chain_waves``: the
+        same for the chain driver (graphs of disjoint chains; one-wave tiles
+        of at most 64*cpt cells); ``adjoint_waves``: the waves per SIMD of the reverse
         kernels of :class:`TissueAdjoint` (0: as many as their registers
         allow); ``adjoint_cpt``: cells per thread of the persistent reverse
         sheet (tile 64 x 4*cpt); ``grid_waves``: the waves per SIMD the grid
@@ -956,8 +957,10 @@ class SimulationOpenCL:
 
     def engine_driver(self):
         """Name of the device execution driver of the last run (``cells``,
-        ``block``, ``grid``, ``sheet``, ``chain`` or ``strand``), or None before the
-        first run."""
+        ``block``, ``grid``, ``sheet``, ``chain`` or ``strand``), or None before
+        the first run. Steps too few for a launch of the sheet or strand driver
+        run on the grid or block kernels, and few uncoupled cells (``cells``)
+        on the strand's."""
         if self._engine is None:
             return None
         d = ctypes.c_int(-1)
