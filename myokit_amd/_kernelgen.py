@@ -1341,6 +1341,8 @@ def generate_kernel(cm, precision, coupling, block_threads=256,
                                    and asg > 0 and persistent
                                    and adjoint_precision in (None, precision)
                                    else '0'),
+        # (workgroups per CU that fit into LDS; the budget of the registers)
+        '#define MK_ADJ_SWAVES ' + str(max(1, asg)),
         '#define MK_ADJ_SREG ' + str(max(1, min(asg, adjoint_sheet_waves(
             precision)))),
         '#define MK_ADJ_WAVES ' + str(max(1, int(

@@ -410,7 +410,7 @@ mk_adj_gather(const double* __restrict__ src,
  * Each workgroup owns a tile of 64 x MK_ATH cells (MK_ATH = 4 * MK_ACPT);
  * thread (lx, w) handles cells (x0 + lx, y0 + w * MK_ACPT + k), k <
  * MK_ACPT, one after the other. The registers are budgeted for MK_ADJ_SREG
- * workgroups per CU, no more than fit into LDS. mu of the tile stays in LDS
+ * workgroups per CU, no more than fit into LDS (MK_ADJ_SWAVES). mu of the tile stays in LDS
  * for the whole segment, abar of the tile and a one-cell ring around it too. The
  * potentials V_s and V_{s+1} come from the trajectory, complete in global
  * memory, so only abar crosses tiles: after each step a tile stores the
