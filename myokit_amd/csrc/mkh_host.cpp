@@ -1852,18 +1852,22 @@ struct Sim : SimBase {
      * reverse steps of the next on sheets that leave room (`overlap_fits`),
      * which outweighs the forward steps' gain where the reverse steps are the
      * same either way, and hid them on the smallest sheets. us per step, this
-     * and the grid driver's kernels, segments of 10, 20, 50 and 100 steps: 24 x
-     * 24 in single precision 16.3 and 15.5, 11.8 and 14.2, 8.8 and 11.2, 7.4
-     * and 10.7, in double 26.3 and 18.4, 21.6 and 17.9, 18.0 and 17.6, 16.0
-     * and 17.3, with a conductance field (one-step reverse kernel) 25.9 and
-     * 17.3, 22.2 and 16.7, 19.5 and 16.5, 17.3 and 16.3; 301 x 217 with a field
-     * (no overlap) 18.2 and 17.3, 14.4 and 15.7 in single precision, 32.4 and
-     * 31.2, 28.1 and 29.4 in double. */
+     * and the grid driver's kernels, 100 steps in segments of 12, 24, 40 and
+     * 60: 64 x 63 in single precision 16.4 and 12.7, 12.8 and 12.4, 10.7 and
+     * 11.8, 9.3 and 11.6, with another field to differentiate 16.9 and 12.8,
+     * 13.3 and 12.5, 11.2 and 11.9, 9.9 and 11.6 (45 x 42 is faster from
+     * segments of 24 on); in double 25.8 and 20.0, 22.1 and 20.3, 19.5 and
+     * 19.6, 17.6 and 18.8, Rush-Larsen 27.7 and 21.2, 24.0 and 21.6, 21.3 and
+     * 20.7, 19.2 and 20.0. With a conductance field (one-step reverse kernel),
+     * 24 x 24 in double, segments of 10, 20, 50 and 100 of 200 steps 25.9 and
+     * 17.3, 22.2 and 16.7, 19.5 and 16.5, 17.3 and 16.3; 301 x 217 (no
+     * overlap), 10 and 20, 18.2 and 17.3, 14.4 and 15.7 in single precision,
+     * 32.4 and 31.2, 28.1 and 29.4 in double. */
     bool adj_short_sheet(long long K, bool overlap_fits) const
     {
         if (forced_driver == MKH_DRIVER_SHEET || adj_sheet >= 0) return false;
         if (adj_sheet_fits())
-            return n <= 4096 && K < (sizeof(R) == 4 ? 16 : 64);
+            return n <= 4096 && K < (sizeof(R) == 4 ? 20 : 48);
         return overlap_fits || K < 16;
     }
 

@@ -74,8 +74,8 @@ def test_conductance_field_uncoupled_and_other_model():
     (200, 64, False, {9: 'block', 10: 'linear'}),
     (1000, 64, True, {9: 'step-overlap', 10: 'linear'}),
     (1000, 32, False, {15: 'step-overlap', 16: 'step'}),
-    ((40, 20), 32, False, {15: 'step-overlap', 16: 'sheet'}),
-    ((40, 20), 64, False, {63: 'step-overlap', 64: 'sheet'}),
+    ((40, 20), 32, False, {19: 'step-overlap', 20: 'sheet'}),
+    ((40, 20), 64, False, {47: 'step-overlap', 48: 'sheet'}),
     ((40, 20), 64, True, {64: 'step-overlap', 300: 'step'}),
     ((300, 130), 64, True, {15: 'step', 16: 'step'}),
 ])
