@@ -1349,7 +1349,9 @@ struct Sim : SimBase {
     /* Sheets of at least this many cells take two steps per launch: on
      * small ones a workgroup's cells, one after the other, take longer than
      * a second launch (us per step, mk_grid and mk_grid2: 301 x 217 6.8 and
-     * 8.4, 3000 x 200 13.8 and 13.2, 1100 x 1100 22.5 and 19.1). */
+     * 8.4, 3000 x 200 13.8 and 13.2, 1100 x 1100 22.5 and 19.1; with the
+     * calls' host work, 1100 x 1100, Beeler-Reuter 24.1 and 20.1, with 4 more
+     * gates, the largest model that has it, 30.9 and 24.0). */
     static constexpr long long two_cells = 600000;
 
     /* Steps s and s + 1 of the batch in one launch (mk_grid2). */
